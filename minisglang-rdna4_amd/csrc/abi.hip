@@ -22,7 +22,7 @@ int launch_moe_gemm2_combine(const GemmArgs& p, int64_t row_blocks, const uint16
                              int row_dtype, hipStream_t stream);
 size_t gemv_workspace_bytes(int64_t M, int64_t N, int64_t K, int grouped, int64_t row_blocks);
 int launch_prefill(const GemmArgs& p, int64_t rows_to_cover, int bm_rows, hipStream_t stream);
-int launch_prefill_lds(const GemmArgs& p, int64_t rows_to_cover, int bm_rows, hipStream_t stream);
+int launch_prefill_staged(const GemmArgs& p, int64_t rows_to_cover, int bm_rows, hipStream_t stream);
 int launch_prefill_dma(const GemmArgs& p, int64_t rows_to_cover, int bm_rows, hipStream_t stream);
 int launch_moe_route(const void* logits, int dtype, int64_t T, int E, int top_k, int renorm, float* tw,
                      int32_t* ids, hipStream_t stream);
@@ -255,8 +255,8 @@ static int run_dense(const char* who, GemmArgs& p, int kernel, hipStream_t strea
   char what[96];
   snprintf(what, sizeof what, "%s(%s)", who, decode ? "decode" : "prefill");
   if (decode) return hip_status(launch_gemv(p, (p.M + 15) / 16, false, stream), what);
-  // LDS-staged kernel for int4 groups of 128+ and MXFP4; the per-wave kernel for the rest
-  int rc = launch_prefill_lds(p, p.M, 0, stream);
+  // the LDS-staged kernels; the per-wave kernel for the rest
+  int rc = launch_prefill_staged(p, p.M, 0, stream);
   if (rc == kErrUnsupported) rc = launch_prefill(p, p.M, 128, stream);
   return hip_status(rc, what);
 }
@@ -460,11 +460,11 @@ int w4a16_linear(const void* x, int x_dtype, int64_t M, int64_t K, int64_t ldx, 
     }
     rc = launch_prefill_dma(q, q.M, 0, st);
     if (rc != kErrUnsupported) return hip_status(rc, "w4a16_linear(prefill, term sum)");
-    rc = launch_prefill_lds(p, p.M, 0, st);
+    rc = launch_prefill_staged(p, p.M, 0, st);
     if (rc == kErrUnsupported) rc = launch_prefill(p, p.M, 128, st);
     rc = hip_status(rc, "w4a16_linear(prefill)");
   } else {
-    rc = launch_prefill_lds(p, p.M, 0, st);
+    rc = launch_prefill_staged(p, p.M, 0, st);
     if (rc == kErrUnsupported) rc = launch_prefill(p, p.M, 128, st);
     rc = hip_status(rc, "w4a16_linear(prefill)");
   }
@@ -617,7 +617,7 @@ static int moe_gemm_run(const char* who, GemmArgs& p, bool decode, int64_t E, vo
     return hip_status(launch_gemv(p, rb, false, stream), "w4a8_moe_gemm(decode)");
   }
   const int bm_rows = p.bm % 128 == 0 ? 128 : 64;
-  int rc = launch_prefill_lds(p, nblk * p.bm, bm_rows, stream);
+  int rc = launch_prefill_staged(p, nblk * p.bm, bm_rows, stream);
   if (rc == kErrUnsupported) rc = launch_prefill(p, nblk * p.bm, bm_rows, stream);
   return hip_status(rc, "w4a8_moe_gemm(prefill)");
 }

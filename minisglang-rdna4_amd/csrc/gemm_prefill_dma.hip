@@ -1,24 +1,30 @@
 // Large-M W4A8 GEMM (prefill band and grouped MoE GEMMs) with the activation tile copied straight
 // from global memory into LDS by the buffer unit (buffer_load ... lds), three LDS stages deep.
 //
-// Same arithmetic and tile shapes as gemm_prefill_lds.hip (python/minisgl/quant/kernels.py:1632,
-// 1686-1734, 744-773): y[m,n] = s_m * sum_g scale[g,n] * sum_{k in g} e4m3(x[m,k]) w(n,k), f32
-// accumulation, one MFMA per (row block, strip, K step) of 128.
+// The math of the reference's wmma_tiled_tuned arm and of its grouped MoE GEMMs
+// (python/minisgl/quant/kernels.py:1632, 1686-1734, 744-773): y[m,n] = s_m * sum_g scale[g,n] *
+// sum_{k in g} e4m3(x[m,k]) w(n,k), f32 accumulation. Per (row block, strip, K step of 128): one
+// 16x16x128 MFMA, or for groups of 64 and 32 four 16x16x32 ones (half the rate, but a group's partial
+// must be scaled by itself: the full-rate MFMA with the other blocks masked out takes 2 or 4 times its
+// cycles).
 //
-// What changes is how a K step's operands reach LDS:
+// How a K step's operands reach LDS:
 //   A (BM x 128 fp8) and, for MXFP4, the fp4 weight strips and their E8M0 bytes are loaded by
 //   LDS-DMA: one 1 KiB block per wave instruction, written in lane order, which is exactly the
 //   MFMA operand order, so no VGPR holds them and no ds_write is issued;
-//   int4 weights still go through registers: each workgroup unpacks every strip once (to the fp8
-//   operand) and writes it to LDS, with its fp16 scales and zero words.
+//   int4 weights go through registers: each workgroup unpacks every strip once to the fp8 operand and
+//   writes it to LDS, with its fp16 scales. Symmetric groups of 128+ are unpacked as q - 7.5 with one
+//   table lookup and the half step taken back through the row sums; the other forms as e4m3(q - z),
+//   which needs no row sums (decode_lut4). With zero points applied per accumulator instead (two FMAs
+//   per element and a row-sum MFMA per row block) M=1777 K=2560 N=9728 took 102 us, so 86. Groups of
+//   32 on the kernel that masks the full-rate MFMA and loads operands straight from global memory:
+//   M=2048 K=2816 N=2048 196 us, here 44.
 // Each stage is its own __shared__ array and every stage index is a compile-time constant (the K
 // loop is unrolled by three), so the compiler tells the stages apart: reading stage k does not
 // wait for the DMAs in flight to stages k+1 and k+2. Step k issues the loads of step k+2 (int4:
 // between its MFMAs), computes step k, writes the int4 registers of step k+1, then waits for its
 // own step-k+1 loads (a counted vmcnt, the loads of step k+2 stay in flight) and meets the other
 // waves at one s_barrier.
-#include <cstdlib>
-
 #include "prefill.h"
 
 namespace w4a8 {
@@ -30,6 +36,9 @@ gemm_dma_kernel(const GemmArgs p) {
   constexpr int BM = WM * RB * 16, BN = WN * NSB * 16;
   constexpr int NSTRIP = BN / 16;
   constexpr bool kFp4 = MODE == kPE8M0;
+  // groups per K tile, and the modes whose weights are decoded as e4m3(q - z) (see decode_lut4)
+  constexpr int GPT = prefill_gpt(MODE);
+  constexpr bool kLut = prefill_lut(MODE), kLutZ = prefill_lut_zeros(MODE);
   using S = LdsStage<BM, BN, MODE>;
   constexpr int A_PER = (BM / 8) / NW;                 // A 1 KiB blocks per wave per step
   static_assert(A_PER * NW == BM / 8, "A blocks / waves");
@@ -48,7 +57,8 @@ gemm_dma_kernel(const GemmArgs p) {
   constexpr int B_PER = kFp4 ? 0 : NSTRIP * 64 / T;    // int4 16-byte chunks per thread per step
   static_assert(kFp4 || B_PER * T == NSTRIP * 64, "int4 chunks / threads");
   // vector-memory operations every wave issues per step (all unconditional, so one count holds)
-  constexpr int NOPS = (kFp4 ? S_DMA + A_PER + B_DMA : A_PER + B_PER + 1 + (MODE == kPAsym ? 1 : 0)) + (kSeedL ? 1 : 0);
+  constexpr int ZL = kLutZ ? (GPT > 1 ? 2 : 1) : 0;    // zero words per chunk: its one or two groups
+  constexpr int NOPS = (kFp4 ? S_DMA + A_PER + B_DMA : A_PER + B_PER * (1 + ZL) + 1) + (kSeedL ? 1 : 0);
 
   __shared__ __align__(16) unsigned char st0[kStage];
   __shared__ __align__(16) unsigned char st1[kStage];
@@ -107,10 +117,10 @@ gemm_dma_kernel(const GemmArgs p) {
   const unsigned char* scales = reinterpret_cast<const unsigned char*>(p.scales) + (size_t)(expert * p.s_expert_stride) * kEsz;
   const int32_t* zeros = p.zeros ? p.zeros + expert * p.z_expert_stride : nullptr;
   const int ngroups = K >> (31 - __builtin_clz((unsigned)p.group));
-  const BufRsrc rs_a = make_rsrc(p.xq, 0xffffffffu);
-  const BufRsrc rs_w = make_rsrc(wt, (uint32_t)((size_t)nstrips * KT * kTileBytes));
-  const BufRsrc rs_s = make_rsrc(scales, (uint32_t)((size_t)(kFp4 ? K / 32 : ngroups) * N * kEsz));
-  const BufRsrc rs_z = make_rsrc(zeros, zeros ? (uint32_t)((size_t)ngroups * (N / 8) * 4) : 0u);
+  static_assert(GPT == 1 || !kFp4, "sub-tile groups are int4");
+  const uint32_t w_bytes = (uint32_t)((size_t)nstrips * KT * kTileBytes);
+  const uint32_t s_bytes = (uint32_t)((size_t)(kFp4 ? K / 32 : ngroups) * N * kEsz);
+  const uint32_t z_bytes = zeros ? (uint32_t)((size_t)ngroups * (N / 8) * 4) : 0u;
 
   // ---- per-lane source offsets (fixed across K steps; the step adds a scalar offset)
   // A block b = wave + i*NW of a step is row block b/2, half b%2; lane l reads row (l & 15) of it,
@@ -131,10 +141,15 @@ gemm_dma_kernel(const GemmArgs p) {
       a_voff[i] = (uint32_t)((ok ? ar : 0) * p.ldx) + (b & 1) * 64 + 16 * (lane >> 4);
     }
   }
+  // K past the last whole tile (formats with groups below 128 only; A in operand order has none)
+  constexpr bool kKTail = (GPT > 1 || kFp4) && !AT;
+  const int ktail = K - (KT - 1) * kTileK;
+  const uint32_t a_back = (wave & 1) * 64 + 16 * (lane >> 4) >= ktail ? kTileK : 0;
+  static_assert(NW % 2 == 0, "a wave's A blocks are all the same half");
   // seeds: wave w copies rows 64 (w % (BM / 64)) + lane of the tile (waves past BM / 64 copy the same
   // rows again, so every wave issues one DMA per step and one vmcnt count holds)
   constexpr int kSeedW = BM / 64 > 0 ? BM / 64 : 1;
-  const BufRsrc rs_seed = make_rsrc(p.seeds, kSeedL ? (uint32_t)((size_t)KT * p.seeds_ld * 4) : 0u);
+  const uint32_t seed_bytes = kSeedL ? (uint32_t)((size_t)KT * p.seeds_ld * 4) : 0u;
   uint32_t seed_voff = 0;
   if constexpr (kSeedL) {
     int64_t sr = blk_row0 + 64 * (wave % kSeedW) + lane;
@@ -148,6 +163,10 @@ gemm_dma_kernel(const GemmArgs p) {
   // nearly every VGPR through the K loop.
   __shared__ float e_sc[BM];
   __shared__ int e_ok[BM];
+  __shared__ uint4 zlut[kLutZ ? 16 : 1];
+  if constexpr (kLutZ) {
+    if (threadIdx.x < 16) zlut[threadIdx.x] = zero_point_lut((int)threadIdx.x);
+  }
   const int er = (int)threadIdx.x;
   float er_sc = 0.f;
   bool er_ok = false;
@@ -173,10 +192,12 @@ gemm_dma_kernel(const GemmArgs p) {
   // zero words 8 B per strip (threads past the counts load duplicates of the last and write the
   // same bytes again)
   uint32_t b_voff[kFp4 ? 1 : B_PER];
-  constexpr int S_CHUNKS = NSTRIP * 2;
+  constexpr int S_CHUNKS = NSTRIP * 2 * GPT;
+  static_assert(kFp4 || S_CHUNKS <= T, "scale chunks / threads");
   const int sc_c = (int)threadIdx.x < S_CHUNKS ? (int)threadIdx.x : S_CHUNKS - 1;
-  const int z_c = (int)threadIdx.x < NSTRIP ? (int)threadIdx.x : NSTRIP - 1;
-  uint32_t s_voff = 0, z_voff = 0;
+  uint32_t s_voff = 0;
+  uint32_t z_voff[kLutZ ? B_PER : 1];
+  int z_sh[kLutZ ? B_PER : 1];
   if constexpr (!kFp4) {
 #pragma unroll
     for (int i = 0; i < B_PER; ++i) {
@@ -184,33 +205,56 @@ gemm_dma_kernel(const GemmArgs p) {
       bool ok;
       const int gs = gstrip(c >> 6, ok);
       b_voff[i] = (uint32_t)(((size_t)gs * KT * 64 + (c & 63)) * 16);
+      if constexpr (kLutZ) {
+        // the chunk's first 16 codes are K 16q.. of the tile, the other 16 K 64 + 16q..: groups
+        // q * GPT / 8 and that + GPT / 2
+        const int l = c & 63, n = gs * 16 + (l & 15);
+        z_voff[i] = (uint32_t)((((l >> 4) * GPT / 8) * (N / 8) + n / 8) * 4);
+        z_sh[i] = 4 * (n & 7);
+      }
     }
     bool ok;
-    s_voff = (uint32_t)((gstrip(sc_c >> 1, ok) * 16 + (sc_c & 1) * 8) * 2);
-    z_voff = (uint32_t)(gstrip(z_c, ok) * 2 * 4);
+    const int sc_s = sc_c % (NSTRIP * 2), sc_g = sc_c / (NSTRIP * 2);
+    s_voff = (uint32_t)((sc_g * N + gstrip(sc_s >> 1, ok) * 16 + (sc_s & 1) * 8) * 2);
   }
 
   // int4 register sets, one per stage index (two are live at a time)
   v4u rbw[3][kFp4 ? 1 : B_PER];
   uint4 rsc[3];
-  uint2 rzp[3];
+  uint32_t rzp[3][kLutZ ? B_PER : 1][ZL > 0 ? ZL : 1];
 
   // loads of K step kt into stage I (DMA) / register set I (int4 weights, scales, zeros)
-  // part: 1 = the A DMAs (and fp4 strips / E8M0 bytes), 2 = the int4 weight, scale and zero loads
-  auto issue = [&](auto I, int kt, int part = 3) __attribute__((always_inline)) {
+  // part: 1 = the A DMAs (and fp4 strips / E8M0 bytes), 2 = the int4 weight, scale and zero loads.
+  // Tail: steps past the last read empty buffers (at the last step's offsets): those loads touch no
+  // memory and nothing uses what they bring, so every step issues the same instructions and the one
+  // vmcnt count holds to the end.
+  auto issue = [&](auto I, int kt, int part, auto Tail) __attribute__((always_inline)) {
     constexpr int R = decltype(I)::value;
     unsigned char* st = stage(I);
+    constexpr bool kRagged = kKTail && decltype(Tail)::value;  // the last tile is always loaded by a tail step
+    const uint32_t live = decltype(Tail)::value ? (uint32_t)__builtin_amdgcn_readfirstlane(kt < KT ? -1 : 0) : 0xffffffffu;
+    if constexpr (decltype(Tail)::value) kt = kt < KT ? kt : KT - 1;
+    const BufRsrc rs_a = make_rsrc(p.xq, live);
+    const BufRsrc rs_w = make_rsrc(wt, w_bytes & live);
+    const BufRsrc rs_s = make_rsrc(scales, s_bytes & live);
+    const BufRsrc rs_z = make_rsrc(zeros, z_bytes & live);
+    const BufRsrc rs_seed = make_rsrc(p.seeds, seed_bytes & live);
     if constexpr (kFp4) {
 #pragma unroll
-      for (int i = 0; i < S_DMA; ++i)
-        lds_dma4(rs_s, st + S::kA + S::kB + (wave + i * NW) * 256, e_voff[i],
-                 (uint32_t)__builtin_amdgcn_readfirstlane(kt * 4 * N));
+      for (int i = 0; i < S_DMA; ++i) {  // scale rows past K: out of the buffer's range, so zeros
+        const uint32_t so_e = (uint32_t)__builtin_amdgcn_readfirstlane(kt * 4 * N);
+        lds_dma4(rs_s, st + S::kA + S::kB + (wave + i * NW) * 256, kRagged ? e_voff[i] + so_e : e_voff[i],
+                 kRagged ? 0 : so_e);
+      }
     }
     const uint32_t so_a = (uint32_t)__builtin_amdgcn_readfirstlane(AT ? kt * 2048 : kt * kTileK);
     if (part & 1) {
+      // the last tile of a K that is no multiple of 128: its chunks past K read the tile before (in
+      // bounds; the operand read masks them out)
+      const uint32_t back = kRagged ? a_back & (uint32_t)__builtin_amdgcn_readfirstlane(kt == KT - 1 ? -1 : 0) : 0u;
 #pragma unroll
       for (int i = 0; i < A_PER; ++i)
-        lds_dma16(rs_a, st + (wave + i * NW) * 1024, a_voff[i], so_a);
+        lds_dma16(rs_a, st + (wave + i * NW) * 1024, a_voff[i] - back, so_a);
       if constexpr (kSeedL)
         lds_dma4(rs_seed, st + kSeedOff + (wave % kSeedW) * 256, seed_voff,
                  (uint32_t)__builtin_amdgcn_readfirstlane(kt * (int)p.seeds_ld * 4));
@@ -224,9 +268,16 @@ gemm_dma_kernel(const GemmArgs p) {
       const uint32_t so_b = (uint32_t)__builtin_amdgcn_readfirstlane(kt * kTileBytes);
 #pragma unroll
       for (int i = 0; i < B_PER; ++i) rbw[R][i] = bload128v(rs_w, b_voff[i], so_b);
-      const int g = kt >> gshift;
-      rsc[R] = bload128(rs_s, s_voff, (uint32_t)__builtin_amdgcn_readfirstlane(g * N * 2));
-      if (MODE == kPAsym) rzp[R] = bload64(rs_z, z_voff, (uint32_t)__builtin_amdgcn_readfirstlane(g * (N / 8) * 4));
+      const int g = GPT > 1 ? kt * GPT : kt >> gshift;
+      const uint32_t so_s = (uint32_t)__builtin_amdgcn_readfirstlane(g * N * 2);
+      rsc[R] = kRagged ? bload128(rs_s, s_voff + so_s, 0) : bload128(rs_s, s_voff, so_s);  // past K: zeros
+      if constexpr (kLutZ) {
+#pragma unroll
+        for (int i = 0; i < B_PER; ++i)
+#pragma unroll
+          for (int h = 0; h < ZL; ++h)
+            rzp[R][i][h] = bload32(rs_z, z_voff[i], (uint32_t)__builtin_amdgcn_readfirstlane((g + h * (GPT / 2)) * (N / 8) * 4));
+      }
     }
   };
   // int4: unpack register set R into stage I
@@ -239,12 +290,21 @@ gemm_dma_kernel(const GemmArgs p) {
       for (int i = 0; i < B_PER; ++i) {
         const int c = (int)threadIdx.x + i * T;
         const int s = c >> 6, l = c & 63;
-        const v8i u = unpack_tile_int4(make_uint4(rbw[R][i].x, rbw[R][i].y, rbw[R][i].z, rbw[R][i].w));
+        const uint4 w = make_uint4(rbw[R][i].x, rbw[R][i].y, rbw[R][i].z, rbw[R][i].w);
+        v8i u;
+        if constexpr (kLutZ) {
+          const uint4 t0 = zlut[(rzp[R][i][0] >> z_sh[i]) & 15u];
+          const uint4 t1 = ZL > 1 ? zlut[(rzp[R][i][ZL - 1] >> z_sh[i]) & 15u] : t0;
+          u = unpack_tile_lut(w, t0, t1);
+        } else if constexpr (kLut) {
+          u = unpack_tile_lut(w, zero_point_lut(8), zero_point_lut(8));
+        } else {
+          u = unpack_tile_int4(w);
+        }
         *reinterpret_cast<uint4*>(sb + ((s * 2 + 0) * 64 + l) * 16) = make_uint4(u[0], u[1], u[2], u[3]);
         *reinterpret_cast<uint4*>(sb + ((s * 2 + 1) * 64 + l) * 16) = make_uint4(u[4], u[5], u[6], u[7]);
       }
       *reinterpret_cast<uint4*>(st + S::kA + S::kB + sc_c * 16) = rsc[R];
-      if (MODE == kPAsym) *reinterpret_cast<uint2*>(st + S::kA + S::kB + S::kS + z_c * 8) = rzp[R];
     }
   };
 
@@ -257,19 +317,33 @@ gemm_dma_kernel(const GemmArgs p) {
 
   // per-lane LDS offsets of this wave's operands within a stage; the empty asm keeps each in one
   // VGPR so every read is that VGPR plus an immediate
-  uint32_t oa = (uint32_t)(wm * RB * 2048 + lane * 16);
-  uint32_t ob = (uint32_t)(S::kA + wn * NSB * (kFp4 ? 1024 : 2048) + lane * 16);
+  // GPT > 1: 8-byte operands of the 16x16x32 MFMA, lane (row, q) holding K 8q.. of each 32: chunk
+  // q / 2 of the 16-byte chunks, half q % 2
+  const int lo = GPT > 1 ? (((lane >> 5) * 16 + (lane & 15)) * 16 + ((lane >> 4) & 1) * 8) : lane * 16;
+  uint32_t oa = (uint32_t)(wm * RB * 2048 + lo);
+  uint32_t ob = (uint32_t)(S::kA + wn * NSB * (kFp4 ? 1024 : 2048) + lo);
   uint32_t os = (uint32_t)(S::kA + S::kB + (kFp4 ? wn * NSB * 256 + lane : (wn * NSB * 16 + (lane & 15)) * 2));
-  uint32_t oz = (uint32_t)(S::kA + S::kB + S::kS + (wn * NSB * 2 + ((lane & 15) >> 3)) * 4);
-  asm volatile("" : "+v"(oa), "+v"(ob), "+v"(os), "+v"(oz));
-  const int zsh = 4 * (lane & 7);
+  asm volatile("" : "+v"(oa), "+v"(ob), "+v"(os));
 
   // MFMA work of one K step from stage I (operands read one row block / strip ahead of their
   // MFMAs). mid(i) runs right after the MFMAs of int4 strip i (i = 0, 1) or MXFP4 row block i, so
   // its work (the loads of a later step, the unpack of the next step's weights) overlaps MFMAs in
-  // flight.
-  auto compute = [&](auto I, auto mid) __attribute__((always_inline)) {
+  // flight. Waves of two row blocks and four strips have few MFMAs to hide it behind and wait on LDS instead:
+  // there mid(0) fills the wait for the step's first operands (K=4096 N=6144 M=512 30.9 against 30.0
+  // us, K=2816 N=2048 M=2048 in groups of 32 43.2 against 42.1; 256-row tiles equal or 1% slower).
+  constexpr bool kMidFirst = RB <= 2 && NSB > 2;
+  auto compute = [&](auto I, auto mid, int valid) __attribute__((always_inline)) {
     const unsigned char* st = stage(I);
+    // valid: the tile's K (128 but for a ragged last one, whose operand bytes past it are cleared)
+    const bool mlo = 16 * (lane >> 4) < valid, mhi = 64 + 16 * (lane >> 4) < valid;
+    auto a_operand = [&](const unsigned char* at) __attribute__((always_inline)) {
+      v8i a = lds_operand(at, 0);
+      if constexpr (kKTail) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) a[i] = (i < 4 ? mlo : mhi) ? a[i] : 0;
+      }
+      return a;
+    };
     if constexpr (kFp4) {
       uint4 braw[NSB];
       int sbyte[NSB];
@@ -278,62 +352,131 @@ gemm_dma_kernel(const GemmArgs p) {
         braw[j] = *reinterpret_cast<const uint4*>(st + ob + j * 1024);
         sbyte[j] = (int)st[os + j * 256];
       }
-      v8i a0 = lds_operand(st + oa, 0);
+      v8i a0 = a_operand(st + oa);
 #pragma unroll
       for (int rb = 0; rb < RB; ++rb) {
         v8i a1;
-        if (rb + 1 < RB) a1 = lds_operand(st + oa + (rb + 1) * 2048, 0);
+        if (rb + 1 < RB) a1 = a_operand(st + oa + (rb + 1) * 2048);
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int j = 0; j < NSB; ++j) acc[rb][j] = mfma_f8f4_sb(a0, fp4_operand(braw[j]), acc[rb][j], sbyte[j]);
         mid(rb);
         if (rb + 1 < RB) a0 = a1;
       }
+    } else if constexpr (GPT > 1) {
+      // the tile in 32-wide pieces, piece s at byte (s / 2) * 1024 + (s % 2) * 512 of the 16-row block
+      constexpr int PPG = 4 / GPT;  // pieces per group
+      long a[RB][4];
+#pragma unroll
+      for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+          a[rb][s] = 32 * s < valid ? *reinterpret_cast<const long*>(st + oa + rb * 2048 + (s >> 1) * 1024 + (s & 1) * 512) : 0;
+      long bn[4];
+#pragma unroll
+      for (int s = 0; s < 4; ++s) bn[s] = *reinterpret_cast<const long*>(st + ob + (s >> 1) * 1024 + (s & 1) * 512);
+      float scn[GPT];
+#pragma unroll
+      for (int g = 0; g < GPT; ++g) scn[g] = f16_to_f32(*reinterpret_cast<const uint16_t*>(st + os + g * NSTRIP * 32));
+      v4f cp[RB];
+      float scp = 0.f;
+      if constexpr (kMidFirst) {
+        __builtin_amdgcn_sched_barrier(0);
+        mid(0);
+      }
+#pragma unroll
+      for (int j = 0; j < NSB; ++j) {
+        long b[4];
+        float sc[GPT];
+#pragma unroll
+        for (int s = 0; s < 4; ++s) b[s] = bn[s];
+#pragma unroll
+        for (int g = 0; g < GPT; ++g) sc[g] = scn[g];
+        if (j + 1 < NSB) {
+#pragma unroll
+          for (int s = 0; s < 4; ++s)
+            bn[s] = *reinterpret_cast<const long*>(st + ob + (j + 1) * 2048 + (s >> 1) * 1024 + (s & 1) * 512);
+#pragma unroll
+          for (int g = 0; g < GPT; ++g)
+            scn[g] = f16_to_f32(*reinterpret_cast<const uint16_t*>(st + os + g * NSTRIP * 32 + (j + 1) * 32));
+        }
+#pragma unroll
+        for (int g = 0; g < GPT; ++g) {
+          // keeps one group's partials live at a time (and the one before it, below)
+          __builtin_amdgcn_sched_barrier(0);
+          v4f cj[RB];
+#pragma unroll
+          for (int rb = 0; rb < RB; ++rb) {
+            cj[rb] = __builtin_amdgcn_mfma_f32_16x16x32_fp8_fp8(a[rb][g * PPG], b[g * PPG], zero4, 0, 0, 0);
+            if constexpr (PPG == 2)
+              cj[rb] = __builtin_amdgcn_mfma_f32_16x16x32_fp8_fp8(a[rb][g * PPG + 1], b[g * PPG + 1], cj[rb], 0, 0, 0);
+          }
+          if (g == GPT - 1 && j < 2 && (j > 0 || !kMidFirst)) mid(j);
+          // the previous group's scale FMAs run between this group's MFMAs
+          if (j > 0 || g > 0) {
+            const int jp = g > 0 ? j : j - 1;
+#pragma unroll
+            for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+              for (int r = 0; r < 4; ++r) acc[rb][jp][r] += scp * cp[rb][r];
+#pragma unroll
+            for (int rb = 0; rb < RB; ++rb) {
+              __builtin_amdgcn_sched_group_barrier(0x008, PPG, 0);
+              __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);
+            }
+          }
+#pragma unroll
+          for (int rb = 0; rb < RB; ++rb) cp[rb] = cj[rb];
+          scp = sc[g];
+        }
+      }
+#pragma unroll
+      for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[rb][NSB - 1][r] += scp * cp[rb][r];
     } else {
       v8i a[RB];
 #pragma unroll
       for (int rb = 0; rb < RB; ++rb) a[rb] = lds_operand(st + oa + rb * 2048, 0);
       v4f pre[RB];
 #pragma unroll
-      for (int rb = 0; rb < RB; ++rb) {  // symmetric: -R/2; zero points: +R/2
-        if constexpr (kSeedL)
+      for (int rb = 0; rb < RB; ++rb) {  // symmetric: -R/2 undoes the codes' half step
+        if constexpr (kLut)
+          pre[rb] = zero4;
+        else if constexpr (kSeedL)
           pre[rb] = *reinterpret_cast<const v4f*>(st + kSeedOff + (wm * RB * 16 + rb * 16 + 4 * (lane >> 4)) * 4);
         else
-          pre[rb] = mfma_f8f8(a[rb], splat8(MODE == kPSym ? 0xB0B0B0B0u : kE4M3Half4), zero4);
+          pre[rb] = mfma_f8f8(a[rb], splat8(0xB0B0B0B0u), zero4);
       }
       v4f cp[RB];
-      float scp = 0.f, cfp = 0.f;
+      float scp = 0.f;
       v8i bn = lds_operand(st + ob, 0);
       float scn = f16_to_f32(*reinterpret_cast<const uint16_t*>(st + os));
-      uint32_t zn = MODE == kPAsym ? *reinterpret_cast<const uint32_t*>(st + oz) : 0u;
+      if constexpr (kMidFirst) {
+        __builtin_amdgcn_sched_barrier(0);
+        mid(0);
+      }
 #pragma unroll
       for (int j = 0; j <= NSB; ++j) {
         v4f cj[RB];
-        float scj = 0.f, cfj = 0.f;
+        float scj = 0.f;
         if (j < NSB) {
           const v8i b = bn;
           scj = scn;
-          if (MODE == kPAsym) cfj = 15.0f - 2.0f * (float)((zn >> zsh) & 15u);
           if (j + 1 < NSB) {
             bn = lds_operand(st + ob + (j + 1) * 2048, 0);
             scn = f16_to_f32(*reinterpret_cast<const uint16_t*>(st + os + (j + 1) * 32));
-            if (MODE == kPAsym) zn = *reinterpret_cast<const uint32_t*>(st + oz + (j + 1) * 8);
           }
           __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-          for (int rb = 0; rb < RB; ++rb) cj[rb] = mfma_f8f8(a[rb], b, MODE == kPSym ? pre[rb] : zero4);
-          if (j < 2) mid(j);
+          for (int rb = 0; rb < RB; ++rb) cj[rb] = mfma_f8f8(a[rb], b, pre[rb]);
+          if (j < 2 && (j > 0 || !kMidFirst)) mid(j);
         }
         if (j > 0) {
 #pragma unroll
           for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-              if (MODE == kPSym)
-                acc[rb][j - 1][r] += scp * cp[rb][r];
-              else
-                acc[rb][j - 1][r] += scp * (cp[rb][r] + cfp * pre[rb][r]);
-            }
+            for (int r = 0; r < 4; ++r) acc[rb][j - 1][r] += scp * cp[rb][r];
           // issue the previous strip's scale FMAs between this strip's MFMAs (one MFMA, then four
           // VALU ops), so they run while the matrix pipe works instead of after it
           if (j < NSB) {
@@ -348,7 +491,6 @@ gemm_dma_kernel(const GemmArgs p) {
 #pragma unroll
           for (int rb = 0; rb < RB; ++rb) cp[rb] = cj[rb];
           scp = scj;
-          cfp = cfj;
         }
       }
     }
@@ -362,46 +504,38 @@ gemm_dma_kernel(const GemmArgs p) {
   // while the step's first MFMAs wait (1-4% on configs[3] and configs[5] shapes). The weight
   // registers go first because the unpack one step later waits on them, while the A DMAs are only
   // waited for at the end of the next step (weights first: configs[3] 2-8% faster, MoE T=4096 2%).
-  auto step = [&](auto C, int kt) __attribute__((always_inline)) {
+  auto step = [&](auto C, int kt, auto Tail) __attribute__((always_inline)) {
+    if (decltype(Tail)::value && kt >= KT) return;
     constexpr int c = decltype(C)::value, n1 = (c + 1) % 3, n2 = (c + 2) % 3;
     static_assert(kFp4 || NSB >= 2, "int4 steps issue their loads after strips 0 and 1");
+    const int valid = decltype(Tail)::value && kKTail && kt == KT - 1 ? ktail : kTileK;
     if constexpr (kFp4) {
       compute(C, [&](int rb) __attribute__((always_inline)) {
-        if (rb == 1) issue(IC<n2>{}, kt + 2);
-      });
+        // past the last step nothing is loaded (unlike int4 below, whose unpack the branch would hold
+        // back, MXFP4 is 2% faster at M=1000 K=N=4096 with the branch than with empty loads)
+        if (rb == 1 && (!decltype(Tail)::value || kt + 2 < KT)) issue(IC<n2>{}, kt + 2, 3, Tail);
+      }, valid);
     } else {
       compute(C, [&](int j) __attribute__((always_inline)) {
         if (j == 0) {
-          issue(IC<n2>{}, kt + 2, 2);
-          commit(IC<n1>{}, IC<n1>{});
+          issue(IC<n2>{}, kt + 2, 2, Tail);
+          if (!decltype(Tail)::value || kt + 1 < KT) commit(IC<n1>{}, IC<n1>{});
         } else {
-          issue(IC<n2>{}, kt + 2, 1);
+          issue(IC<n2>{}, kt + 2, 1, Tail);
         }
-      });
+      }, valid);
     }
     __builtin_amdgcn_sched_barrier(0);
-    wait_vm_lgkm0<NOPS>();
+    if (kFp4 && decltype(Tail)::value && kt + 2 >= KT) wait_vm_lgkm0<0>();
+    else wait_vm_lgkm0<NOPS>();
     __builtin_amdgcn_s_barrier();
   };
-  // the same step near the end of K: loads only while steps remain, a full wait otherwise
-  auto step_tail = [&](auto C, int kt) __attribute__((always_inline)) {
-    constexpr int c = decltype(C)::value, n1 = (c + 1) % 3, n2 = (c + 2) % 3;
-    if (kt >= KT) return;
-    const bool more = kt + 2 < KT;
-    if (more) issue(IC<n2>{}, kt + 2);
-    compute(C, [&](int j) __attribute__((always_inline)) {
-      if (j == 0 && kt + 1 < KT) commit(IC<n1>{}, IC<n1>{});
-    });
-    if (more) wait_vm_lgkm0<NOPS>();
-    else wait_vm_lgkm0<0>();
-    __builtin_amdgcn_s_barrier();
-  };
-
   // prologue: steps 0 and 1 in flight, step 0 in LDS. The epilogue rows' loads above are older
   // than both, so the counted wait covers them; their LDS writes land before the first step's
   // barrier (its wait takes lgkmcnt to 0), long before the epilogue reads them.
-  issue(IC<0>{}, 0);
-  issue(IC<1>{}, 1);
+  issue(IC<0>{}, 0, 3, IC<0>{});
+  issue(IC<1>{}, 1, 3, IC<1>{});
+  if constexpr (kLutZ) lds_barrier();  // the zero-point table, before the first decode reads it
   commit(IC<0>{}, IC<0>{});
   wait_vm_lgkm0<NOPS>();
   if (er < BM) {
@@ -410,16 +544,19 @@ gemm_dma_kernel(const GemmArgs p) {
   }
   __builtin_amdgcn_s_barrier();
   int kt = 0;
-  for (; kt + 4 < KT; kt += 3) {
-    step(IC<0>{}, kt);
-    step(IC<1>{}, kt + 1);
-    step(IC<2>{}, kt + 2);
+  for (; kt + (kKTail ? 5 : 4) < KT; kt += 3) {  // kKTail: loads of steps up to KT - 2 only
+    step(IC<0>{}, kt, IC<0>{});
+    step(IC<1>{}, kt + 1, IC<0>{});
+    step(IC<2>{}, kt + 2, IC<0>{});
   }
-  step_tail(IC<0>{}, kt);
-  step_tail(IC<1>{}, kt + 1);
-  step_tail(IC<2>{}, kt + 2);
-  step_tail(IC<0>{}, kt + 3);
-  step_tail(IC<1>{}, kt + 4);
+  step(IC<0>{}, kt, IC<1>{});
+  step(IC<1>{}, kt + 1, IC<1>{});
+  step(IC<2>{}, kt + 2, IC<1>{});
+  step(IC<0>{}, kt + 3, IC<1>{});
+  if constexpr (kKTail) step(IC<1>{}, kt + 4, IC<1>{});
+  // the empty loads of the last two steps write LDS too: all landed before the epilogue reuses it
+  wait_vm_lgkm0<0>();
+  __builtin_amdgcn_s_barrier();
 
   // epilogue: lane holds rows 4*(lane>>4)+r of each row block, channel (lane & 15) of each strip
   const int64_t row0 = blk_row0 + (int64_t)wm * RB * 16;
@@ -465,11 +602,23 @@ static int launch_dma_cfg(const GemmArgs& p, int64_t row_tiles, hipStream_t stre
   return launch_dma_cfg_at<WM, WN, RB, NSB, MODE, false>(p, row_tiles, stream);
 }
 
+// the modes whose weights are decoded with their zero point: g128 with zero points, g64 and g32
+template <int WM, int WN, int RB, int NSB>
+static int launch_dma_lut(const GemmArgs& p, int mode, int64_t row_tiles, hipStream_t stream) {
+  switch (mode) {
+    case kPAsym: return launch_dma_cfg_at<WM, WN, RB, NSB, kPAsym>(p, row_tiles, stream);
+    case kPG64: return launch_dma_cfg_at<WM, WN, RB, NSB, kPG64>(p, row_tiles, stream);
+    case kPG64Z: return launch_dma_cfg_at<WM, WN, RB, NSB, kPG64Z>(p, row_tiles, stream);
+    case kPG32: return launch_dma_cfg_at<WM, WN, RB, NSB, kPG32>(p, row_tiles, stream);
+    default: return launch_dma_cfg_at<WM, WN, RB, NSB, kPG32Z>(p, row_tiles, stream);
+  }
+}
+
 template <int WM, int WN, int RB, int NSB>
 static int launch_dma_modes(const GemmArgs& p, int mode, int64_t row_tiles, hipStream_t stream) {
   if (mode == kPSym) return launch_dma_cfg<WM, WN, RB, NSB, kPSym>(p, row_tiles, stream);
-  if (mode == kPAsym) return launch_dma_cfg<WM, WN, RB, NSB, kPAsym>(p, row_tiles, stream);
-  return launch_dma_cfg<WM, WN, RB, NSB, kPE8M0>(p, row_tiles, stream);
+  if (mode == kPE8M0) return launch_dma_cfg<WM, WN, RB, NSB, kPE8M0>(p, row_tiles, stream);
+  return launch_dma_lut<WM, WN, RB, NSB>(p, mode, row_tiles, stream);
 }
 // grouped tiles: A rows gathered through the sorted ids, or (p.a_tiled, symmetric int4, A rows at
 // their padded positions: gemm2) the padded rows' codes in operand order with their seeds
@@ -477,37 +626,39 @@ template <int WM, int WN, int RB, int NSB>
 static int launch_dma_modes_grouped(const GemmArgs& p, int mode, int64_t row_tiles, hipStream_t stream) {
   if (mode == kPSym && p.a_tiled) return launch_dma_cfg_at<WM, WN, RB, NSB, kPSym, true>(p, row_tiles, stream);
   if (mode == kPSym) return launch_dma_cfg_at<WM, WN, RB, NSB, kPSym>(p, row_tiles, stream);
-  if (mode == kPAsym) return launch_dma_cfg_at<WM, WN, RB, NSB, kPAsym>(p, row_tiles, stream);
-  return launch_dma_cfg_at<WM, WN, RB, NSB, kPE8M0>(p, row_tiles, stream);
+  if (mode == kPE8M0) return launch_dma_cfg_at<WM, WN, RB, NSB, kPE8M0>(p, row_tiles, stream);
+  return launch_dma_lut<WM, WN, RB, NSB>(p, mode, row_tiles, stream);
 }
 
-// Formats and shapes as launch_prefill_lds, plus at least three K steps (the pipeline's depth).
+// int4 with groups of 32, 64 and 128+ and MXFP4, on 16-byte aligned rows; kErrUnsupported otherwise.
 // bm_rows: rows per workgroup the caller requires (grouped: 64 or 128; 0 for dense).
 int launch_prefill_dma(const GemmArgs& p, int64_t rows_to_cover, int bm_rows, hipStream_t stream) {
   int mode;
   if (p.wfmt == kInt4 && p.sfmt == kScaleF16 && p.group % kTileK == 0)
     mode = p.zeros ? kPAsym : kPSym;
+  else if (p.wfmt == kInt4 && p.sfmt == kScaleF16 && p.group == 64)
+    mode = p.zeros ? kPG64Z : kPG64;
+  else if (p.wfmt == kInt4 && p.sfmt == kScaleF16 && p.group == 32)
+    mode = p.zeros ? kPG32Z : kPG32;
   else if (p.wfmt == kE2M1 && p.sfmt == kScaleE8M0)
     mode = kPE8M0;
   else
     return kErrUnsupported;
   if (p.silu && (p.N / kTileN) % 2) return kErrUnsupported;
-  if (p.K % kTileK || p.KT < 3) return kErrUnsupported;
+  // a K that ends inside its first tile has no tile before it for the chunks past K to read
+  if (p.K % kTileK && (p.KT < 2 || p.a_tiled)) return kErrUnsupported;
+  // grouped rows: a workgroup's rows must sit inside one align block (one expert)
   if (p.sorted_ids && bm_rows != 64 && bm_rows != 128) return kErrUnsupported;
+  // 32-bit offsets within one matrix
   if ((int64_t)p.N * p.KT * 64 >= (int64_t)1 << 31) return kErrUnsupported;
-  if (p.ldx % 16) return kErrUnsupported;  // A rows are read in 16-byte pieces
-  // W4A8_PREFILL_DMA=0 leaves every call to the register-staged kernel (A/B measurements)
-  static const bool enabled = [] {
-    const char* e = getenv("W4A8_PREFILL_DMA");
-    return !(e && atoi(e) == 0);
-  }();
-  if (!enabled) return kErrUnsupported;
+  if (p.ldx % 16) return kErrUnsupported;  // A rows are read in 16-byte pieces, at 32-bit offsets
+  if ((p.a_by_token ? p.num_slots / p.top_k : p.M) * p.ldx > (int64_t)0xffffffff) return kErrUnsupported;
   // Tiles (waves WM x WN, wave tile RB x NSB blocks of 16): the largest whose three stages fit
   // the 160 KiB of LDS and whose registers fit two waves per SIMD. MXFP4 keeps its weights as fp4
   // in LDS and its accumulators are the only per-step state, so it takes 64 x 128 wave tiles
   // (256 x 256 per workgroup: a quarter less LDS read per MFMA than 64 x 64); int4 holds the
   // unpacked fp8 weights plus the partials of its per-group scaling and stays at 64 x 64.
-  if (p.a_tiled && (p.sorted_ids ? (mode != kPSym || p.a_by_token != 0) : (bm_rows != 0 || mode == kPAsym)))
+  if (p.a_tiled && (p.sorted_ids ? (mode != kPSym || p.a_by_token != 0) : (bm_rows != 0 || (mode != kPSym && mode != kPE8M0))))
     return kErrUnsupported;
   if (bm_rows == 64) return launch_dma_modes_grouped<2, 4, 2, 2>(p, mode, (rows_to_cover + 63) / 64, stream);
   if (bm_rows == 128) return launch_dma_modes_grouped<2, 4, 4, 4>(p, mode, (rows_to_cover + 127) / 128, stream);
@@ -536,6 +687,13 @@ int launch_prefill_dma(const GemmArgs& p, int64_t rows_to_cover, int bm_rows, hi
     return launch_dma_modes<2, 4, 2, 2>(p, mode, (rows_to_cover + 63) / 64, stream);
   if (mode == kPE8M0) return launch_dma_cfg<4, 2, 4, 8, kPE8M0>(p, (rows_to_cover + 255) / 256, stream);
   return launch_dma_modes<4, 2, 4, 4>(p, mode, (rows_to_cover + 255) / 256, stream);
+}
+
+// The LDS-staged kernels: NVFP4 on the fp16 MFMA, else the DMA-staged pipeline; kErrUnsupported for
+// what neither takes (the per-wave kernel serves it).
+int launch_prefill_staged(const GemmArgs& p, int64_t rows_to_cover, int bm_rows, hipStream_t stream) {
+  const int rc = launch_prefill_nv(p, rows_to_cover, bm_rows, stream);
+  return rc != kErrUnsupported ? rc : launch_prefill_dma(p, rows_to_cover, bm_rows, stream);
 }
 
 }  // namespace w4a8

@@ -142,6 +142,11 @@ gemm_nv_kernel(const GemmArgs p) {
     const bool ok = lrow_source(p, blk_row0 + (b >> 1) * 16 + (lane & 15), ar);
     a_voff[i] = (uint32_t)((ok ? ar : 0) * p.ldx) + (b & 1) * 64 + 16 * (lane >> 4);
   }
+  // a K that is no multiple of 128: the last tile's chunks past K read the tile before (in bounds) and
+  // are cleared in the operand read
+  const int ktail = K - (KT - 1) * kTileK;
+  const uint32_t a_back = (wave & 1) * 64 + 16 * (lane >> 4) >= ktail ? kTileK : 0;
+  static_assert(NW % 2 == 0, "a wave's A blocks are all the same half");
   // B: fp4 tile lane c = tid + i*T is lane c & 63 of strip c >> 6; its 16 bytes are the two
   // 16-element blocks 2q', 2q'+1 (q' = lane >> 4) of channel lane & 15; their scale bytes are
   // rows 2q' and 2q'+1 of the step's 8 scale rows
@@ -162,15 +167,16 @@ gemm_nv_kernel(const GemmArgs p) {
     constexpr int R = decltype(I)::value;
     unsigned char* st = astage(I);
     const uint32_t so_a = (uint32_t)__builtin_amdgcn_readfirstlane(kt * kTileK);
+    const uint32_t back = a_back & (uint32_t)__builtin_amdgcn_readfirstlane(kt == KT - 1 ? -1 : 0);
 #pragma unroll
-    for (int i = 0; i < A_PER; ++i) lds_dma16(rs_a, st + (wave + i * NW) * 1024, a_voff[i], so_a);
+    for (int i = 0; i < A_PER; ++i) lds_dma16(rs_a, st + (wave + i * NW) * 1024, a_voff[i] - back, so_a);
     const uint32_t so_w = (uint32_t)__builtin_amdgcn_readfirstlane(kt * kTileBytes);
     const uint32_t so_s = (uint32_t)__builtin_amdgcn_readfirstlane(kt * 8 * N);
 #pragma unroll
     for (int i = 0; i < B_PER; ++i) {
       rw[R][i] = bload128v(rs_w, w_voff[i], so_w);
-      rs0[R][i] = bload8(rs_s, s_voff[i], so_s);
-      rs1[R][i] = bload8(rs_s, s_voff[i] + N, so_s);
+      rs0[R][i] = bload8(rs_s, s_voff[i] + so_s, 0);  // scale rows past K: out of range, so zeros
+      rs1[R][i] = bload8(rs_s, s_voff[i] + N + so_s, 0);
     }
   };
   // B registers of set R -> fp16 operands in B stage BI
@@ -209,7 +215,7 @@ gemm_nv_kernel(const GemmArgs p) {
   // the four fp16 sub-steps of a K step from A stage I and B stage BI (each sub-step's B fragments
   // read one sub-step ahead of its MFMAs); mid(s) runs after sub-step s's MFMAs are issued (the
   // next step's B decode and later loads overlap them)
-  auto compute = [&](auto I, auto BI, auto mid) __attribute__((always_inline)) {
+  auto compute = [&](auto I, auto BI, auto mid, bool last) __attribute__((always_inline)) {
     const unsigned char* sa = astage(I);
     const unsigned char* bs = bstage(BI);
     v8h bc[NSB], bn[NSB];
@@ -220,6 +226,8 @@ gemm_nv_kernel(const GemmArgs p) {
     for (int rb = 0; rb < RB; ++rb) {
       alo[rb] = *reinterpret_cast<const uint4*>(sa + oa + rb * 2048);
       ahi[rb] = *reinterpret_cast<const uint4*>(sa + oa + rb * 2048 + 1024);
+      if (last && 16 * (lane >> 4) >= ktail) alo[rb] = make_uint4(0u, 0u, 0u, 0u);
+      if (last && 64 + 16 * (lane >> 4) >= ktail) ahi[rb] = make_uint4(0u, 0u, 0u, 0u);
     }
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
@@ -254,7 +262,7 @@ gemm_nv_kernel(const GemmArgs p) {
     compute(C, D, [&](int s) __attribute__((always_inline)) {
       if (s == 0) commit(IC<n1>{}, IC<1 - d>{});
       if (s == 1) issue(IC<n2>{}, kt + 2);
-    });
+    }, false);
     __builtin_amdgcn_sched_barrier(0);
     wait_vm_lgkm0<NOPS>();
     __builtin_amdgcn_s_barrier();
@@ -267,7 +275,7 @@ gemm_nv_kernel(const GemmArgs p) {
     if (more) issue(IC<n2>{}, kt + 2);
     compute(C, D, [&](int s) __attribute__((always_inline)) {
       if (s == 0 && kt + 1 < KT) commit(IC<n1>{}, IC<1 - d>{});
-    });
+    }, kt + 1 == KT);
     if (more) wait_vm_lgkm0<NOPS>();
     else wait_vm_lgkm0<0>();
     __builtin_amdgcn_s_barrier();
@@ -327,17 +335,18 @@ static int launch_nv_cfg(const GemmArgs& p, int64_t row_tiles, hipStream_t strea
   return hipGetLastError() == hipSuccess ? kOk : kErrHip;
 }
 
-// NVFP4 (e2m1 codes, e4m3 block-16 scales, the f32 global in the zeros slot) with whole 128-K
-// steps, at least two of them, and 16-byte aligned activation rows; kErrUnsupported otherwise.
+// NVFP4 (e2m1 codes, e4m3 block-16 scales, the f32 global in the zeros slot) with at least two K
+// steps and 16-byte aligned activation rows; kErrUnsupported otherwise.
 // bm_rows: rows per workgroup the caller requires (grouped: 64 or 128; 0 for dense).
 int launch_prefill_nv(const GemmArgs& p, int64_t rows_to_cover, int bm_rows, hipStream_t stream) {
   if (!(p.wfmt == kE2M1 && p.sfmt == kScaleE4M3 && p.group == 16 && p.zeros)) return kErrUnsupported;
   if (p.silu && (p.N / kTileN) % 2) return kErrUnsupported;
-  if (p.K % kTileK || p.KT < 2) return kErrUnsupported;
+  if (p.KT < 2) return kErrUnsupported;
   if (p.sorted_ids && bm_rows != 64 && bm_rows != 128) return kErrUnsupported;
   if ((int64_t)p.N * p.KT * 64 >= (int64_t)1 << 31) return kErrUnsupported;
   if ((p.K / 16) * p.N >= (int64_t)1 << 32) return kErrUnsupported;
   if (p.ldx % 16) return kErrUnsupported;
+  if ((p.a_by_token ? p.num_slots / p.top_k : p.M) * p.ldx > (int64_t)0xffffffff) return kErrUnsupported;
   // W4A8_PREFILL_NV=0 leaves NVFP4 to the per-wave kernel (A/B measurements)
   static const bool enabled = [] {
     const char* e = getenv("W4A8_PREFILL_NV");

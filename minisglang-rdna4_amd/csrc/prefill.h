@@ -1,5 +1,5 @@
-// Pieces shared by the LDS-staged prefill / grouped GEMM kernels (gemm_prefill_lds.hip,
-// gemm_prefill_dma.hip): weight-format modes, grouped-row lookup, the silu epilogue, the 1 KiB
+// Pieces shared by the LDS-staged prefill / grouped GEMM kernels (gemm_prefill_dma.hip,
+// gemm_prefill_nv.hip): weight-format modes, grouped-row lookup, the silu epilogue, the 1 KiB
 // MFMA operand read and the per-stage LDS layout.
 #pragma once
 #include <type_traits>
@@ -19,7 +19,47 @@ __device__ __forceinline__ void wait_vm_lgkm0() {
   __builtin_amdgcn_s_waitcnt((N & 15) | (7 << 4) | (0 << 8) | ((N >> 4) << 14));
 }
 
-constexpr int kPSym = 0, kPAsym = 1, kPE8M0 = 2;
+// int4 without / with zero points (groups of 128+), MXFP4, int4 with groups of 64 and 32 (Z: with
+// zero points)
+constexpr int kPSym = 0, kPAsym = 1, kPE8M0 = 2, kPG64 = 3, kPG64Z = 4, kPG32 = 5, kPG32Z = 6;
+constexpr int prefill_gpt(int mode) { return mode == kPG32 || mode == kPG32Z ? 4 : mode == kPG64 || mode == kPG64Z ? 2 : 1; }
+constexpr bool prefill_lut_zeros(int mode) { return mode == kPAsym || mode == kPG64Z || mode == kPG32Z; }
+constexpr bool prefill_lut(int mode) { return prefill_lut_zeros(mode) || mode == kPG64 || mode == kPG32; }
+
+// Decode of an int4 tile with its zero point: e4m3(q - z), exact for every q and z (|q - z| <= 15 has
+// four significant bits), so the MFMA needs no row-sum term. A nibble's sign-magnitude code (see
+// w4a8_common.h) is q = 8 + t for a clear sign bit and q = 7 - t for a set one, t its low three bits:
+// the table of zero point z holds e4m3(8 + t - z) in x, y and e4m3(7 - t - z) in z, w.
+__device__ __forceinline__ uint4 zero_point_lut(int z) {
+  uint32_t d[4] = {0, 0, 0, 0};
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    const int v = (i < 8 ? 8 + i : 15 - i) - z;  // d[2..3]: 7 - t, t = i - 8
+    const int a = v < 0 ? -v : v;
+    // e4m3 of a small integer: exponent 7 + log2, three mantissa bits
+    const int e = a ? 31 - __builtin_clz((unsigned)a) : 0;
+    const uint32_t m = a ? (uint32_t)(((7 + e) << 3) | (((a << 3) >> e) & 7)) : 0u;
+    d[i >> 2] |= (m | (v < 0 ? 0x80u : 0u)) << (8 * (i & 3));
+  }
+  return make_uint4(d[0], d[1], d[2], d[3]);
+}
+// 4 codes in the low nibbles of w's bytes -> 4 e4m3 bytes: both tables looked up, the sign bit picks
+// (a selector byte of 12 or more reads as constant 0, so the mask is one v_perm as well)
+__device__ __forceinline__ uint32_t decode_lut4(uint32_t w, const uint4& t) {
+  const uint32_t i = w & 0x07070707u;
+  const uint32_t pos = __builtin_amdgcn_perm(t.y, t.x, i), neg = __builtin_amdgcn_perm(t.w, t.z, i);
+  const uint32_t m = __builtin_amdgcn_perm(0xffffffffu, 0u, (w & 0x08080808u) | 0x04040404u);  // ff: sign clear
+  return (pos & m) | (neg & ~m);
+}
+// 16 stored bytes -> 8-VGPR fp8 operand; t0 / t1 the tables of the first and second 16 codes' groups
+__device__ __forceinline__ v8i unpack_tile_lut(const uint4& raw, const uint4& t0, const uint4& t1) {
+  v8i b;
+  b[0] = (int)decode_lut4(raw.x, t0); b[1] = (int)decode_lut4(raw.x >> 4, t0);
+  b[2] = (int)decode_lut4(raw.y, t0); b[3] = (int)decode_lut4(raw.y >> 4, t0);
+  b[4] = (int)decode_lut4(raw.z, t1); b[5] = (int)decode_lut4(raw.z >> 4, t1);
+  b[6] = (int)decode_lut4(raw.w, t1); b[7] = (int)decode_lut4(raw.w >> 4, t1);
+  return b;
+}
 
 __device__ __forceinline__ bool lrow_source(const GemmArgs& p, int64_t r, int64_t& ar) {
   if (!p.sorted_ids) {
@@ -59,9 +99,8 @@ template <int BM, int BN, int MODE>
 struct LdsStage {
   static constexpr int kA = BM * 128;                          // fp8 operand order
   static constexpr int kB = MODE == kPE8M0 ? BN * 64 : BN * 128;  // fp4 bytes, or unpacked fp8
-  static constexpr int kS = MODE == kPE8M0 ? BN * 4 : BN * 2;  // E8M0 [strip][lane] | fp16 [strip][16]
-  static constexpr int kZ = MODE == kPAsym ? BN / 2 : 0;       // zero words [strip][2]
-  static constexpr int kBytes = kA + kB + kS + kZ;
+  static constexpr int kS = MODE == kPE8M0 ? BN * 4 : BN * 2 * prefill_gpt(MODE);  // E8M0 [strip][lane] | fp16 [group][strip][16]
+  static constexpr int kBytes = kA + kB + kS;
 };
 
 // Epilogue of the LDS-staged GEMMs. Lane layout: rows row0 + rb*16 + 4*(lane>>4) + r, channel

@@ -1,0 +1,77 @@
+"""The LDS-staged prefill kernels at the edges of what they take: int4 groups of 32 and 64 (four
+16x16x32 MFMAs per K tile, weights decoded as e4m3(q - z)), zero points with groups of 128, a K that
+ends inside a 128-wide tile, and one or two K tiles; dense and grouped, against the CPU oracle."""
+import numpy as np
+import pytest
+import torch
+
+import synth
+from test_gpu_dense import assert_close_to_oracle
+from test_gpu_moe import _stagewise
+
+pytestmark = pytest.mark.gpu
+
+
+def _weight(fmt, g, N, K, seed, E=None):
+    """(w, s, z, e2m1, nvfp4) on the CPU, op layout."""
+    if fmt == "mxfp4":
+        return (*synth.mxfp4_weight(N, K, seed=seed, E=E), None, True, False)
+    if fmt == "nvfp4":
+        return (*synth.nvfp4_weight(N, K, seed=seed, E=E), True, True)
+    return (*synth.int4_weight(N, K, g, seed=seed, asym=fmt == "asym", scale_floor=1e-4, E=E), False, False)
+
+
+FMTS = [("sym", 32), ("asym", 32), ("sym", 64), ("asym", 64), ("asym", 128), ("asym", 256), ("mxfp4", 32), ("nvfp4", 16)]
+
+
+# K: one tile, two, a tail of 32 to 96 behind one and three tiles, more tiles than the K loop unrolls;
+# M and N: one row block and strip past a tile's edge, row tiles of 64, 128 and 256
+@pytest.mark.parametrize("fmt,g", FMTS)
+@pytest.mark.parametrize("M,N,K", [(17, 16, 128), (65, 144, 256), (130, 272, 160), (40, 1040, 480), (300, 528, 1088),
+                                   (257, 4112, 896)])
+def test_prefill_groups_and_k_tails(kernels, oracle, dev, fmt, g, M, N, K):
+    if K % g:
+        pytest.skip("group does not divide K")
+    w, s, z, e2, nv = _weight(fmt, g, N, K, seed=M + N + K)
+    # no x50 outlier channel: the MFMA aligns its products to the largest one and drops what falls below
+    # about 2^-24 of it, so with one product 50 times the rest the distance grows 5 to 7 times (MXFP4 at
+    # M=40 N=1040 K=480: 5.3e-4 against 7.5e-5, the same bits from the decode kernel), past the bar that
+    # assert_close_to_oracle derives for sums of like terms
+    x = synth.activations(M, K, seed=M + K)
+    xq, xs = oracle.act_quant(synth.bits16(x), 0)
+    ref = oracle.gemm(xq, xs, w.numpy(), s.view(torch.uint8).numpy() if nv else s.numpy(),
+                      None if z is None else z.numpy(), g, e2, nv)
+    tiles, sd = kernels.repack_w4(w.to(dev), weight_is_e2m1=e2), s.to(dev)
+    zd = None if z is None else z.to(dev)
+    out = kernels.w4a8_linear(x.to(dev), tiles, sd, zd, g, weight_is_e2m1=e2, kernel="wmma_tiled_tuned")
+    rows = torch.tensor([0, M // 2, M - 1])  # the same rows in a smaller call, and beside a row of NaN
+    xp = torch.cat([x[rows], torch.full((1, K), float("nan"), dtype=x.dtype)])
+    part = kernels.w4a8_linear(xp.to(dev), tiles, sd, zd, g, weight_is_e2m1=e2, kernel="wmma_tiled_tuned")
+    torch.cuda.synchronize()
+    assert_close_to_oracle(out, ref, f"{fmt} g={g} M={M} N={N} K={K}")
+    assert torch.equal(out[rows.to(dev)], part[:3]), "a row's bits depend on the rows beside it"
+
+
+@pytest.mark.parametrize("fmt,g", FMTS)
+@pytest.mark.parametrize("h,i,bm", [(320, 96, 64), (256, 160, 128)])
+def test_moe_groups_and_k_tails(kernels, oracle, dev, fmt, g, h, i, bm):
+    """Grouped tiles of 64 and 128 rows, both GEMMs with a ragged K (h = 320 and i = 96, 160)."""
+    if h % g or i % g:
+        g = max(d for d in (16, 32) if d <= g)
+        if fmt == "asym" and g == 16:
+            g = 32
+    e, T = 4, 150
+    w13, s13, z13, e2, nv = _weight(fmt, g, 2 * i, h, seed=h + i, E=e)
+    w2, s2, z2, _, _ = _weight(fmt, g, h, i, seed=h + i + 1, E=e)
+    x = synth.activations(T, h, seed=7)
+    lg = synth.router_logits(T, e, seed=8)
+    zz = [None if z is None else (z.view(torch.int32) if nv else z).to(dev) for z in (z13, z2)]
+    res = kernels._moe_forward(x.to(dev), kernels.repack_w4(w13.to(dev), e2), s13.to(dev), zz[0],
+                               kernels.repack_w4(w2.to(dev), e2), s2.to(dev), zz[1], lg.to(dev), 2, True,
+                               weight_is_e2m1=e2, block_m=bm)
+    torch.cuda.synchronize()
+    u8 = (lambda t: t.view(torch.uint8)) if nv else (lambda t: t)
+    rel1, rel2, _ = _stagewise(kernels, oracle, res, x, w13, u8(s13), z13, w2, u8(s2), z2, list(range(0, T, 5)),
+                               e2m1=e2, nvfp4=nv)
+    assert rel1 <= 2e-3 and rel2 <= 2e-3  # the bars of test_gpu_moe: bf16 rounding alone is 1.65e-3
+    assert np.isfinite(res["out"].float().cpu().numpy()).all()
