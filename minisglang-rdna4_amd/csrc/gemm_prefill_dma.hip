@@ -29,7 +29,15 @@
 
 namespace w4a8 {
 
-template <int WM, int WN, int RB, int NSB, int MODE, bool AT>
+template <int I, int N, typename F>
+__device__ __forceinline__ void for_stages(F f) {
+  if constexpr (I < N) {
+    f(IC<I>{});
+    for_stages<I + 1, N>(f);
+  }
+}
+
+template <int WM, int WN, int RB, int NSB, int NST, int MODE, bool AT>
 __global__ void __launch_bounds__(WM * WN * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
 gemm_dma_kernel(const GemmArgs p) {
   constexpr int T = WM * WN * 64, NW = WM * WN;
@@ -60,13 +68,19 @@ gemm_dma_kernel(const GemmArgs p) {
   constexpr int ZL = kLutZ ? (GPT > 1 ? 2 : 1) : 0;    // zero words per chunk: its one or two groups
   constexpr int NOPS = (kFp4 ? S_DMA + A_PER + B_DMA : A_PER + B_PER * (1 + ZL) + 1) + (kSeedL ? 1 : 0);
 
+  // NST stages, each its own array; loads run D steps ahead
+  constexpr int D = NST - 1;
+  static_assert(NST == 3 || NST == 4, "stages");
   __shared__ __align__(16) unsigned char st0[kStage];
   __shared__ __align__(16) unsigned char st1[kStage];
   __shared__ __align__(16) unsigned char st2[kStage];
+  __shared__ __align__(16) unsigned char st3[NST > 3 ? kStage : 16];
   auto stage = [&](auto I) __attribute__((always_inline)) -> unsigned char* {
-    if constexpr (decltype(I)::value == 0) return st0;
-    else if constexpr (decltype(I)::value == 1) return st1;
-    else return st2;
+    constexpr int i = decltype(I)::value;
+    if constexpr (i == 0) return st0;
+    else if constexpr (i == 1) return st1;
+    else if constexpr (i == 2) return st2;
+    else return st3;
   };
 
   const int lane = threadIdx.x & 63;
@@ -219,9 +233,9 @@ gemm_dma_kernel(const GemmArgs p) {
   }
 
   // int4 register sets, one per stage index (two are live at a time)
-  v4u rbw[3][kFp4 ? 1 : B_PER];
-  uint4 rsc[3];
-  uint32_t rzp[3][kLutZ ? B_PER : 1][ZL > 0 ? ZL : 1];
+  v4u rbw[NST][kFp4 ? 1 : B_PER];
+  uint4 rsc[NST];
+  uint32_t rzp[NST][kLutZ ? B_PER : 1][ZL > 0 ? ZL : 1];
 
   // loads of K step kt into stage I (DMA) / register set I (int4 weights, scales, zeros)
   // part: 1 = the A DMAs (and fp4 strips / E8M0 bytes), 2 = the int4 weight, scale and zero loads.
@@ -506,55 +520,51 @@ gemm_dma_kernel(const GemmArgs p) {
   // waited for at the end of the next step (weights first: configs[3] 2-8% faster, MoE T=4096 2%).
   auto step = [&](auto C, int kt, auto Tail) __attribute__((always_inline)) {
     if (decltype(Tail)::value && kt >= KT) return;
-    constexpr int c = decltype(C)::value, n1 = (c + 1) % 3, n2 = (c + 2) % 3;
+    constexpr int c = decltype(C)::value, n1 = (c + 1) % NST, nd = (c + D) % NST;
     static_assert(kFp4 || NSB >= 2, "int4 steps issue their loads after strips 0 and 1");
     const int valid = decltype(Tail)::value && kKTail && kt == KT - 1 ? ktail : kTileK;
     if constexpr (kFp4) {
       compute(C, [&](int rb) __attribute__((always_inline)) {
         // past the last step nothing is loaded (unlike int4 below, whose unpack the branch would hold
         // back, MXFP4 is 2% faster at M=1000 K=N=4096 with the branch than with empty loads)
-        if (rb == 1 && (!decltype(Tail)::value || kt + 2 < KT)) issue(IC<n2>{}, kt + 2, 3, Tail);
+        if (rb == 1 && (!decltype(Tail)::value || kt + D < KT)) issue(IC<nd>{}, kt + D, 3, Tail);
       }, valid);
     } else {
       compute(C, [&](int j) __attribute__((always_inline)) {
         if (j == 0) {
-          issue(IC<n2>{}, kt + 2, 2, Tail);
+          issue(IC<nd>{}, kt + D, 2, Tail);
           if (!decltype(Tail)::value || kt + 1 < KT) commit(IC<n1>{}, IC<n1>{});
         } else {
-          issue(IC<n2>{}, kt + 2, 1, Tail);
+          issue(IC<nd>{}, kt + D, 1, Tail);
         }
       }, valid);
     }
     __builtin_amdgcn_sched_barrier(0);
-    if (kFp4 && decltype(Tail)::value && kt + 2 >= KT) wait_vm_lgkm0<0>();
-    else wait_vm_lgkm0<NOPS>();
+    if (kFp4 && decltype(Tail)::value && kt + D >= KT) wait_vm_lgkm0<0>();
+    else wait_vm_lgkm0<NOPS * (D - 1)>();
     __builtin_amdgcn_s_barrier();
   };
   // prologue: steps 0 and 1 in flight, step 0 in LDS. The epilogue rows' loads above are older
   // than both, so the counted wait covers them; their LDS writes land before the first step's
   // barrier (its wait takes lgkmcnt to 0), long before the epilogue reads them.
   issue(IC<0>{}, 0, 3, IC<0>{});
-  issue(IC<1>{}, 1, 3, IC<1>{});
+  for_stages<1, D>([&](auto I) __attribute__((always_inline)) { issue(I, decltype(I)::value, 3, IC<1>{}); });
   if constexpr (kLutZ) lds_barrier();  // the zero-point table, before the first decode reads it
   commit(IC<0>{}, IC<0>{});
-  wait_vm_lgkm0<NOPS>();
+  wait_vm_lgkm0<NOPS * (D - 1)>();
   if (er < BM) {
     e_sc[er] = er_sc;
     e_ok[er] = er_ok ? 1 : 0;
   }
   __builtin_amdgcn_s_barrier();
   int kt = 0;
-  for (; kt + (kKTail ? 5 : 4) < KT; kt += 3) {  // kKTail: loads of steps up to KT - 2 only
-    step(IC<0>{}, kt, IC<0>{});
-    step(IC<1>{}, kt + 1, IC<0>{});
-    step(IC<2>{}, kt + 2, IC<0>{});
-  }
-  step(IC<0>{}, kt, IC<1>{});
-  step(IC<1>{}, kt + 1, IC<1>{});
-  step(IC<2>{}, kt + 2, IC<1>{});
-  step(IC<0>{}, kt + 3, IC<1>{});
-  if constexpr (kKTail) step(IC<1>{}, kt + 4, IC<1>{});
-  // the empty loads of the last two steps write LDS too: all landed before the epilogue reuses it
+  for (; kt + NST - 1 + D + (kKTail ? 1 : 0) < KT; kt += NST)  // kKTail: loads of steps up to KT - 2 only
+    for_stages<0, NST>([&](auto I) __attribute__((always_inline)) { step(I, kt + decltype(I)::value, IC<0>{}); });
+  for_stages<0, NST - 1 + D + (kKTail ? 1 : 0)>([&](auto I) __attribute__((always_inline)) {
+    constexpr int i = decltype(I)::value;
+    step(IC<i % NST>{}, kt + i, IC<1>{});
+  });
+  // the empty loads of the last steps write LDS too: all landed before the epilogue reuses it
   wait_vm_lgkm0<0>();
   __builtin_amdgcn_s_barrier();
 
@@ -573,13 +583,13 @@ gemm_dma_kernel(const GemmArgs p) {
   // the stages are free: the last step's barrier followed every wave's reads and every DMA
   constexpr int kScr = 16 * (NSB * 16 * 4 + 16);  // one wave's row-major tile, f32 worst case
   constexpr int kWps = kStage / kScr;
-  static_assert(3 * kWps >= NW, "epilogue scratch");
+  static_assert(3 * kWps >= NW && NOPS * (D - 1) < 64, "epilogue scratch, vmcnt");
   unsigned char* scr = (wave < kWps ? st0 : wave < 2 * kWps ? st1 : st2) + (wave % kWps) * kScr;
   store_tile_scaled(p, acc, e_rsc, e_valid, row0, lane,
                     [&](int j, bool& ok) __attribute__((always_inline)) { return gstrip(wn * NSB + j, ok); }, scr);
 }
 
-template <int WM, int WN, int RB, int NSB, int MODE, bool AT = false>
+template <int WM, int WN, int RB, int NSB, int NST, int MODE, bool AT = false>
 static int launch_dma_cfg_at(const GemmArgs& p, int64_t row_tiles, hipStream_t stream) {
   constexpr int BN = WN * NSB * 16;
   const int64_t ncols = p.silu ? p.N / 2 : p.N;
@@ -590,45 +600,54 @@ static int launch_dma_cfg_at(const GemmArgs& p, int64_t row_tiles, hipStream_t s
     while ((gx * gy) % 8) ++gy;
   const dim3 grid((unsigned)gx, (unsigned)gy);
   const dim3 block(WM * WN * 64);
-  auto kern = gemm_dma_kernel<WM, WN, RB, NSB, MODE, AT>;
+  auto kern = gemm_dma_kernel<WM, WN, RB, NSB, NST, MODE, AT>;
   hipLaunchKernelGGL(kern, grid, block, 0, stream, p);
   return hipGetLastError() == hipSuccess ? kOk : kErrHip;
 }
 
-// dense calls with p.a_tiled take the tiled-A instantiation (grouped ones: launch_dma_modes_grouped)
-template <int WM, int WN, int RB, int NSB, int MODE>
-static int launch_dma_cfg(const GemmArgs& p, int64_t row_tiles, hipStream_t stream) {
-  if (p.a_tiled) return launch_dma_cfg_at<WM, WN, RB, NSB, MODE, true>(p, row_tiles, stream);
-  return launch_dma_cfg_at<WM, WN, RB, NSB, MODE, false>(p, row_tiles, stream);
-}
-
-// the modes whose weights are decoded with their zero point: g128 with zero points, g64 and g32
-template <int WM, int WN, int RB, int NSB>
-static int launch_dma_lut(const GemmArgs& p, int mode, int64_t row_tiles, hipStream_t stream) {
+// int4 without row-major-only limits: p.a_tiled takes the tiled-A instantiation; the modes whose
+// weights are decoded with their zero point (g128 with zero points, g64 and g32) are row-major
+template <int WM, int WN, int RB, int NSB, int NST, bool AT>
+static int launch_dma_int4(const GemmArgs& p, int mode, int64_t row_tiles, hipStream_t stream) {
   switch (mode) {
-    case kPAsym: return launch_dma_cfg_at<WM, WN, RB, NSB, kPAsym>(p, row_tiles, stream);
-    case kPG64: return launch_dma_cfg_at<WM, WN, RB, NSB, kPG64>(p, row_tiles, stream);
-    case kPG64Z: return launch_dma_cfg_at<WM, WN, RB, NSB, kPG64Z>(p, row_tiles, stream);
-    case kPG32: return launch_dma_cfg_at<WM, WN, RB, NSB, kPG32>(p, row_tiles, stream);
-    default: return launch_dma_cfg_at<WM, WN, RB, NSB, kPG32Z>(p, row_tiles, stream);
+    case kPSym:
+      if constexpr (AT) {
+        if (p.a_tiled) return launch_dma_cfg_at<WM, WN, RB, NSB, NST, kPSym, true>(p, row_tiles, stream);
+      }
+      return launch_dma_cfg_at<WM, WN, RB, NSB, NST, kPSym>(p, row_tiles, stream);
+    case kPAsym: return launch_dma_cfg_at<WM, WN, RB, NSB, NST, kPAsym>(p, row_tiles, stream);
+    case kPG64: return launch_dma_cfg_at<WM, WN, RB, NSB, NST, kPG64>(p, row_tiles, stream);
+    case kPG64Z: return launch_dma_cfg_at<WM, WN, RB, NSB, NST, kPG64Z>(p, row_tiles, stream);
+    case kPG32: return launch_dma_cfg_at<WM, WN, RB, NSB, NST, kPG32>(p, row_tiles, stream);
+    default: return launch_dma_cfg_at<WM, WN, RB, NSB, NST, kPG32Z>(p, row_tiles, stream);
   }
 }
-
-template <int WM, int WN, int RB, int NSB>
-static int launch_dma_modes(const GemmArgs& p, int mode, int64_t row_tiles, hipStream_t stream) {
-  if (mode == kPSym) return launch_dma_cfg<WM, WN, RB, NSB, kPSym>(p, row_tiles, stream);
-  if (mode == kPE8M0) return launch_dma_cfg<WM, WN, RB, NSB, kPE8M0>(p, row_tiles, stream);
-  return launch_dma_lut<WM, WN, RB, NSB>(p, mode, row_tiles, stream);
+template <int WM, int WN, int RB, int NSB, int NST, bool AT>
+static int launch_dma_mx(const GemmArgs& p, int64_t row_tiles, hipStream_t stream) {
+  if constexpr (AT) {
+    if (p.a_tiled) return launch_dma_cfg_at<WM, WN, RB, NSB, NST, kPE8M0, true>(p, row_tiles, stream);
+  }
+  return launch_dma_cfg_at<WM, WN, RB, NSB, NST, kPE8M0>(p, row_tiles, stream);
 }
+
 // grouped tiles: A rows gathered through the sorted ids, or (p.a_tiled, symmetric int4, A rows at
 // their padded positions: gemm2) the padded rows' codes in operand order with their seeds
 template <int WM, int WN, int RB, int NSB>
-static int launch_dma_modes_grouped(const GemmArgs& p, int mode, int64_t row_tiles, hipStream_t stream) {
-  if (mode == kPSym && p.a_tiled) return launch_dma_cfg_at<WM, WN, RB, NSB, kPSym, true>(p, row_tiles, stream);
-  if (mode == kPSym) return launch_dma_cfg_at<WM, WN, RB, NSB, kPSym>(p, row_tiles, stream);
-  if (mode == kPE8M0) return launch_dma_cfg_at<WM, WN, RB, NSB, kPE8M0>(p, row_tiles, stream);
-  return launch_dma_lut<WM, WN, RB, NSB>(p, mode, row_tiles, stream);
+static int launch_dma_grouped(const GemmArgs& p, int mode, int64_t row_tiles, hipStream_t stream) {
+  if (mode == kPE8M0) return launch_dma_mx<WM, WN, RB, NSB, 3, false>(p, row_tiles, stream);
+  return launch_dma_int4<WM, WN, RB, NSB, 3, true>(p, mode, row_tiles, stream);
 }
+
+// Dense tile shapes (pick_tile) and what a K step of a full round of workgroups (one per CU) costs, relative to the
+// format's largest tile. A wave of the smaller ones has fewer MFMAs behind each LDS operand and
+// barrier, so their cost per output is higher; what they win is a grid that fills the 256 CUs. The two
+// smallest fit a CU twice and are measured at up to 256 workgroups (a round of the 64 x 128 one is
+// twice 256, at twice the cost). us per K step of a round, int4 symmetric: 1.26 / 1.02 / 0.78 / 0.54 /
+// 0.46; MXFP4: 1.41 / 1.13 / 0.85 / 0.70 / 0.63 / 0.46 / 0.40. Zero points and groups of 64 and 32 raise
+// all of a format's tiles alike (256 x 128: 1.29, 2.0 and 2.4).
+static const DmaTile kInt4Tiles[] = {{256, 128, 1.0f}, {192, 128, 0.81f}, {128, 128, 0.64f}, {64, 128, 0.45f}, {64, 64, 0.38f}};
+static const DmaTile kMxTiles[] = {{256, 256, 1.0f}, {192, 256, 0.80f}, {128, 256, 0.60f}, {192, 128, 0.50f},
+                                   {128, 128, 0.45f}, {64, 128, 0.33f}, {64, 64, 0.29f}};
 
 // int4 with groups of 32, 64 and 128+ and MXFP4, on 16-byte aligned rows; kErrUnsupported otherwise.
 // bm_rows: rows per workgroup the caller requires (grouped: 64 or 128; 0 for dense).
@@ -653,40 +672,39 @@ int launch_prefill_dma(const GemmArgs& p, int64_t rows_to_cover, int bm_rows, hi
   if ((int64_t)p.N * p.KT * 64 >= (int64_t)1 << 31) return kErrUnsupported;
   if (p.ldx % 16) return kErrUnsupported;  // A rows are read in 16-byte pieces, at 32-bit offsets
   if ((p.a_by_token ? p.num_slots / p.top_k : p.M) * p.ldx > (int64_t)0xffffffff) return kErrUnsupported;
-  // Tiles (waves WM x WN, wave tile RB x NSB blocks of 16): the largest whose three stages fit
-  // the 160 KiB of LDS and whose registers fit two waves per SIMD. MXFP4 keeps its weights as fp4
-  // in LDS and its accumulators are the only per-step state, so it takes 64 x 128 wave tiles
-  // (256 x 256 per workgroup: a quarter less LDS read per MFMA than 64 x 64); int4 holds the
-  // unpacked fp8 weights plus the partials of its per-group scaling and stays at 64 x 64.
   if (p.a_tiled && (p.sorted_ids ? (mode != kPSym || p.a_by_token != 0) : (bm_rows != 0 || (mode != kPSym && mode != kPE8M0))))
     return kErrUnsupported;
-  if (bm_rows == 64) return launch_dma_modes_grouped<2, 4, 2, 2>(p, mode, (rows_to_cover + 63) / 64, stream);
-  if (bm_rows == 128) return launch_dma_modes_grouped<2, 4, 4, 4>(p, mode, (rows_to_cover + 127) / 128, stream);
-  // Grids of at most half a workgroup per CU take smaller tiles. int4: 128 x 128 when that gives
-  // 192 or more workgroups, else 64 x 128 (the configs[2] M=512 calls, M=1024 on 4096-wide
-  // weights): K=4096 N=6144 M=512 39.5 -> 29.9 us, K=4096 N=4096 M=1024 42.4 -> 32.4 us, K=14336
-  // N=4096 M=1024 126.7 -> 94.2 us (128 x 128); K=4096 N=4096 M=512 50.7 -> 21.8 us, K=14336
-  // N=4096 M=512 146.9 -> 64.6 us (64 x 128; 128 x 128 gave 28.2 and 85.5 there). A grid of 144
-  // (K=4096 N=6144 M=768) measured slower with 128 x 128 tiles (55.5 against 48.2 us) and keeps
-  // 256 x 128. MXFP4 (256 x 256) takes 64 x 128 tiles. The tile shape does not change any
-  // output's arithmetic.
-  const int64_t ncols = p.silu ? p.N / 2 : p.N;
-  const int64_t bn_default = mode == kPE8M0 ? 256 : 128;
-  const int64_t g_default = (ncols + bn_default - 1) / bn_default * ((rows_to_cover + 255) / 256);
-  if (mode != kPE8M0 && g_default <= 128) {
-    if ((ncols + 127) / 128 * ((rows_to_cover + 127) / 128) >= 192)
-      return launch_dma_modes<4, 2, 2, 4>(p, mode, (rows_to_cover + 127) / 128, stream);
-    return launch_dma_modes<2, 4, 2, 2>(p, mode, (rows_to_cover + 63) / 64, stream);
+  if (bm_rows == 64) return launch_dma_grouped<2, 4, 2, 2>(p, mode, (rows_to_cover + 63) / 64, stream);
+  if (bm_rows == 128) return launch_dma_grouped<2, 4, 4, 4>(p, mode, (rows_to_cover + 127) / 128, stream);
+  // Dense tiles (waves WM x WN, wave tile RB x NSB blocks of 16). The largest are those whose three
+  // stages fit the 160 KiB of LDS and whose registers fit two waves per SIMD. MXFP4 keeps its weights
+  // as fp4 in LDS and its accumulators are the only per-step state, so it takes 64 x 128 wave tiles
+  // (256 x 256 per workgroup: a quarter less LDS read per MFMA than 64 x 64); int4 holds the unpacked
+  // fp8 weights plus the partials of its per-group scaling and stays at 64 x 64. The 64 x 64 tile takes
+  // four stages (two of its workgroups still fit a CU; AWQ M=100 K=4096 N=6144 22.9 -> 21.1 us, more
+  // stages gained nothing).
+  if (mode == kPE8M0) {
+    const int t = pick_tile(kMxTiles, p, rows_to_cover);
+    const int64_t rt = (rows_to_cover + kMxTiles[t].bm - 1) / kMxTiles[t].bm;
+    switch (t) {
+      case 0: return launch_dma_mx<4, 2, 4, 8, 3, true>(p, rt, stream);
+      case 1: return launch_dma_mx<4, 2, 3, 8, 3, true>(p, rt, stream);
+      case 2: return launch_dma_mx<4, 2, 2, 8, 3, true>(p, rt, stream);
+      case 3: return launch_dma_mx<4, 2, 3, 4, 3, true>(p, rt, stream);
+      case 4: return launch_dma_mx<4, 2, 2, 4, 3, true>(p, rt, stream);
+      case 5: return launch_dma_mx<2, 4, 2, 2, 3, true>(p, rt, stream);
+      default: return launch_dma_mx<2, 2, 2, 2, 4, true>(p, rt, stream);
+    }
   }
-  // a default grid of 257-384 workgroups runs one and a half rounds of the CUs; 128 x 128 tiles
-  // even it out (K=4096 N=6144 M=2048: 384 workgroups, 96.5 -> 91.6 us; a grid of 576 measured
-  // slower that way, 143.3 -> 146.7 us)
-  if (mode != kPE8M0 && g_default > 256 && g_default <= 384)
-    return launch_dma_modes<4, 2, 2, 4>(p, mode, (rows_to_cover + 127) / 128, stream);
-  if (mode == kPE8M0 && g_default <= 128)
-    return launch_dma_modes<2, 4, 2, 2>(p, mode, (rows_to_cover + 63) / 64, stream);
-  if (mode == kPE8M0) return launch_dma_cfg<4, 2, 4, 8, kPE8M0>(p, (rows_to_cover + 255) / 256, stream);
-  return launch_dma_modes<4, 2, 4, 4>(p, mode, (rows_to_cover + 255) / 256, stream);
+  const int t = pick_tile(kInt4Tiles, p, rows_to_cover);
+  const int64_t rt = (rows_to_cover + kInt4Tiles[t].bm - 1) / kInt4Tiles[t].bm;
+  switch (t) {
+    case 0: return launch_dma_int4<4, 2, 4, 4, 3, true>(p, mode, rt, stream);
+    case 1: return launch_dma_int4<4, 2, 3, 4, 3, true>(p, mode, rt, stream);
+    case 2: return launch_dma_int4<4, 2, 2, 4, 3, true>(p, mode, rt, stream);
+    case 3: return launch_dma_int4<2, 4, 2, 2, 3, true>(p, mode, rt, stream);
+    default: return launch_dma_int4<2, 2, 2, 2, 4, true>(p, mode, rt, stream);
+  }
 }
 
 // The LDS-staged kernels: NVFP4 on the fp16 MFMA, else the DMA-staged pipeline; kErrUnsupported for

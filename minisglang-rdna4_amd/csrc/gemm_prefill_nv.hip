@@ -356,10 +356,18 @@ int launch_prefill_nv(const GemmArgs& p, int64_t rows_to_cover, int bm_rows, hip
   // LDS: three A stages and two fp16 B stages; 256 x 128 uses all 160 KiB
   if (bm_rows == 64) return launch_nv_cfg<2, 4, 2, 2>(p, (rows_to_cover + 63) / 64, stream);
   if (bm_rows == 128) return launch_nv_cfg<4, 2, 2, 4>(p, (rows_to_cover + 127) / 128, stream);
-  const int64_t ncols = p.silu ? p.N / 2 : p.N;
-  if ((ncols + 127) / 128 * ((rows_to_cover + 255) / 256) <= 128)
-    return launch_nv_cfg<2, 4, 2, 2>(p, (rows_to_cover + 63) / 64, stream);
-  return launch_nv_cfg<4, 2, 4, 4>(p, (rows_to_cover + 255) / 256, stream);
+  // tile as in gemm_prefill_dma.hip (pick_tile); us per K step of a round of 256 workgroups 1.63 / 1.33 /
+  // 1.0 / 0.75 / 0.61
+  static const DmaTile tiles[] = {{256, 128, 1.0f}, {192, 128, 0.83f}, {128, 128, 0.62f}, {64, 128, 0.46f}, {64, 64, 0.37f}};
+  const int t = pick_tile(tiles, p, rows_to_cover);
+  const int64_t rt = (rows_to_cover + tiles[t].bm - 1) / tiles[t].bm;
+  switch (t) {
+    case 0: return launch_nv_cfg<4, 2, 4, 4>(p, rt, stream);
+    case 1: return launch_nv_cfg<4, 2, 3, 4>(p, rt, stream);
+    case 2: return launch_nv_cfg<4, 2, 2, 4>(p, rt, stream);
+    case 3: return launch_nv_cfg<2, 4, 2, 2>(p, rt, stream);
+    default: return launch_nv_cfg<2, 2, 2, 2>(p, rt, stream);
+  }
 }
 
 }  // namespace w4a8

@@ -348,6 +348,36 @@ __device__ __forceinline__ void store_tile(const GemmArgs& p, const v4f (&acc)[R
   store_tile_scaled(p, acc, sc, valid, row0, lane, strip, scr);
 }
 
+// A dense tile shape and what one K step of a full round of its workgroups (one per CU) costs, relative
+// to the others of its format.
+struct DmaTile {
+  int bm, bn;
+  float cost;
+};
+// The tile whose rounds of the grid take least. Up to six rounds a partial round counts as a whole one
+// (M=1777 K=2560 N=9728 int4: 532 workgroups of 256 x 128, 2.08 rounds, 81.5 us; 760 of 192 x 128, 2.97
+// rounds, 74.0); over more rounds the workgroups drift apart and half of the partial one is charged.
+// The tile does not change any output's arithmetic.
+template <int NT>
+inline int pick_tile(const DmaTile (&tiles)[NT], const GemmArgs& p, int64_t rows) {
+  int best = 0;
+  float least = 0.f;
+  for (int i = 0; i < NT; ++i) {
+    const DmaTile& t = tiles[i];
+    const int64_t colw = p.silu ? t.bn / 2 : t.bn;
+    const int64_t ncols = p.silu ? p.N / 2 : p.N;
+    const int64_t g = (ncols + colw - 1) / colw * ((rows + t.bm - 1) / t.bm);
+    if (t.bn == 64 && g > 256) continue;
+    const float r = (float)g / 256.0f, up = (float)((g + 255) / 256);
+    const float est = t.cost * (up <= 6.0f ? up : 0.5f * (r + up));
+    if (i == 0 || est < least) {
+      best = i;
+      least = est;
+    }
+  }
+  return best;
+}
+
 // Launch of the DMA-staged kernel (gemm_prefill_dma.hip); kErrUnsupported when it does not apply.
 int launch_prefill_dma(const GemmArgs& p, int64_t rows_to_cover, int bm_rows, hipStream_t stream);
 // NVFP4 on the fp16 MFMA (gemm_prefill_nv.hip); kErrUnsupported for other formats and shapes.

@@ -75,3 +75,26 @@ def test_moe_groups_and_k_tails(kernels, oracle, dev, fmt, g, h, i, bm):
                                e2m1=e2, nvfp4=nv)
     assert rel1 <= 2e-3 and rel2 <= 2e-3  # the bars of test_gpu_moe: bf16 rounding alone is 1.65e-3
     assert np.isfinite(res["out"].float().cpu().numpy()).all()
+
+
+# one row past 64, 128, 192 and 256 rows, and sizes that take each dense tile shape: 64 x 64 (few
+# workgroups), 64 x 128, 128 x 128, 192- and 256-row tiles, and MXFP4's 256-wide ones
+@pytest.mark.parametrize("fmt,g", [("sym", 128), ("asym", 32), ("mxfp4", 32), ("nvfp4", 16)])
+@pytest.mark.parametrize("M,N", [(65, 80), (129, 8208), (193, 12304), (321, 14352), (577, 16400), (1153, 8208)])
+def test_dense_tile_shapes(kernels, oracle, dev, fmt, g, M, N):
+    """Every tile shape gives a row the same bits: the call's rows against the same rows in calls of
+    seven, and those against the oracle."""
+    K = 384
+    w, s, z, e2, nv = _weight(fmt, g, N, K, seed=M + N)
+    x = synth.activations(M, K, seed=M + 1)
+    tiles, sd = kernels.repack_w4(w.to(dev), weight_is_e2m1=e2), s.to(dev)
+    zd = None if z is None else z.to(dev)
+    rows = torch.tensor(sorted({0, 15, 63, 64, M // 2, M - 2, M - 1}))
+    out, part = (kernels.w4a8_linear(t.to(dev), tiles, sd, zd, g, weight_is_e2m1=e2, kernel="wmma_tiled_tuned")
+                 for t in (x, x[rows].contiguous()))
+    torch.cuda.synchronize()
+    assert torch.equal(out[rows.to(dev)], part), f"{fmt} M={M} N={N}: a row's bits depend on the tile"
+    xq, xs = oracle.act_quant(synth.bits16(x[rows]), 0)
+    ref = oracle.gemm(xq, xs, w.numpy(), s.view(torch.uint8).numpy() if nv else s.numpy(),
+                      None if z is None else z.numpy(), g, e2, nv)
+    assert_close_to_oracle(part, ref, f"{fmt} M={M} N={N}")
