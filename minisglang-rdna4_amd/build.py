@@ -1,4 +1,5 @@
-"""Build libw4a8_mi355x.so (gfx950) from csrc/*.hip with hipcc, in-tree.
+"""Build libw4a8_mi355x.so (gfx950) from csrc/*.hip with hipcc and w4a8_host.so (the operators' host
+path, no device code) from csrc/host.cpp with the host compiler, in-tree.
 
 Objects compile in parallel into _build/, the shared library lands in _lib/. Every call
 recompiles (the build is the "does it build" check), so keep it cheap: one object per source.
@@ -45,6 +46,29 @@ def _compile(src: Path) -> Path:
     return obj
 
 
+def _build_host() -> Path:
+    """csrc/host.cpp against the installed torch's C++ libraries (loaded before it at run time)."""
+    import sysconfig
+
+    import torch
+
+    tdir = Path(torch.__file__).resolve().parent
+    out = LIBDIR / "w4a8_host.so"
+    tmp = out.with_suffix(".so.tmp")
+    rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-shared", "-fPIC", "-fvisibility=hidden",
+           "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}",
+           f"-I{tdir / 'include'}", f"-I{tdir / 'include' / 'torch' / 'csrc' / 'api' / 'include'}", f"-I{rocm}/include",
+           f"-I{sysconfig.get_paths()['include']}", str(CSRC / "host.cpp"), "-o", str(tmp), f"-L{tdir / 'lib'}",
+           "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_python"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"{cmd[0]} failed for host.cpp:\n{r.stderr[-4000:]}")
+    os.replace(tmp, out)
+    return out
+
+
 def lib_path() -> Path:
     return LIBDIR / LIBNAME
 
@@ -55,7 +79,9 @@ def build(verbose: bool = False) -> Path:
     srcs = sorted(CSRC.glob("*.hip"))
     jobs = min(len(srcs), max(1, min(8, os.cpu_count() or 1)))
     with cf.ThreadPoolExecutor(jobs) as ex:
+        host = ex.submit(_build_host)
         objs = list(ex.map(_compile, srcs))
+        host.result()
     out = lib_path()
     tmp = out.with_suffix(".so.tmp")
     cmd = [_hipcc(), f"--offload-arch={ARCH}", "-shared", "-fPIC", *map(str, objs), "-o", str(tmp)]

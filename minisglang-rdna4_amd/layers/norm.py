@@ -22,6 +22,7 @@ import torch
 
 _pkg = __name__.rsplit(".", 2)[0]
 _abi = importlib.import_module(f"{_pkg}._abi")
+_host = importlib.import_module(f"{_pkg}._host")
 engaged = importlib.import_module(f"{_pkg}._hip_engage").engaged
 
 _MAX_K = 32768
@@ -36,6 +37,10 @@ def _native_ok(*ts: torch.Tensor | None) -> bool:
 
 def _launch(x: torch.Tensor, weight: torch.Tensor | None, eps: float, plus_one: bool,
             residual: torch.Tensor | None, quant: bool, out: torch.Tensor | None = None):
+    if out is None:
+        r = _host.load().rms_norm(x, weight, eps, plus_one, residual, quant)
+        if r is not None:
+            return r
     K = x.shape[-1]
     x2 = x.reshape(-1, K)
     if x2.stride(-1) != 1:

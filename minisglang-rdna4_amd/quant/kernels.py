@@ -19,7 +19,7 @@ import os
 
 import torch
 
-from .. import _abi
+from .. import _abi, _host
 from .._hip_engage import engaged
 
 # AWQ "gemm" reverse pack order: undoes the [0,2,4,6,1,3,5,7] channel interleave of AWQ packing
@@ -210,6 +210,14 @@ _PREFILL_NAMES = ("wmma_tiled_tuned", "mfma_prefill")
 _IN_PROLOGUE_NAMES = ("prefill_wmma", "prefill_wmma_ashuffle")
 
 
+# the ledger's names of the calls that the host extension serves: by arm, e2m1 weights, producer pair
+_LINEAR_LEDGER = {
+    (arm, e2, pre): f"w4a8_mi355x.gemm({name}{'+e2m1' if e2 else ''}{'+prequant' if pre else ''})"
+    for arm, name in ((_abi.KERNEL_DECODE, "decode_gemv"), (_abi.KERNEL_PREFILL, "wmma_tiled_tuned"))
+    for e2 in (False, True) for pre in (False, True)
+}
+
+
 def _pick_dense_kernel(m: int, weight_is_e2m1: bool = False, group_size: int = 128,
                        k: int | None = None, n: int | None = None) -> str:
     """Per-M arm choice, same rule as python/minisgl/quant/kernels.py:1456-1632: the streaming
@@ -347,6 +355,12 @@ def w4a8_linear(
     kernels.py:1686-1734). Supplying the producer pair skips the op's own act-quant launch and is
     bit-identical to it. Names ``prefill_wmma``/``prefill_wmma_ashuffle`` are the reference's
     in-prologue-quant arms and refuse a pre-quantized pair loudly, as there."""
+    if x.is_cuda and (kernel is None or kernel == "decode_gemv"):
+        r = _host.load().linear(x, w_packed, scales, w_zeros, group_size, weight_is_e2m1, x_fp8, act_scales, False,
+                                _abi.KERNEL_AUTO if kernel is None else _abi.KERNEL_DECODE)
+        if r is not None:
+            engaged(_LINEAR_LEDGER[r[1], bool(weight_is_e2m1), x_fp8 is not None])
+            return r[0]
     N = _n_of(w_packed)
     K = x.shape[-1]
     if kernel is None:
@@ -379,6 +393,12 @@ def w4a8_linear_silu(
     round-silu-round-multiply replica of tools/w4a8_gemm_silu_parity.py:52-54."""
     if x.shape[0] > _W4A8_GEMV_MAX_INT4 or x.shape[1] % _W4A8_GEMV_K_MULTIPLE:
         raise AssertionError(f"w4a8_linear_silu: decode-only (M<=16, K%32==0), got {tuple(x.shape)}")
+    if x.is_cuda:
+        r = _host.load().linear(x, w_packed, scales, w_zeros, group_size, weight_is_e2m1, None, None, True,
+                                _abi.KERNEL_DECODE)
+        if r is not None:
+            engaged("w4a8_mi355x.gemm_silu(e2m1)" if weight_is_e2m1 else "w4a8_mi355x.gemm_silu(int4)")
+            return r[0]
     out, repacked = _dense(x, w_packed, scales, w_zeros, group_size, weight_is_e2m1, None, None, True,
                            _abi.KERNEL_DECODE)
     engaged(f"w4a8_mi355x.gemm_silu({'e2m1' if weight_is_e2m1 else 'int4'}{'+repack' if repacked else ''})")
@@ -727,12 +747,45 @@ def w4a8_moe(
     """Grouped W4A8 MoE forward (python/minisgl/quant/kernels.py:562-882): route -> align ->
     gemm1 with fused silu(gate)*up (output in x's dtype) -> per-row act-quant of that buffer ->
     gemm2 -> top-k weighted combine in f32 -> x's dtype. Returns (M, K)."""
+    if topk_ids is None and x_fp8 is None and act_scales is None and activation == "silu" and x.is_cuda and x.dim() == 2:
+        out = _moe_plain(x, w13, w13_scales, w13_zeros, w2, w2_scales, w2_zeros, gating_output, top_k, renormalize,
+                         block_m, weight_is_e2m1)
+        if out is not None:
+            return out
     return _moe_forward(x, w13, w13_scales, w13_zeros, w2, w2_scales, w2_zeros, gating_output, top_k, renormalize,
                         topk_weights=topk_weights, topk_ids=topk_ids, block_m=block_m, weight_is_e2m1=weight_is_e2m1,
                         activation=activation, x_fp8=x_fp8, act_scales=act_scales)["out"]
 
 
 _MOE_SLOTS_MAX = int(os.environ.get("W4A8_MOE_SLOTS_MAX", "8"))
+
+
+def _moe_plain(x, w13, w13_scales, w13_zeros, w2, w2_scales, w2_zeros, gating_output, top_k, renormalize, block_m,
+               weight_is_e2m1):
+    """_moe_forward's output through the host extension, with the same choices and ledger entries; None
+    where it does not take the call."""
+    M = x.shape[0]
+    if block_m is None:
+        block_m = _moe_block_m_auto(M, w13.shape[0], top_k)
+    slots = M <= _MOE_SLOTS_MAX and block_m < 64
+    r = _host.load().moe(x, w13, w13_scales, w13_zeros, w2, w2_scales, w2_zeros, gating_output, top_k, renormalize,
+                         weight_is_e2m1, block_m, slots, _MOE_ROUTED, _MOE_G2FUSE, M <= _MOE_G2C_MAX_TOKENS)
+    if r is None:
+        return None
+    out, took = r
+    arm = "gemv" if block_m < 64 else "mfma"
+    e2 = "+e2m1" if weight_is_e2m1 else ""
+    if took & 1:
+        engaged(f"w4a8_mi355x.moe_route_gemm1_silu(gemv{e2})")
+    else:
+        engaged("w4a8_mi355x.moe_route_slots" if slots else "w4a8_mi355x.moe_route_align")
+        engaged(f"w4a8_mi355x.moe_gemm1_silu({arm}{e2})")
+    if took & 2:
+        engaged(f"w4a8_mi355x.moe_gemm2_combine({arm}{e2})")
+    else:
+        engaged(f"w4a8_mi355x.moe_gemm2({arm}{e2})")
+        engaged("w4a8_mi355x.moe_combine")
+    return out
 
 
 def _moe_forward(x, w13, w13_scales, w13_zeros, w2, w2_scales, w2_zeros, gating_output, top_k, renormalize, *,
