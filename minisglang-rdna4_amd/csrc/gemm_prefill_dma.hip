@@ -646,6 +646,9 @@ static int launch_dma_grouped(const GemmArgs& p, int mode, int64_t row_tiles, hi
 // 0.46; MXFP4: 1.41 / 1.13 / 0.85 / 0.70 / 0.63 / 0.46 / 0.40. Zero points and groups of 64 and 32 raise
 // all of a format's tiles alike (256 x 128: 1.29, 2.0 and 2.4).
 static const DmaTile kInt4Tiles[] = {{256, 128, 1.0f}, {192, 128, 0.81f}, {128, 128, 0.64f}, {64, 128, 0.45f}, {64, 64, 0.38f}};
+// with the activations in operand order also gemm_prefill_wide.hip's tile (2.08 us)
+static const DmaTile kInt4TiledA[] = {{256, 128, 1.0f}, {192, 128, 0.81f}, {128, 128, 0.64f}, {64, 128, 0.45f},
+                                      {64, 64, 0.38f}, {256, 256, 1.65f}};
 static const DmaTile kMxTiles[] = {{256, 256, 1.0f}, {192, 256, 0.80f}, {128, 256, 0.60f}, {192, 128, 0.50f},
                                    {128, 128, 0.45f}, {64, 128, 0.33f}, {64, 64, 0.29f}};
 
@@ -696,14 +699,15 @@ int launch_prefill_dma(const GemmArgs& p, int64_t rows_to_cover, int bm_rows, hi
       default: return launch_dma_mx<2, 2, 2, 2, 4, true>(p, rt, stream);
     }
   }
-  const int t = pick_tile(kInt4Tiles, p, rows_to_cover);
-  const int64_t rt = (rows_to_cover + kInt4Tiles[t].bm - 1) / kInt4Tiles[t].bm;
+  const int t = p.a_tiled ? pick_tile(kInt4TiledA, p, rows_to_cover) : pick_tile(kInt4Tiles, p, rows_to_cover);
+  const int64_t rt = (rows_to_cover + kInt4TiledA[t].bm - 1) / kInt4TiledA[t].bm;
   switch (t) {
     case 0: return launch_dma_int4<4, 2, 4, 4, 3, true>(p, mode, rt, stream);
     case 1: return launch_dma_int4<4, 2, 3, 4, 3, true>(p, mode, rt, stream);
     case 2: return launch_dma_int4<4, 2, 2, 4, 3, true>(p, mode, rt, stream);
     case 3: return launch_dma_int4<2, 4, 2, 2, 3, true>(p, mode, rt, stream);
-    default: return launch_dma_int4<2, 2, 2, 2, 4, true>(p, mode, rt, stream);
+    case 4: return launch_dma_int4<2, 2, 2, 2, 4, true>(p, mode, rt, stream);
+    default: return launch_prefill_wide(p, rows_to_cover, stream);
   }
 }
 
