@@ -605,8 +605,7 @@ static int launch_dma_cfg_at(const GemmArgs& p, int64_t row_tiles, hipStream_t s
   return hipGetLastError() == hipSuccess ? kOk : kErrHip;
 }
 
-// int4 without row-major-only limits: p.a_tiled takes the tiled-A instantiation; the modes whose
-// weights are decoded with their zero point (g128 with zero points, g64 and g32) are row-major
+// int4; p.a_tiled takes the tiled-A instantiation (groups of 64 and 32 are row-major)
 template <int WM, int WN, int RB, int NSB, int NST, bool AT>
 static int launch_dma_int4(const GemmArgs& p, int mode, int64_t row_tiles, hipStream_t stream) {
   switch (mode) {
@@ -615,7 +614,11 @@ static int launch_dma_int4(const GemmArgs& p, int mode, int64_t row_tiles, hipSt
         if (p.a_tiled) return launch_dma_cfg_at<WM, WN, RB, NSB, NST, kPSym, true>(p, row_tiles, stream);
       }
       return launch_dma_cfg_at<WM, WN, RB, NSB, NST, kPSym>(p, row_tiles, stream);
-    case kPAsym: return launch_dma_cfg_at<WM, WN, RB, NSB, NST, kPAsym>(p, row_tiles, stream);
+    case kPAsym:
+      if constexpr (AT) {
+        if (p.a_tiled) return launch_dma_cfg_at<WM, WN, RB, NSB, NST, kPAsym, true>(p, row_tiles, stream);
+      }
+      return launch_dma_cfg_at<WM, WN, RB, NSB, NST, kPAsym>(p, row_tiles, stream);
     case kPG64: return launch_dma_cfg_at<WM, WN, RB, NSB, NST, kPG64>(p, row_tiles, stream);
     case kPG64Z: return launch_dma_cfg_at<WM, WN, RB, NSB, NST, kPG64Z>(p, row_tiles, stream);
     case kPG32: return launch_dma_cfg_at<WM, WN, RB, NSB, NST, kPG32>(p, row_tiles, stream);
@@ -630,7 +633,7 @@ static int launch_dma_mx(const GemmArgs& p, int64_t row_tiles, hipStream_t strea
   return launch_dma_cfg_at<WM, WN, RB, NSB, NST, kPE8M0>(p, row_tiles, stream);
 }
 
-// grouped tiles: A rows gathered through the sorted ids, or (p.a_tiled, symmetric int4, A rows at
+// grouped tiles: A rows gathered through the sorted ids, or (p.a_tiled, int4 in groups of 128+, A rows at
 // their padded positions: gemm2) the padded rows' codes in operand order with their seeds
 template <int WM, int WN, int RB, int NSB>
 static int launch_dma_grouped(const GemmArgs& p, int mode, int64_t row_tiles, hipStream_t stream) {
@@ -675,7 +678,8 @@ int launch_prefill_dma(const GemmArgs& p, int64_t rows_to_cover, int bm_rows, hi
   if ((int64_t)p.N * p.KT * 64 >= (int64_t)1 << 31) return kErrUnsupported;
   if (p.ldx % 16) return kErrUnsupported;  // A rows are read in 16-byte pieces, at 32-bit offsets
   if ((p.a_by_token ? p.num_slots / p.top_k : p.M) * p.ldx > (int64_t)0xffffffff) return kErrUnsupported;
-  if (p.a_tiled && (p.sorted_ids ? (mode != kPSym || p.a_by_token != 0) : (bm_rows != 0 || (mode != kPSym && mode != kPE8M0))))
+  if (p.a_tiled && (p.sorted_ids ? ((mode != kPSym && mode != kPAsym) || p.a_by_token != 0)
+                                 : (bm_rows != 0 || prefill_gpt(mode) > 1)))
     return kErrUnsupported;
   if (bm_rows == 64) return launch_dma_grouped<2, 4, 2, 2>(p, mode, (rows_to_cover + 63) / 64, stream);
   if (bm_rows == 128) return launch_dma_grouped<2, 4, 4, 4>(p, mode, (rows_to_cover + 127) / 128, stream);

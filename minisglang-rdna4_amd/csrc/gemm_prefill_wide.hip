@@ -1,5 +1,5 @@
-// The dense symmetric int4 prefill GEMM on 256 x 256 tiles, for activations in operand order
-// (GemmArgs::a_tiled) with their row-sum seeds; the math and the bits of gemm_prefill_dma.hip's tiles.
+// The dense int4 prefill GEMM (groups of 128+) on 256 x 256 tiles, for activations in operand order
+// (GemmArgs::a_tiled), symmetric with their row-sum seeds or with zero points; the math and the bits of gemm_prefill_dma.hip's tiles.
 //
 // What bounds the 256 x 128 tile there is not its MFMAs but what goes with each: 1 KiB of LDS operands
 // per MFMA, and a barrier every 16 of them. A 256 x 256 tile halves the barriers and takes a quarter
@@ -14,6 +14,8 @@
 //     256 x 128 step; the 4-bit weights are loaded to registers two steps ahead and unpacked one ahead.
 // Whole calls, 256 x 128 -> 256 x 256, us: K=4096 N=28672 M=8192 1134 -> 955 (2.0 PFLOP/s), N=6144 M=8192
 // 259 -> 220, N=4096 M=8192 181 -> 153, K=14336 N=4096 M=4096 308 -> 267, K=1024 N=4096 M=4096 37.0 -> 32.1.
+// With zero points (row-major 256 x 128 tiles before, two FMAs per output and step): N=28672 M=8192
+// 1372 -> 953, N=14336 M=3000 292 -> 192.
 // The unpack placed one row block earlier or later, the DMAs ahead of the step's LDS reads, and a raised
 // wave priority around the MFMAs all measured within 1%.
 #include "prefill.h"
@@ -28,14 +30,17 @@ __device__ __forceinline__ void wide_steps(F f) {
   }
 }
 
-template <int WM, int WN, int RB, int NSB>
+template <int WM, int WN, int RB, int NSB, int MODE>
 __global__ void __launch_bounds__(WM * WN * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
 gemm_wide_kernel(const GemmArgs p) {
   constexpr int T = WM * WN * 64, NW = WM * WN;
   constexpr int BM = WM * RB * 16, BN = WN * NSB * 16, NSTRIP = BN / 16;
   constexpr int kA = BM * 128, kB = BN * 128, kS = BN * 2;
-  constexpr int kScaleOff = kA, kSeedOff = kScaleOff + kS, kDma = kSeedOff + BM * 4;
+  constexpr int kScaleOff = kA, kSeedOff = kScaleOff + kS, kDma = kSeedOff + (kZ ? 0 : BM * 4);
+  static_assert(MODE == kPSym || MODE == kPAsym, "int4, groups of 128 or more");
+  constexpr bool kZ = MODE == kPAsym;  // weights decoded as e4m3(q - z), no seeds
   constexpr int A_PER = BM / 8 / NW, B_PER = NSTRIP * 64 / T;
+  constexpr int W_PER = B_PER * (kZ ? 2 : 1);  // loads of a step's weights (and zero words) per thread
   static_assert(A_PER * NW == BM / 8 && B_PER * T == NSTRIP * 64, "blocks / waves");
   constexpr int kScaleW = BN / 128, kSeedW = BM / 64;  // waves whose dword DMAs cover the scales, the seeds
   static_assert(NW % kScaleW == 0 && NW % kSeedW == 0, "every wave issues one DMA of each");
@@ -81,7 +86,8 @@ gemm_wide_kernel(const GemmArgs p) {
 
   const uint32_t w_bytes = (uint32_t)((size_t)nstrips * KT * kTileBytes);
   const uint32_t s_bytes = (uint32_t)((size_t)(KT >> gshift) * N * 2);
-  const uint32_t seed_bytes = (uint32_t)((size_t)KT * p.seeds_ld * 4);
+  const uint32_t seed_bytes = kZ ? 0u : (uint32_t)((size_t)KT * p.seeds_ld * 4);
+  const uint32_t z_bytes = kZ ? (uint32_t)((size_t)(KT >> gshift) * (N / 8) * 4) : 0u;
 
   // per-lane source offsets (rows past M read the last 16-row block / seed; their outputs are not stored)
   uint32_t a_voff[A_PER];
@@ -99,12 +105,15 @@ gemm_wide_kernel(const GemmArgs p) {
   bool ok_;
   const int sd = 64 * (wave % kScaleW) + lane;  // dword of the tile's scale row: two channels of strip sd / 8
   const uint32_t s_voff = (uint32_t)((gstrip(sd >> 3, ok_) * 16 + (sd & 7) * 2) * 2);
-  uint32_t b_voff[B_PER];
+  uint32_t b_voff[B_PER], z_voff[B_PER];
 #pragma unroll
   for (int i = 0; i < B_PER; ++i) {
-    const int c = (int)threadIdx.x + i * T;
-    b_voff[i] = (uint32_t)(((size_t)gstrip(c >> 6, ok_) * KT * 64 + (c & 63)) * 16);
+    const int c = (int)threadIdx.x + i * T, gs = gstrip(c >> 6, ok_);
+    b_voff[i] = (uint32_t)(((size_t)gs * KT * 64 + (c & 63)) * 16);
+    z_voff[i] = (uint32_t)((gs * 2 + ((c >> 3) & 1)) * 4);
   }
+  __shared__ uint4 zlut[kZ ? 16 : 1];
+  if (kZ && threadIdx.x < 16) zlut[threadIdx.x] = zero_point_lut((int)threadIdx.x);
 
   __shared__ float e_sc[BM];
   const int er = (int)threadIdx.x;
@@ -112,6 +121,7 @@ gemm_wide_kernel(const GemmArgs p) {
   if (er < BM && blk_row0 + er < p.M) er_sc = p.act_scales[blk_row0 + er];
 
   v4u rbw[2][B_PER];
+  uint32_t rzp[2][B_PER];
   // Tail: loads past the last step read empty buffers, as in gemm_dma_kernel
   auto live_of = [&](int kt, auto Tail) __attribute__((always_inline)) {
     return decltype(Tail)::value ? (uint32_t)__builtin_amdgcn_readfirstlane(kt < KT ? -1 : 0) : 0xffffffffu;
@@ -127,22 +137,36 @@ gemm_wide_kernel(const GemmArgs p) {
     for (int i = 0; i < A_PER; ++i) lds_dma16(rs_a, st + (wave + i * NW) * 1024, a_voff[i], so);
     lds_dma4(rs_s, st + kScaleOff + (wave % kScaleW) * 256, s_voff,
              (uint32_t)__builtin_amdgcn_readfirstlane((kt >> gshift) * N * 2));
-    lds_dma4(rs_seed, st + kSeedOff + (wave % kSeedW) * 256, seed_voff,
-             (uint32_t)__builtin_amdgcn_readfirstlane(kt * (int)p.seeds_ld * 4));
+    if constexpr (!kZ)
+      lds_dma4(rs_seed, st + kSeedOff + (wave % kSeedW) * 256, seed_voff,
+               (uint32_t)__builtin_amdgcn_readfirstlane(kt * (int)p.seeds_ld * 4));
   };
   auto issue_w = [&](auto R_, int kt, auto Tail) __attribute__((always_inline)) {
     constexpr int R = decltype(R_)::value;
-    const BufRsrc rs_w = make_rsrc(p.wt, w_bytes & live_of(kt, Tail));
+    const uint32_t live = live_of(kt, Tail);
+    const BufRsrc rs_w = make_rsrc(p.wt, w_bytes & live), rs_z = make_rsrc(p.zeros, z_bytes & live);
     if constexpr (decltype(Tail)::value) kt = kt < KT ? kt : KT - 1;
     const uint32_t so = (uint32_t)__builtin_amdgcn_readfirstlane(kt * kTileBytes);
 #pragma unroll
     for (int i = 0; i < B_PER; ++i) rbw[R][i] = bload128v(rs_w, b_voff[i], so);
+    if constexpr (kZ) {
+      const uint32_t so_z = (uint32_t)__builtin_amdgcn_readfirstlane((kt >> gshift) * (N / 8) * 4);
+#pragma unroll
+      for (int i = 0; i < B_PER; ++i) rzp[R][i] = bload32(rs_z, z_voff[i], so_z);
+    }
   };
   auto commit = [&](auto I, int i) __attribute__((always_inline)) {  // chunk i of the stage's weights
     constexpr int R = decltype(I)::value;
     unsigned char* sb = bstage(I);
     const int c = (int)threadIdx.x + i * T, s = c >> 6, l = c & 63;
-    const v8i u = unpack_tile_int4(make_uint4(rbw[R][i].x, rbw[R][i].y, rbw[R][i].z, rbw[R][i].w));
+    const uint4 w = make_uint4(rbw[R][i].x, rbw[R][i].y, rbw[R][i].z, rbw[R][i].w);
+    v8i u;
+    if constexpr (kZ) {
+      const uint4 t = zlut[(rzp[R][i] >> (4 * (lane & 7))) & 15u];
+      u = unpack_tile_lut(w, t, t);
+    } else {
+      u = unpack_tile_int4(w);
+    }
     *reinterpret_cast<uint4*>(sb + ((s * 2 + 0) * 64 + l) * 16) = make_uint4(u[0], u[1], u[2], u[3]);
     *reinterpret_cast<uint4*>(sb + ((s * 2 + 1) * 64 + l) * 16) = make_uint4(u[4], u[5], u[6], u[7]);
   };
@@ -169,7 +193,7 @@ gemm_wide_kernel(const GemmArgs p) {
     v8i b[NSB];
     float sc[NSB];
     v8i a0 = lds_operand(st + oa, 0);
-    v4f e0 = *reinterpret_cast<const v4f*>(st + oe);
+    v4f e0 = kZ ? v4f{0.f, 0.f, 0.f, 0.f} : *reinterpret_cast<const v4f*>(st + oe);
 #pragma unroll
     for (int j = 0; j < NSB; ++j) b[j] = lds_operand(sb + ob + j * 2048, 0);
 #pragma unroll
@@ -181,7 +205,7 @@ gemm_wide_kernel(const GemmArgs p) {
       v4f e1;
       if (rb + 1 < RB) {
         a1 = lds_operand(st + oa + (rb + 1) * 2048, 0);
-        e1 = *reinterpret_cast<const v4f*>(st + oe + (rb + 1) * 64);
+        e1 = kZ ? v4f{0.f, 0.f, 0.f, 0.f} : *reinterpret_cast<const v4f*>(st + oe + (rb + 1) * 64);
       }
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -213,7 +237,7 @@ gemm_wide_kernel(const GemmArgs p) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) acc[RB - 1][j][r] += sc[j] * cj[j][r];
     __builtin_amdgcn_sched_barrier(0);
-    wait_vm_lgkm0<B_PER>();
+    wait_vm_lgkm0<W_PER>();
     __builtin_amdgcn_s_barrier();
   };
   static_assert(B_PER <= 2, "weight chunks per thread");
@@ -223,9 +247,10 @@ gemm_wide_kernel(const GemmArgs p) {
   __builtin_amdgcn_sched_barrier(0);
   issue_w(IC<1>{}, 1, IC<1>{});
   __builtin_amdgcn_sched_barrier(0);
+  if constexpr (kZ) lds_barrier();  // the zero-point table, before the first decode reads it
 #pragma unroll
   for (int i = 0; i < B_PER; ++i) commit(IC<0>{}, i);
-  wait_vm_lgkm0<B_PER>();
+  wait_vm_lgkm0<W_PER>();
   if (er < BM) e_sc[er] = er_sc;  // read after the K loop's barriers
   __builtin_amdgcn_s_barrier();
   int kt = 0;
@@ -262,7 +287,10 @@ gemm_wide_kernel(const GemmArgs p) {
 int launch_prefill_wide(const GemmArgs& p, int64_t rows, hipStream_t stream) {
   const int64_t ncols = p.silu ? p.N / 2 : p.N, colw = p.silu ? 128 : 256;
   const dim3 grid((unsigned)((ncols + colw - 1) / colw), (unsigned)((rows + 255) / 256));
-  hipLaunchKernelGGL((gemm_wide_kernel<2, 4, 8, 4>), grid, dim3(512), 0, stream, p);
+  if (p.zeros)
+    hipLaunchKernelGGL((gemm_wide_kernel<2, 4, 8, 4, kPAsym>), grid, dim3(512), 0, stream, p);
+  else
+    hipLaunchKernelGGL((gemm_wide_kernel<2, 4, 8, 4, kPSym>), grid, dim3(512), 0, stream, p);
   return hipGetLastError() == hipSuccess ? kOk : kErrHip;
 }
 

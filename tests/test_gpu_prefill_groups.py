@@ -6,6 +6,7 @@ import pytest
 import torch
 
 import synth
+from conftest import pkg
 from test_gpu_dense import assert_close_to_oracle
 from test_gpu_moe import _stagewise
 
@@ -102,25 +103,28 @@ def test_dense_tile_shapes(kernels, oracle, dev, fmt, g, M, N):
 
 @pytest.mark.parametrize("M,N,K,silu", [(4096, 4096, 384, False), (4090, 4080, 512, False), (4093, 4096, 640, True),
                                         (7900, 2048, 1152, True), (3841, 4096, 4224, False)])
-def test_wide_tile_matches_the_others(kernels, dev, M, N, K, silu):
+@pytest.mark.parametrize("asym,g", [(False, 128), (True, 128), (True, 256)])
+def test_wide_tile_matches_the_others(kernels, dev, M, N, K, silu, asym, g):
     """256 x 256 tiles (activations in operand order, grids that one round of them fills): 3 to 33 K
     tiles, ragged rows and strips and the silu arm, bit for bit against the row-major kernel (w4a8_gemm
     without a workspace) on the same codes."""
-    abi = __import__("conftest").pkg("_abi")
+    if K % g:
+        pytest.skip("group does not divide K")
+    abi = pkg("_abi")
     lib = abi.load()
-    w, s, _ = synth.int4_weight(N, K, 128, seed=N + K, asym=False, scale_floor=1e-4)
-    tiles, sd = kernels.repack_w4(w.to(dev)), s.to(dev)
+    w, s, z = synth.int4_weight(N, K, g, seed=N + K, asym=asym, scale_floor=1e-4)
+    tiles, sd, zd = kernels.repack_w4(w.to(dev)), s.to(dev), None if z is None else z.to(dev)
     x = synth.activations(M, K, seed=M).to(dev)
     q, sc = kernels.act_quant(x)
     nout = N // 2 if silu else N
     out, ref = (torch.empty((M, nout), dtype=x.dtype, device=dev) for _ in range(2))
     wsb = lib.w4a8_linear_workspace_bytes(M, K)
     ws = torch.empty(wsb, dtype=torch.uint8, device=dev)
-    abi.check(lib.w4a8_linear(abi.ptr(x), abi.BF16, M, K, K, abi.ptr(tiles), N, abi.ptr(sd), abi.SCALE_F16, None,
-                              abi.W_INT4, 128, abi.ptr(out), abi.BF16, nout, int(silu), abi.ptr(ws), wsb,
+    abi.check(lib.w4a8_linear(abi.ptr(x), abi.BF16, M, K, K, abi.ptr(tiles), N, abi.ptr(sd), abi.SCALE_F16,
+                              abi.ptr(zd), abi.W_INT4, g, abi.ptr(out), abi.BF16, nout, int(silu), abi.ptr(ws), wsb,
                               abi.KERNEL_PREFILL, abi.stream_of(x)), "w4a8_linear")
-    abi.check(lib.w4a8_gemm(abi.ptr(q), K, abi.ptr(sc), M, abi.ptr(tiles), N, K, abi.ptr(sd), abi.SCALE_F16, None,
-                            abi.W_INT4, 128, abi.ptr(ref), abi.BF16, nout, int(silu), None, 0, abi.KERNEL_PREFILL,
+    abi.check(lib.w4a8_gemm(abi.ptr(q), K, abi.ptr(sc), M, abi.ptr(tiles), N, K, abi.ptr(sd), abi.SCALE_F16,
+                            abi.ptr(zd), abi.W_INT4, g, abi.ptr(ref), abi.BF16, nout, int(silu), None, 0, abi.KERNEL_PREFILL,
                             abi.stream_of(x)), "w4a8_gemm")
     torch.cuda.synchronize()
     assert torch.equal(out, ref), f"max {(out.float() - ref.float()).abs().max().item():.3e}"
