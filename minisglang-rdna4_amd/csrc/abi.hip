@@ -84,7 +84,7 @@ static bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 
 
 static const int kGemvMaxRows = 16;
 
-// Dense symmetric int4 prefill calls of at least W4A8_PREFILL_TILED rows (default 1024; 0 turns it
+// Dense int4 (groups of 128+) and MXFP4 prefill calls of at least W4A8_PREFILL_TILED rows (default 1024; 0 turns it
 // off) that the DMA-staged kernel takes (its own checks, launch_prefill_dma) have their codes in
 // that kernel's operand order with the row-sum seeds, which it then reads instead of computing them.
 // w4a8_linear quantizes x straight into that order (act_quant_tiled_lds_kernel, one launch as the
@@ -109,9 +109,9 @@ static int64_t tiled_min_n() {
 }
 static bool dma_tiled_ok(const GemmArgs& p, int64_t min_n = 16384) {
   const int64_t min_rows = tiled_min_rows();
-  const bool sym4 = p.wfmt == kInt4 && p.sfmt == kScaleF16 && p.group % 128 == 0 && !p.zeros;
+  const bool int4 = p.wfmt == kInt4 && p.sfmt == kScaleF16 && p.group % 128 == 0;  // with zeros: the seeds go unused
   const bool mx = p.wfmt == kE2M1 && p.sfmt == kScaleE8M0 && p.group == 32;  // MXFP4: A layout only, no seeds
-  return min_rows > 0 && p.M >= min_rows && p.N >= min_n && (sym4 || mx) && p.K % 128 == 0 && p.KT >= 3 && !(p.silu && (p.N / 16) % 2) &&
+  return min_rows > 0 && p.M >= min_rows && p.N >= min_n && (int4 || mx) && p.K % 128 == 0 && p.KT >= 3 && !(p.silu && (p.N / 16) % 2) &&
          p.N * p.KT * 64 < ((int64_t)1 << 31) && p.M * p.K < ((int64_t)1 << 31);
 }
 
@@ -681,8 +681,8 @@ int w4a8_moe_gemm_quant(const void* a, int a_dtype, int64_t lda, const int32_t* 
   // rows that can hold data (the grid bound; *ntp bounds the work on the device)
   const int64_t nblk = moe_max_blocks(numel, E, block_m, P);
   const int64_t rows = nblk * block_m < P ? nblk * block_m : P;
-  const bool sym4 = wfmt == kInt4 && scale_fmt == kScaleF16 && group_size % 128 == 0 && !zeros;
-  if (!decode && sym4 && tiled_min_rows() > 0 && K % 128 == 0 && p.KT >= 3 && N * p.KT * 64 < ((int64_t)1 << 31)) {
+  const bool int4 = wfmt == kInt4 && scale_fmt == kScaleF16 && group_size % 128 == 0;
+  if (!decode && int4 && tiled_min_rows() > 0 && K % 128 == 0 && p.KT >= 3 && N * p.KT * 64 < ((int64_t)1 << 31)) {
     // the padded rows quantized straight into the DMA GEMM's operand order with the row-sum seeds
     const int64_t Pp = (P + 15) / 16 * 16;
     float* seeds = reinterpret_cast<float*>(codes + round256(Pp * K));
