@@ -15,7 +15,7 @@
 // Whole calls, 256 x 128 -> 256 x 256, us: K=4096 N=28672 M=8192 1134 -> 955 (2.0 PFLOP/s), N=6144 M=8192
 // 259 -> 220, N=4096 M=8192 181 -> 153, K=14336 N=4096 M=4096 308 -> 267, K=1024 N=4096 M=4096 37.0 -> 32.1.
 // With zero points (row-major 256 x 128 tiles before, two FMAs per output and step): N=28672 M=8192
-// 1372 -> 953, N=14336 M=3000 292 -> 192.
+// 1325 -> 970, N=14336 M=3000 279 -> 204.
 // The unpack placed one row block earlier or later, the DMAs ahead of the step's LDS reads, and a raised
 // wave priority around the MFMAs all measured within 1%.
 #include "prefill.h"
@@ -33,12 +33,12 @@ __device__ __forceinline__ void wide_steps(F f) {
 template <int WM, int WN, int RB, int NSB, int MODE>
 __global__ void __launch_bounds__(WM * WN * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
 gemm_wide_kernel(const GemmArgs p) {
+  static_assert(MODE == kPSym || MODE == kPAsym, "int4, groups of 128 or more");
+  constexpr bool kZ = MODE == kPAsym;  // weights decoded as e4m3(q - z), no seeds
   constexpr int T = WM * WN * 64, NW = WM * WN;
   constexpr int BM = WM * RB * 16, BN = WN * NSB * 16, NSTRIP = BN / 16;
   constexpr int kA = BM * 128, kB = BN * 128, kS = BN * 2;
   constexpr int kScaleOff = kA, kSeedOff = kScaleOff + kS, kDma = kSeedOff + (kZ ? 0 : BM * 4);
-  static_assert(MODE == kPSym || MODE == kPAsym, "int4, groups of 128 or more");
-  constexpr bool kZ = MODE == kPAsym;  // weights decoded as e4m3(q - z), no seeds
   constexpr int A_PER = BM / 8 / NW, B_PER = NSTRIP * 64 / T;
   constexpr int W_PER = B_PER * (kZ ? 2 : 1);  // loads of a step's weights (and zero words) per thread
   static_assert(A_PER * NW == BM / 8 && B_PER * T == NSTRIP * 64, "blocks / waves");
