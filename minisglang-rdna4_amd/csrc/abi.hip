@@ -109,7 +109,7 @@ static int64_t tiled_min_n() {
 }
 static bool dma_tiled_ok(const GemmArgs& p, int64_t min_n = 16384) {
   const int64_t min_rows = tiled_min_rows();
-  const bool int4 = p.wfmt == kInt4 && p.sfmt == kScaleF16 && p.group % 128 == 0;  // with zeros: the seeds go unused
+  const bool int4 = p.wfmt == kInt4 && p.sfmt == kScaleF16 && p.group % 128 == 0;  // with zeros: no seeds
   const bool mx = p.wfmt == kE2M1 && p.sfmt == kScaleE8M0 && p.group == 32;  // MXFP4: A layout only, no seeds
   return min_rows > 0 && p.M >= min_rows && p.N >= min_n && (int4 || mx) && p.K % 128 == 0 && p.KT >= 3 && !(p.silu && (p.N / 16) % 2) &&
          p.N * p.KT * 64 < ((int64_t)1 << 31) && p.M * p.K < ((int64_t)1 << 31);
@@ -328,7 +328,7 @@ int w4a8_linear(const void* x, int x_dtype, int64_t M, int64_t K, int64_t ldx, c
     const int64_t Mp = (M + 15) / 16 * 16;
     uint8_t* xt = reinterpret_cast<uint8_t*>(xs) + round256(M * 4);
     float* seeds = reinterpret_cast<float*>(xt + round256(Mp * K));
-    rc = launch_act_quant_tiled(x, x_dtype, M, K, ldx, xt, xs, seeds, Mp, nullptr, st);
+    rc = launch_act_quant_tiled(x, x_dtype, M, K, ldx, xt, xs, wfmt == kInt4 && !zeros ? seeds : nullptr, Mp, nullptr, st);
     if (rc) return hip_status(rc, "w4a8_linear(act quant, tiled)");
     GemmArgs q = p;
     q.xsrc = nullptr;
@@ -686,7 +686,7 @@ int w4a8_moe_gemm_quant(const void* a, int a_dtype, int64_t lda, const int32_t* 
     // the padded rows quantized straight into the DMA GEMM's operand order with the row-sum seeds
     const int64_t Pp = (P + 15) / 16 * 16;
     float* seeds = reinterpret_cast<float*>(codes + round256(Pp * K));
-    rc = launch_act_quant_tiled(a, a_dtype, rows, K, lda, codes, xs, seeds, Pp, ntp, st);
+    rc = launch_act_quant_tiled(a, a_dtype, rows, K, lda, codes, xs, zeros ? nullptr : seeds, Pp, ntp, st);
     if (rc) return hip_status(rc, "w4a8_moe_gemm_quant(act quant, tiled)");
     GemmArgs q = p;
     q.a_tiled = 1; q.seeds = seeds; q.seeds_ld = Pp;
@@ -696,12 +696,11 @@ int w4a8_moe_gemm_quant(const void* a, int a_dtype, int64_t lda, const int32_t* 
   const int64_t Pp = (P + 15) / 16 * 16;
   if (decode && tiled_min_rows() > 0 && numel >= 16 * E && K % 128 == 0 && Pp * K < ((int64_t)1 << 31)) {
     // the grouped GEMV reads each 16-row block's codes in operand order: per tile two 1 KiB runs
-    // instead of 16 rows' 64-byte pieces (any weight format; the seeds go unused). Only where the
+    // instead of 16 rows' 64-byte pieces (any weight format; no seeds). Only where the
     // blocks are about full (16+ slots per expert): a block's rows without data read row 0's
     // pieces in the row-major form, one cache line, but whole runs in this one (configs[4] gemm2
     // T=512 177.5 -> 170.6 us whole call, T=256 120.1 -> 119.2; T=32 gemm2 23.6 -> 27.4 us)
-    float* seeds = reinterpret_cast<float*>(codes + round256(Pp * K));
-    rc = launch_act_quant_tiled(a, a_dtype, rows, K, lda, codes, xs, seeds, Pp, ntp, st);
+    rc = launch_act_quant_tiled(a, a_dtype, rows, K, lda, codes, xs, nullptr, Pp, ntp, st);
     if (rc) return hip_status(rc, "w4a8_moe_gemm_quant(act quant, tiled)");
     GemmArgs q = p;
     q.a_tiled = 1;

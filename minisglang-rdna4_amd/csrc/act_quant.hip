@@ -165,6 +165,7 @@ act_quant_tiled_kernel(const uint16_t* __restrict__ x, int64_t ldx, int64_t M, i
         half[h] = make_uint4(c0.x, c0.y, c1.x, c1.y);
         *reinterpret_cast<uint4*>(qt + ((blk * KT + kt) * 2 + h) * 1024 + lane * 16) = half[h];
       }
+      if (!seeds) continue;
       v8i a;
       a[0] = (int)half[0].x; a[1] = (int)half[0].y; a[2] = (int)half[0].z; a[3] = (int)half[0].w;
       a[4] = (int)half[1].x; a[5] = (int)half[1].y; a[6] = (int)half[1].z; a[7] = (int)half[1].w;
@@ -237,6 +238,7 @@ act_quant_tiled_lds_kernel(const uint16_t* __restrict__ x, int64_t ldx, int64_t 
       uint8_t* dst = qt + (blk * KT + kt) * 2048 + lane * 16;
       *reinterpret_cast<uint4*>(dst) = h0;
       *reinterpret_cast<uint4*>(dst + 1024) = h1;
+      if (!seeds) continue;
       v8i a;
       a[0] = (int)h0.x; a[1] = (int)h0.y; a[2] = (int)h0.z; a[3] = (int)h0.w;
       a[4] = (int)h1.x; a[5] = (int)h1.y; a[6] = (int)h1.z; a[7] = (int)h1.w;
@@ -311,6 +313,7 @@ act_quant_tiled_short_kernel(const uint16_t* __restrict__ x, int64_t ldx, int64_
       uint8_t* dst = qt + (blk * KT + kt) * 2048 + lane * 16;
       *reinterpret_cast<uint4*>(dst) = h0;
       *reinterpret_cast<uint4*>(dst + 1024) = h1;
+      if (!seeds) continue;
       v8i a;
       a[0] = (int)h0.x; a[1] = (int)h0.y; a[2] = (int)h0.z; a[3] = (int)h0.w;
       a[4] = (int)h1.x; a[5] = (int)h1.y; a[6] = (int)h1.z; a[7] = (int)h1.w;
@@ -321,6 +324,75 @@ act_quant_tiled_short_kernel(const uint16_t* __restrict__ x, int64_t ldx, int64_
             make_float4(pre[0], pre[1], pre[2], pre[3]);
     }
     __syncthreads();  // the codes of the next block overwrite cb
+  }
+}
+
+// The same for rows of 4097 to 16384 elements, with x read once: a workgroup of 16 waves holds 4 rows in
+// registers (thread t: the 8-element chunks t + 1024 i of each), takes their maxima through one barrier,
+// and writes each chunk's 8 codes straight to their operand-order place. Four rows are the fewest whose
+// pieces fill a 64-byte segment of the output (4 rows x 16 bytes), which L2 then writes whole. The
+// two-pass kernel has a quarter as many workgroups and reads x twice: whole MXFP4 calls at K=8192 N=8192
+// M=1024 66.5 -> 59.3 us, K=14336 N=4096 M=2000 109 -> 106. Longer rows (four chunks per thread) spill:
+// K=28672 M=4096 106 -> 170 us, so they keep the two passes, as do the calls that need seeds (the tiles
+// pass through its registers, where reading the codes back would cost what the second read of x does).
+template <int CPT>
+__global__ void __launch_bounds__(1024)
+act_quant_tiled_rows_kernel(const uint16_t* __restrict__ x, int64_t ldx, int64_t M, int64_t K, int dtype,
+                            uint8_t* __restrict__ qt, float* __restrict__ scales, const int32_t* __restrict__ row_count) {
+  __shared__ float red[4][16];
+  int64_t rows = M;  // as act_quant_tiled_kernel
+  if (row_count) {
+    const int64_t rc = *row_count;
+    rows = rc < M ? rc : M;
+  }
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int KT = (int)(K / kTileK), nch = (int)(K / 8);
+  const int64_t units = (rows + 15) / 16 * 4;  // whole 16-row blocks: rows past the bound give zero codes
+  for (int64_t u = blockIdx.x; u < units; u += gridDim.x) {
+    uint4 raw[4][CPT];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int64_t m = u * 4 + r;
+#pragma unroll
+      for (int i = 0; i < CPT; ++i) {
+        const int c = (int)threadIdx.x + 1024 * i;
+        raw[r][i] = (m < rows && c < nch) ? *reinterpret_cast<const uint4*>(x + m * ldx + (int64_t)c * 8)
+                                          : make_uint4(0u, 0u, 0u, 0u);
+      }
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      float v = 0.f;
+#pragma unroll
+      for (int i = 0; i < CPT; ++i) v = fmaxf(v, amax8(raw[r][i], dtype));
+      v = wave_max(v);
+      if (lane == 0) red[r][wave] = v;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      float v = red[r][lane & 15];
+      v = fmaxf(v, dpp_f<kDppXor1>(v));
+      v = fmaxf(v, dpp_f<kDppXor2>(v));
+      v = fmaxf(v, dpp_f<kDppHalfMirror>(v));
+      v = fmaxf(v, dpp_f<kDppRowMirror>(v));
+      const int64_t m = u * 4 + r;
+      const float s = act_row_scale(v);
+      const float inv = 1.0f / s;
+      if (threadIdx.x == 0 && m < rows) scales[m] = s;
+      uint8_t* dst = qt + (m >> 4) * KT * 2048 + (m & 15) * 16;
+#pragma unroll
+      for (int i = 0; i < CPT; ++i) {
+        const int c = (int)threadIdx.x + 1024 * i;
+        if (c < nch) {
+          float f[8];
+          unpack8(raw[r][i], dtype, f);
+          // chunk c: tile c / 16, half (c % 16) / 8, 16-byte piece (c % 8) / 2, its half c % 2
+          *reinterpret_cast<uint2*>(dst + (int64_t)(c >> 3) * 1024 + ((c >> 1) & 3) * 256 + (c & 1) * 8) = quant8(f, inv);
+        }
+      }
+    }
+    __syncthreads();  // red is rewritten for the next rows
   }
 }
 
@@ -349,6 +421,7 @@ static int launch_act_quant_tiled_lds(const uint16_t* x, int dtype, int64_t M, i
   return hipGetLastError() == hipSuccess ? kOk : kErrHip;
 }
 
+// seeds null: the GEMM needs none (only symmetric int4 does)
 int launch_act_quant_tiled(const void* x, int dtype, int64_t M, int64_t K, int64_t ldx, uint8_t* qt, float* scales,
                            float* seeds, int64_t seeds_ld, const int32_t* row_count, hipStream_t stream) {
   if (M <= 0) return kOk;
@@ -362,6 +435,12 @@ int launch_act_quant_tiled(const void* x, int dtype, int64_t M, int64_t K, int64
   if (cpl <= 4) return launch_act_quant_tiled_lds<4>(xp, dtype, M, K, ldx, qt, scales, seeds, seeds_ld, row_count, stream);
   if (cpl <= 8) return launch_act_quant_tiled_lds<8>(xp, dtype, M, K, ldx, qt, scales, seeds, seeds_ld, row_count, stream);
   const int64_t nblk = (M + 15) / 16;
+  if (!seeds && K <= 2 * 8192) {
+    const dim3 g((unsigned)(nblk < 4096 ? nblk * 4 : 16384)), b(1024);
+    auto kern = K <= 8192 ? act_quant_tiled_rows_kernel<1> : act_quant_tiled_rows_kernel<2>;
+    hipLaunchKernelGGL(kern, g, b, 0, stream, xp, ldx, M, K, dtype, qt, scales, row_count);
+    return hipGetLastError() == hipSuccess ? kOk : kErrHip;
+  }
   const dim3 g((unsigned)(nblk < 8192 ? nblk : 8192)), b(1024);
   hipLaunchKernelGGL(act_quant_tiled_kernel, g, b, 0, stream, reinterpret_cast<const uint16_t*>(x), ldx, M, K, dtype,
                      qt, scales, seeds, seeds_ld, row_count);

@@ -128,3 +128,27 @@ def test_wide_tile_matches_the_others(kernels, dev, M, N, K, silu, asym, g):
                             abi.stream_of(x)), "w4a8_gemm")
     torch.cuda.synchronize()
     assert torch.equal(out, ref), f"max {(out.float() - ref.float()).abs().max().item():.3e}"
+
+
+@pytest.mark.parametrize("fmt", ["asym", "mxfp4"])
+@pytest.mark.parametrize("M,K", [(1024, 4224), (1037, 8192), (1026, 8320), (1100, 16384), (1030, 16512)])
+def test_long_rows_quantized_in_operand_order(kernels, dev, fmt, M, K):
+    """Rows of more than 4096 elements on formats without seeds: four rows per workgroup up to 16384
+    elements (one and two chunks per thread, ragged row blocks), two passes beyond, bit for bit against
+    the row-major quant and GEMM."""
+    N = 2048
+    abi = pkg("_abi")
+    lib = abi.load()
+    w, s, z, e2, _ = _weight(fmt, 128, N, K, seed=K)
+    tiles, sd, zd = kernels.repack_w4(w.to(dev), e2), s.to(dev), None if z is None else z.to(dev)
+    x = synth.activations(M, K, seed=M, outliers=True).to(dev)
+    x[3] = 0
+    q, sc = kernels.act_quant(x)
+    out = kernels.w4a8_linear(x, tiles, sd, zd, 32 if e2 else 128, weight_is_e2m1=e2)
+    ref = torch.empty_like(out)
+    abi.check(lib.w4a8_gemm(abi.ptr(q), K, abi.ptr(sc), M, abi.ptr(tiles), N, K, abi.ptr(sd),
+                            abi.SCALE_E8M0 if e2 else abi.SCALE_F16, abi.ptr(zd), abi.W_E2M1 if e2 else abi.W_INT4,
+                            32 if e2 else 128, abi.ptr(ref), abi.BF16, N, 0, None, 0, abi.KERNEL_PREFILL,
+                            abi.stream_of(x)), "w4a8_gemm")
+    torch.cuda.synchronize()
+    assert torch.equal(out, ref)
