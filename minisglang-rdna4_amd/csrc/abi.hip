@@ -24,6 +24,7 @@ size_t gemv_workspace_bytes(int64_t M, int64_t N, int64_t K, int grouped, int64_
 int launch_prefill(const GemmArgs& p, int64_t rows_to_cover, int bm_rows, hipStream_t stream);
 int launch_prefill_staged(const GemmArgs& p, int64_t rows_to_cover, int bm_rows, hipStream_t stream);
 int launch_prefill_dma(const GemmArgs& p, int64_t rows_to_cover, int bm_rows, hipStream_t stream);
+bool prefill_takes_wide(const GemmArgs& p);
 int launch_moe_route(const void* logits, int dtype, int64_t T, int E, int top_k, int renorm, float* tw,
                      int32_t* ids, hipStream_t stream);
 int launch_moe_align(const int32_t* ids, int64_t numel, int E, int bm, int64_t P, int32_t* sorted_ids,
@@ -107,12 +108,31 @@ static int64_t tiled_min_n() {
   }();
   return n;
 }
-static bool dma_tiled_ok(const GemmArgs& p, int64_t min_n = 16384) {
-  const int64_t min_rows = tiled_min_rows();
+static bool dma_tiled_ok(const GemmArgs& p, int64_t min_n, int64_t min_rows) {
   const bool int4 = p.wfmt == kInt4 && p.sfmt == kScaleF16 && p.group % 128 == 0;  // with zeros: no seeds
   const bool mx = p.wfmt == kE2M1 && p.sfmt == kScaleE8M0 && p.group == 32;  // MXFP4: A layout only, no seeds
   return min_rows > 0 && p.M >= min_rows && p.N >= min_n && (int4 || mx) && p.K % 128 == 0 && p.KT >= 3 && !(p.silu && (p.N / 16) % 2) &&
          p.N * p.KT * 64 < ((int64_t)1 << 31) && p.M * p.K < ((int64_t)1 << 31);
+}
+static bool dma_tiled_ok(const GemmArgs& p) { return dma_tiled_ok(p, 16384, tiled_min_rows()); }
+
+// w4a8_linear's own calls, whose quant is one launch in either layout, take it below that too:
+//  - int4 where the 256 x 256 tile is the cheapest of its grid (it takes operand order only). us, 1024
+//    rows and up only -> this: K=4096 N=28672 M=512 86 -> 72 and M=448 52.0 -> 45.7, K=8192 N=14336 M=900
+//    93 -> 77, AWQ K=4096 N=14336 M=1000 51.0 -> 45.5. On the smaller tiles it loses: K=14336 N=4096 M=512
+//    62 -> 78 (two quant passes over few rows), K=4096 N=6144 M=512 32 -> 34, N=14336 M=129 28 -> 31;
+//  - MXFP4 up to K=16384: K=14336 N=4096 M=200 23.7 -> 18.4 and M=700 44.1 -> 32.1, K=8192 N=8192 M=700
+//    37.1 -> 29.5, K=4096 N=14336 M=200 16.1 -> 13.9 (M=400 20.1 -> 20.4), K=8192 N=28672 M=200 to 1000
+//    within 3%. Longer rows take the two-pass quant: K=28672 N=8192 M=200 52.5 -> 65.4.
+// Below 128 rows nothing was measured to gain.
+static const int64_t kTiledFewRows = 128;
+static int64_t linear_tiled_min_rows() {
+  const int64_t n = tiled_min_rows();
+  return n < kTiledFewRows ? n : kTiledFewRows;
+}
+static bool linear_tiled_ok(const GemmArgs& p) {
+  if (p.M >= tiled_min_rows()) return dma_tiled_ok(p, tiled_min_n(), tiled_min_rows());
+  return dma_tiled_ok(p, tiled_min_n(), linear_tiled_min_rows()) && (p.wfmt == kE2M1 ? p.K <= 16384 : prefill_takes_wide(p));
 }
 
 // Bound on align blocks that can hold routed rows: every expert with rows contributes
@@ -150,13 +170,12 @@ static int check_weights(const char* who, int64_t N, int64_t K, int scale_fmt, c
 }
 
 // w4a8_linear's workspace: the row-major codes and scales of x (what every call needs), then for
-// the calls that may take the tiled prefill (tiled_min_rows) the codes of whole 16-row blocks in
+// the calls that may take the tiled prefill (linear_tiled_min_rows) the codes of whole 16-row blocks in
 // the GEMM's operand order and one row-sum seed per row and K tile. A workspace of only the first
 // part is accepted; such calls run the row-major GEMM, with the same results.
 static int64_t round256(int64_t b);
 static int64_t linear_ws_rowmajor(int64_t M, int64_t K) { return round256(M * K) + round256(M * 4); }
-static int64_t linear_ws_tiled(int64_t M, int64_t K) {
-  const int64_t min_rows = tiled_min_rows();
+static int64_t linear_ws_tiled(int64_t M, int64_t K, int64_t min_rows) {
   if (min_rows <= 0 || M < min_rows) return 0;
   const int64_t Mp = (M + 15) / 16 * 16, KT = (K + 127) / 128;
   return round256(Mp * K) + round256(KT * Mp * 4);
@@ -218,8 +237,8 @@ int w4a8_repack_weights(const int32_t* w_packed, int64_t N, int64_t K, int wfmt,
 int64_t w4a8_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int kernel) {
   if (M < 0 || N <= 0 || K <= 0) return -1;
   // prefill: room for the codes rewritten in the GEMM's operand order with their row-sum seeds,
-  // which wide symmetric int4 weights take (the call runs without it too, on the row-major codes)
-  if (kernel == 2 || (kernel == 0 && M > kGemvMaxRows)) return N >= 16384 ? linear_ws_tiled(M, K) : 0;
+  // which wide int4 and MXFP4 weights take (the call runs without it too, on the row-major codes)
+  if (kernel == 2 || (kernel == 0 && M > kGemvMaxRows)) return N >= 16384 ? linear_ws_tiled(M, K, tiled_min_rows()) : 0;
   return (int64_t)gemv_workspace_bytes(M, N, K, 0, (M + 15) / 16);
 }
 
@@ -279,7 +298,7 @@ int w4a8_gemm(const uint8_t* x_fp8, int64_t ldx, const float* act_scales, int64_
   p.xq = x_fp8; p.ldx = ldx; p.act_scales = act_scales;
   const hipStream_t st = (hipStream_t)stream;
   const bool decode = kernel == 1 || (kernel == 0 && M <= kGemvMaxRows);
-  if (!decode && dma_tiled_ok(p) && workspace && aligned16(workspace) && workspace_bytes >= linear_ws_tiled(M, K)) {
+  if (!decode && dma_tiled_ok(p) && workspace && aligned16(workspace) && workspace_bytes >= linear_ws_tiled(M, K, tiled_min_rows())) {
     // the caller's codes rewritten in the GEMM's operand order with their seeds (as w4a8_linear)
     const int64_t Mp = (M + 15) / 16 * 16;
     uint8_t* xt = reinterpret_cast<uint8_t*>(workspace);
@@ -296,7 +315,7 @@ int w4a8_gemm(const uint8_t* x_fp8, int64_t ldx, const float* act_scales, int64_
 
 int64_t w4a8_linear_workspace_bytes(int64_t M, int64_t K) {
   if (M < 0 || K <= 0) return -1;
-  return linear_ws_rowmajor(M, K) + linear_ws_tiled(M, K);
+  return linear_ws_rowmajor(M, K) + linear_ws_tiled(M, K, linear_tiled_min_rows());
 }
 
 int w4a8_linear(const void* x, int x_dtype, int64_t M, int64_t K, int64_t ldx, const void* w_tile, int64_t N,
@@ -323,7 +342,7 @@ int w4a8_linear(const void* x, int x_dtype, int64_t M, int64_t K, int64_t ldx, c
                 (long long)workspace_bytes);
   uint8_t* xq = reinterpret_cast<uint8_t*>(workspace);
   float* xs = reinterpret_cast<float*>(xq + round256(M * K));
-  if (!decode && dma_tiled_ok(p, tiled_min_n()) && workspace_bytes >= need + linear_ws_tiled(M, K)) {
+  if (!decode && linear_tiled_ok(p) && workspace_bytes >= need + linear_ws_tiled(M, K, linear_tiled_min_rows())) {
     // prefill on the DMA-staged kernel: x quantized straight into its operand order, with the seeds
     const int64_t Mp = (M + 15) / 16 * 16;
     uint8_t* xt = reinterpret_cast<uint8_t*>(xs) + round256(M * 4);

@@ -380,7 +380,7 @@ inline int pick_tile(const DmaTile (&tiles)[NT], const GemmArgs& p, int64_t rows
 
 // Launch of the DMA-staged kernel (gemm_prefill_dma.hip); kErrUnsupported when it does not apply.
 int launch_prefill_dma(const GemmArgs& p, int64_t rows_to_cover, int bm_rows, hipStream_t stream);
-// Dense symmetric int4 on 256 x 256 tiles, A in operand order (gemm_prefill_wide.hip).
+// Dense int4 in groups of 128+ on 256 x 256 tiles, A in operand order (gemm_prefill_wide.hip).
 int launch_prefill_wide(const GemmArgs& p, int64_t rows, hipStream_t stream);
 // NVFP4 on the fp16 MFMA (gemm_prefill_nv.hip); kErrUnsupported for other formats and shapes.
 int launch_prefill_nv(const GemmArgs& p, int64_t rows_to_cover, int bm_rows, hipStream_t stream);

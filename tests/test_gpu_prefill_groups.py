@@ -7,7 +7,7 @@ import torch
 
 import synth
 from conftest import pkg
-from test_gpu_dense import assert_close_to_oracle
+from test_gpu_dense import _row_major_gemm, assert_close_to_oracle
 from test_gpu_moe import _stagewise
 
 pytestmark = pytest.mark.gpu
@@ -150,5 +150,23 @@ def test_long_rows_quantized_in_operand_order(kernels, dev, fmt, M, K):
                             abi.SCALE_E8M0 if e2 else abi.SCALE_F16, abi.ptr(zd), abi.W_E2M1 if e2 else abi.W_INT4,
                             32 if e2 else 128, abi.ptr(ref), abi.BF16, N, 0, None, 0, abi.KERNEL_PREFILL,
                             abi.stream_of(x)), "w4a8_gemm")
+    torch.cuda.synchronize()
+    assert torch.equal(out, ref)
+
+
+# below 1024 rows: int4 where 256 x 256 tiles fit the grid (one quant kernel each side of K = 4096),
+# MXFP4 from 128 rows up to K = 16384, and one row or K tile outside each
+@pytest.mark.parametrize("fmt,M,N,K", [("sym", 448, 28672, 512), ("sym", 511, 24576, 4224), ("asym", 500, 28672, 384),
+                                        ("asym", 1023, 14336, 4224), ("mxfp4", 127, 2048, 384), ("mxfp4", 128, 2048, 384),
+                                        ("mxfp4", 129, 2064, 4224), ("mxfp4", 1023, 2048, 16384),
+                                        ("mxfp4", 200, 2048, 16512), ("mxfp4", 130, 2032, 512)])
+def test_few_rows_in_operand_order(kernels, dev, fmt, M, N, K):
+    w, s, z, e2, _ = _weight(fmt, 128, N, K, seed=M + K)
+    g = 32 if e2 else 128
+    tiles, sd, zd = kernels.repack_w4(w.to(dev), e2), s.to(dev), None if z is None else z.to(dev)
+    x = synth.activations(M, K, seed=M, outliers=True).to(dev)
+    q, sc = kernels.act_quant(x)
+    out = kernels.w4a8_linear(x, tiles, sd, zd, g, weight_is_e2m1=e2)
+    ref = _row_major_gemm(q, sc, tiles, sd, zd, g, N, K, e2, x.dtype)
     torch.cuda.synchronize()
     assert torch.equal(out, ref)
