@@ -121,9 +121,10 @@ static bool dma_tiled_ok(const GemmArgs& p) { return dma_tiled_ok(p, 16384, tile
 //    rows and up only -> this: K=4096 N=28672 M=512 86 -> 72 and M=448 52.0 -> 45.7, K=8192 N=14336 M=900
 //    93 -> 77, AWQ K=4096 N=14336 M=1000 51.0 -> 45.5. On the smaller tiles it loses: K=14336 N=4096 M=512
 //    62 -> 78 (two quant passes over few rows), K=4096 N=6144 M=512 32 -> 34, N=14336 M=129 28 -> 31;
-//  - MXFP4 up to K=16384: K=14336 N=4096 M=200 23.7 -> 18.4 and M=700 44.1 -> 32.1, K=8192 N=8192 M=700
+//  - MXFP4 up to K=32768: K=14336 N=4096 M=200 23.7 -> 18.4 and M=700 44.1 -> 32.1, K=8192 N=8192 M=700
 //    37.1 -> 29.5, K=4096 N=14336 M=200 16.1 -> 13.9 (M=400 20.1 -> 20.4), K=8192 N=28672 M=200 to 1000
-//    within 3%. Longer rows take the two-pass quant: K=28672 N=8192 M=200 52.5 -> 65.4.
+//    within 3%; K=28672 N=8192 M=130 88.7 -> 81.0, M=400 136 -> 115, M=1000 189 -> 194, K=24576 N=4096
+//    M=130 60.6 -> 48.0. Longer rows take the two-pass quant, which lost at few rows (M=130 88.7 -> 108).
 // Below 128 rows nothing was measured to gain.
 static const int64_t kTiledFewRows = 128;
 static int64_t linear_tiled_min_rows() {
@@ -132,7 +133,7 @@ static int64_t linear_tiled_min_rows() {
 }
 static bool linear_tiled_ok(const GemmArgs& p) {
   if (p.M >= tiled_min_rows()) return dma_tiled_ok(p, tiled_min_n(), tiled_min_rows());
-  return dma_tiled_ok(p, tiled_min_n(), linear_tiled_min_rows()) && (p.wfmt == kE2M1 ? p.K <= 16384 : prefill_takes_wide(p));
+  return dma_tiled_ok(p, tiled_min_n(), linear_tiled_min_rows()) && (p.wfmt == kE2M1 ? p.K <= 32768 : prefill_takes_wide(p));
 }
 
 // Bound on align blocks that can hold routed rows: every expert with rows contributes

@@ -327,14 +327,16 @@ act_quant_tiled_short_kernel(const uint16_t* __restrict__ x, int64_t ldx, int64_
   }
 }
 
-// The same for rows of 4097 to 16384 elements, with x read once: a workgroup of 16 waves holds 4 rows in
+// The same for rows of 4097 to 16384 elements, and of up to 32768 in calls of up to 1024 rows, with x read once: a workgroup of 16 waves holds 4 rows in
 // registers (thread t: the 8-element chunks t + 1024 i of each), takes their maxima through one barrier,
 // and writes each chunk's 8 codes straight to their operand-order place. Four rows are the fewest whose
 // pieces fill a 64-byte segment of the output (4 rows x 16 bytes), which L2 then writes whole. The
 // two-pass kernel has a quarter as many workgroups and reads x twice: whole MXFP4 calls at K=8192 N=8192
-// M=1024 66.5 -> 59.3 us, K=14336 N=4096 M=2000 109 -> 106. Longer rows (four chunks per thread) spill:
-// K=28672 M=4096 106 -> 170 us, so they keep the two passes, as do the calls that need seeds (the tiles
-// pass through its registers, where reading the codes back would cost what the second read of x does).
+// M=1024 66.5 -> 59.3 us, K=14336 N=4096 M=2000 109 -> 106. Longer rows need it only while the two passes
+// have few workgroups: K=28672 N=8192 M=1024 209 -> 193 us and M=400 136 -> 115, K=24576 N=4096 M=1024
+// 119 -> 103, but K=28672 N=8192 M=2000 344 -> 349 and M=4096 690 -> 705. Calls that need seeds keep the two
+// passes (the tiles pass through its registers, where reading the codes back would cost what the second
+// read of x does).
 template <int CPT>
 __global__ void __launch_bounds__(1024)
 act_quant_tiled_rows_kernel(const uint16_t* __restrict__ x, int64_t ldx, int64_t M, int64_t K, int dtype,
@@ -371,6 +373,13 @@ act_quant_tiled_rows_kernel(const uint16_t* __restrict__ x, int64_t ldx, int64_t
     __syncthreads();
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
+      // long rows: the maximum's unpacked values are not kept for the codes, which would spill; at one and
+      // two chunks they fit, and unpacking again costs (K=14336 N=4096 M=130 29.4 -> 31.4 us)
+      if constexpr (CPT > 2) {
+#pragma unroll
+        for (int i = 0; i < CPT; ++i)
+          asm volatile("" : "+v"(raw[r][i].x), "+v"(raw[r][i].y), "+v"(raw[r][i].z), "+v"(raw[r][i].w));
+      }
       float v = red[r][lane & 15];
       v = fmaxf(v, dpp_f<kDppXor1>(v));
       v = fmaxf(v, dpp_f<kDppXor2>(v));
@@ -435,9 +444,11 @@ int launch_act_quant_tiled(const void* x, int dtype, int64_t M, int64_t K, int64
   if (cpl <= 4) return launch_act_quant_tiled_lds<4>(xp, dtype, M, K, ldx, qt, scales, seeds, seeds_ld, row_count, stream);
   if (cpl <= 8) return launch_act_quant_tiled_lds<8>(xp, dtype, M, K, ldx, qt, scales, seeds, seeds_ld, row_count, stream);
   const int64_t nblk = (M + 15) / 16;
-  if (!seeds && K <= 2 * 8192) {
+  if (!seeds && (K <= 16384 || (K <= 32768 && nblk <= 64))) {
     const dim3 g((unsigned)(nblk < 4096 ? nblk * 4 : 16384)), b(1024);
-    auto kern = K <= 8192 ? act_quant_tiled_rows_kernel<1> : act_quant_tiled_rows_kernel<2>;
+    auto kern = K <= 8192 ? act_quant_tiled_rows_kernel<1>
+                          : K <= 16384 ? act_quant_tiled_rows_kernel<2>
+                          : K <= 24576 ? act_quant_tiled_rows_kernel<3> : act_quant_tiled_rows_kernel<4>;
     hipLaunchKernelGGL(kern, g, b, 0, stream, xp, ldx, M, K, dtype, qt, scales, row_count);
     return hipGetLastError() == hipSuccess ? kOk : kErrHip;
   }

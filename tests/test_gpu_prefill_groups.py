@@ -134,8 +134,8 @@ def test_wide_tile_matches_the_others(kernels, dev, M, N, K, silu, asym, g):
 @pytest.mark.parametrize("M,K", [(1024, 4224), (1037, 8192), (1026, 8320), (1100, 16384), (1030, 16512)])
 def test_long_rows_quantized_in_operand_order(kernels, dev, fmt, M, K):
     """Rows of more than 4096 elements on formats without seeds: four rows per workgroup up to 16384
-    elements (one and two chunks per thread, ragged row blocks), two passes beyond, bit for bit against
-    the row-major quant and GEMM."""
+    elements (one and two chunks per thread, ragged row blocks), two passes beyond on more than 1024 rows,
+    bit for bit against the row-major quant and GEMM."""
     N = 2048
     abi = pkg("_abi")
     lib = abi.load()
@@ -155,11 +155,13 @@ def test_long_rows_quantized_in_operand_order(kernels, dev, fmt, M, K):
 
 
 # below 1024 rows: int4 where 256 x 256 tiles fit the grid (one quant kernel each side of K = 4096),
-# MXFP4 from 128 rows up to K = 16384, and one row or K tile outside each
+# MXFP4 from 128 rows up to K = 32768 (three and four chunks per thread), and one row or K tile outside each
 @pytest.mark.parametrize("fmt,M,N,K", [("sym", 448, 28672, 512), ("sym", 511, 24576, 4224), ("asym", 500, 28672, 384),
                                         ("asym", 1023, 14336, 4224), ("mxfp4", 127, 2048, 384), ("mxfp4", 128, 2048, 384),
                                         ("mxfp4", 129, 2064, 4224), ("mxfp4", 1023, 2048, 16384),
-                                        ("mxfp4", 200, 2048, 16512), ("mxfp4", 130, 2032, 512)])
+                                        ("mxfp4", 200, 2048, 16512), ("mxfp4", 130, 2032, 512), ("mxfp4", 1023, 2048, 24576),
+                                        ("mxfp4", 131, 2048, 24704), ("mxfp4", 1024, 2048, 32768),
+                                        ("mxfp4", 1025, 2048, 28672), ("mxfp4", 200, 2048, 32896)])
 def test_few_rows_in_operand_order(kernels, dev, fmt, M, N, K):
     w, s, z, e2, _ = _weight(fmt, 128, N, K, seed=M + K)
     g = 32 if e2 else 128
