@@ -140,6 +140,8 @@ gemm_dma_kernel(const GemmArgs p) {
   // A block b = wave + i*NW of a step is row block b/2, half b%2; lane l reads row (l & 15) of it,
   // bytes [64*half + 16*(l >> 4), +16) of the step's 128
   // AT: block b's 1 KiB sits whole in the tiled codes (row blocks past M read the last one)
+  // kKTail: K may end inside a tile (formats with groups below 128 only; A in operand order has whole ones)
+  constexpr bool kKTail = (GPT > 1 || kFp4) && !AT;
   uint32_t a_voff[A_PER];
   const int64_t nblk16 = (p.M + 15) / 16;
 #pragma unroll
@@ -155,8 +157,6 @@ gemm_dma_kernel(const GemmArgs p) {
       a_voff[i] = (uint32_t)((ok ? ar : 0) * p.ldx) + (b & 1) * 64 + 16 * (lane >> 4);
     }
   }
-  // K past the last whole tile (formats with groups below 128 only; A in operand order has none)
-  constexpr bool kKTail = (GPT > 1 || kFp4) && !AT;
   const int ktail = K - (KT - 1) * kTileK;
   const uint32_t a_back = (wave & 1) * 64 + 16 * (lane >> 4) >= ktail ? kTileK : 0;
   static_assert(NW % 2 == 0, "a wave's A blocks are all the same half");
@@ -198,8 +198,7 @@ gemm_dma_kernel(const GemmArgs p) {
     for (int i = 0; i < B_DMA; ++i) {
       bool ok;
       b_gs[i] = gstrip(wave + i * NW, ok);
-      const int m = lane & 15;
-      e_voff[i] = (uint32_t)((m >> 2) * N + b_gs[i] * 16 + (m & 3) * 4);
+      e_voff[i] = e8m0_word(lane, b_gs[i], N);
     }
   }
   // int4: chunk c = tid + i*T is lane c & 63 of strip c >> 6; scales 2 chunks of 16 B per strip,
@@ -220,16 +219,14 @@ gemm_dma_kernel(const GemmArgs p) {
       const int gs = gstrip(c >> 6, ok);
       b_voff[i] = (uint32_t)(((size_t)gs * KT * 64 + (c & 63)) * 16);
       if constexpr (kLutZ) {
-        // the chunk's first 16 codes are K 16q.. of the tile, the other 16 K 64 + 16q..: groups
-        // q * GPT / 8 and that + GPT / 2
         const int l = c & 63, n = gs * 16 + (l & 15);
-        z_voff[i] = (uint32_t)((((l >> 4) * GPT / 8) * (N / 8) + n / 8) * 4);
+        z_voff[i] = zero_word(l, n, GPT, N);
         z_sh[i] = 4 * (n & 7);
       }
     }
     bool ok;
     const int sc_s = sc_c % (NSTRIP * 2), sc_g = sc_c / (NSTRIP * 2);
-    s_voff = (uint32_t)((sc_g * N + gstrip(sc_s >> 1, ok) * 16 + (sc_s & 1) * 8) * 2);
+    s_voff = scale_piece(sc_g, gstrip(sc_s >> 1, ok), sc_s & 1, N);
   }
 
   // int4 register sets, one per stage index (two are live at a time)
@@ -256,9 +253,8 @@ gemm_dma_kernel(const GemmArgs p) {
     if constexpr (kFp4) {
 #pragma unroll
       for (int i = 0; i < S_DMA; ++i) {  // scale rows past K: out of the buffer's range, so zeros
-        const uint32_t so_e = (uint32_t)__builtin_amdgcn_readfirstlane(kt * 4 * N);
-        lds_dma4(rs_s, st + S::kA + S::kB + (wave + i * NW) * 256, kRagged ? e_voff[i] + so_e : e_voff[i],
-                 kRagged ? 0 : so_e);
+        const BufOffset o = row_step(e_voff[i], (uint32_t)__builtin_amdgcn_readfirstlane(kt * 4 * N), kRagged);
+        lds_dma4(rs_s, st + S::kA + S::kB + (wave + i * NW) * 256, o.v, o.s);
       }
     }
     const uint32_t so_a = (uint32_t)__builtin_amdgcn_readfirstlane(AT ? kt * 2048 : kt * kTileK);
@@ -283,14 +279,17 @@ gemm_dma_kernel(const GemmArgs p) {
 #pragma unroll
       for (int i = 0; i < B_PER; ++i) rbw[R][i] = bload128v(rs_w, b_voff[i], so_b);
       const int g = GPT > 1 ? kt * GPT : kt >> gshift;
-      const uint32_t so_s = (uint32_t)__builtin_amdgcn_readfirstlane(g * N * 2);
-      rsc[R] = kRagged ? bload128(rs_s, s_voff + so_s, 0) : bload128(rs_s, s_voff, so_s);  // past K: zeros
+      const BufOffset o = row_step(s_voff, (uint32_t)__builtin_amdgcn_readfirstlane(g * N * 2), kRagged);
+      rsc[R] = bload128(rs_s, o.v, o.s);  // scale and zero rows past K: out of the buffers' ranges, so zeros
       if constexpr (kLutZ) {
 #pragma unroll
         for (int i = 0; i < B_PER; ++i)
 #pragma unroll
-          for (int h = 0; h < ZL; ++h)
-            rzp[R][i][h] = bload32(rs_z, z_voff[i], (uint32_t)__builtin_amdgcn_readfirstlane((g + h * (GPT / 2)) * (N / 8) * 4));
+          for (int h = 0; h < ZL; ++h) {
+            const uint32_t so_z = (uint32_t)__builtin_amdgcn_readfirstlane((g + h * (GPT / 2)) * (N / 8) * 4);
+            const BufOffset oz = row_step(z_voff[i], so_z, kRagged);
+            rzp[R][i][h] = bload32(rs_z, oz.v, oz.s);
+          }
       }
     }
   };

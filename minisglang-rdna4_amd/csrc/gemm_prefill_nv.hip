@@ -157,7 +157,7 @@ gemm_nv_kernel(const GemmArgs p) {
     bool ok;
     const int gs = gstrip(c >> 6, ok);
     w_voff[i] = (uint32_t)(((size_t)gs * KT * 64 + (c & 63)) * 16);
-    s_voff[i] = (uint32_t)(2 * ((c & 63) >> 4) * N + gs * 16 + (c & 15));
+    s_voff[i] = e4m3_byte(c & 63, 0, gs, N);
   }
 
   v4u rw[3][B_PER];
@@ -175,8 +175,9 @@ gemm_nv_kernel(const GemmArgs p) {
 #pragma unroll
     for (int i = 0; i < B_PER; ++i) {
       rw[R][i] = bload128v(rs_w, w_voff[i], so_w);
-      rs0[R][i] = bload8(rs_s, s_voff[i] + so_s, 0);  // scale rows past K: out of range, so zeros
-      rs1[R][i] = bload8(rs_s, s_voff[i] + N + so_s, 0);
+      const BufOffset o = row_step(s_voff[i], so_s, true);  // scale rows past K: out of range, so zeros
+      rs0[R][i] = bload8(rs_s, o.v, o.s);
+      rs1[R][i] = bload8(rs_s, o.v + N, o.s);
     }
   };
   // B registers of set R -> fp16 operands in B stage BI

@@ -4,6 +4,7 @@
 #pragma once
 #include <type_traits>
 
+#include "buf_offsets.h"
 #include "gemm_args.h"
 
 namespace w4a8 {

@@ -130,7 +130,8 @@ __device__ __forceinline__ float from_dtype(uint16_t h, int dtype) {
 }
 
 // ---- buffer loads: wave-uniform base and size in a resource descriptor (SGPRs), 32-bit per-lane
-// offset, and a scalar offset that the compiler computes with SALU. Loads past `bytes` return 0.
+// offset, and a scalar offset that the compiler computes with SALU. Loads whose per-lane offset is past
+// `bytes` return 0; the scalar offset is not part of that check.
 typedef unsigned int v4u __attribute__((ext_vector_type(4)));
 typedef __amdgpu_buffer_rsrc_t BufRsrc;
 

@@ -1,0 +1,71 @@
+"""The prefill kernels' loads in the tiles of a K that is no multiple of 128, walked on the CPU: csrc/
+buf_offsets.h, whose functions form every offset of those loads, compiled for the host and asked for each
+lane of each step. A load must lie inside the matrix it reads (the last expert's, with nothing behind it)
+or past the size that the unit checks its vector offset against, where it gives zeros."""
+import subprocess
+
+import pytest
+
+from conftest import REPO
+
+WALK = r"""
+#include <cstdio>
+#include <cstdlib>
+#include "buf_offsets.h"
+using namespace w4a8;
+
+static void fail(const char* what, int K, int N, int g, int kt, int lane, BufOffset o) {
+  printf("%s: K=%d N=%d group=%d tile %d lane %d: offsets %u + %u\n", what, K, N, g, kt, lane, o.v, o.s);
+  exit(1);
+}
+// inside the matrix, or wholly past its checked size
+static void load(const char* what, BufOffset o, uint64_t size, uint64_t bytes, int K, int N, int g, int kt, int lane) {
+  const uint64_t at = (uint64_t)o.v + o.s;
+  if (!(at + size <= bytes || o.v >= bytes)) fail(what, K, N, g, kt, lane, o);
+}
+
+int main(int argc, char** argv) {
+  const int K = atoi(argv[1]), N = atoi(argv[2]), KT = (K + 127) / 128;
+  for (int kt = 0; kt < KT; ++kt) {
+    // the kernels hand `ragged` to the steps that may load the last tile; steps before it are in range either way
+    const bool ragged = kt == KT - 1;
+    for (int lane = 0; lane < 64; ++lane)
+      for (int strip = 0; strip < N / 16; ++strip) {
+        for (int g = 32; g <= 64; g *= 2) {
+          if (K % g) continue;
+          const int gpt = 128 / g;
+          const uint64_t groups = K / g, z_bytes = groups * (N / 8) * 4, s_bytes = groups * N * 2;
+          for (int h = 0; h < 2; ++h)
+            load("zero words", row_step(zero_word(lane, strip * 16 + (lane & 15), gpt, N),
+                                        (uint32_t)((kt * gpt + h * (gpt / 2)) * (N / 8) * 4), ragged), 4, z_bytes, K, N, g, kt, lane);
+          for (int c = 0; c < gpt; ++c)
+            load("scales", row_step(scale_piece(c, strip, lane & 1, N), (uint32_t)(kt * gpt * N * 2), ragged), 16, s_bytes, K,
+                 N, g, kt, lane);
+        }
+        if (K % 32 == 0)
+          load("E8M0 bytes", row_step(e8m0_word(lane, strip, N), (uint32_t)(kt * 4 * N), ragged), 4, (uint64_t)K / 32 * N, K,
+               N, 32, kt, lane);
+        for (int h = 0; h < 2; ++h)
+          load("e4m3 bytes", row_step(e4m3_byte(lane, h, strip, N), (uint32_t)(kt * 8 * N), true), 1, (uint64_t)K / 16 * N, K,
+               N, 16, kt, lane);
+      }
+  }
+  return 0;
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def walk(tmp_path_factory):
+    d = tmp_path_factory.mktemp("walk")
+    (d / "walk.cpp").write_text(WALK)
+    subprocess.run(["g++", "-O1", "-std=c++17", "-I", str(REPO / "minisglang-rdna4_amd" / "csrc"), str(d / "walk.cpp"),
+                    "-o", str(d / "walk")], check=True)
+    return d / "walk"
+
+
+@pytest.mark.parametrize("K", [160, 192, 224, 256, 480, 544, 1088])
+@pytest.mark.parametrize("N", [16, 48, 1040])
+def test_ragged_tile_loads_stay_inside(walk, K, N):
+    r = subprocess.run([str(walk), str(K), str(N)], capture_output=True, text=True)
+    assert r.returncode == 0, r.stdout
