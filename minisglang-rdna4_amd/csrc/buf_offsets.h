@@ -3,7 +3,7 @@
 //
 // Of a load's two offsets only the vector one is checked against the descriptor's size; the scalar one is
 // added behind the check. A load that may fall outside its matrix therefore carries everything in the
-// vector offset, where a read past the end gives zeros.
+// vector offset, where a read past the end gives zeros, and no vector offset goes below zero.
 #pragma once
 #include <stdint.h>
 
@@ -19,6 +19,17 @@ namespace w4a8 {
 struct BufOffset {
   uint32_t v, s;  // per lane and range-checked; wave-uniform and not
 };
+
+// A 16-byte piece of an activation row: lane l of block half h of row block b reads row (l & 15) of it
+W4A8_HD uint32_t a_piece(uint32_t row_off, int half, int lane) { return row_off + 64 * half + 16 * (lane >> 4); }
+// 128 for the lanes whose piece of a tile with ktail inputs lies past them, else 0
+W4A8_HD uint32_t a_back(int half, int lane, int ktail) { return 64 * half + 16 * (lane >> 4) >= ktail ? 128u : 0u; }
+// last: all ones for the last tile of K, else 0. There the lanes with `back` read the tile before (the
+// operand read masks theirs out). The piece's offset is from kABias bytes ahead of the activations, where
+// the descriptor starts, so that the lanes of row 0 that step back do not go below zero; every address
+// read lies inside its row.
+constexpr int kABias = 128;
+W4A8_HD uint32_t a_step(uint32_t biased_piece, uint32_t back, uint32_t last) { return biased_piece - (back & last); }
 
 // Zero word of channel n: lane l of a strip reads codes K 16q.. of the tile and K 64 + 16q.. (q = l >> 4),
 // of groups q * gpt / 8 and that + gpt / 2 (gpt groups per tile; one for groups of 128 and more)

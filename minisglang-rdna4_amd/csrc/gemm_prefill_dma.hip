@@ -142,6 +142,7 @@ gemm_dma_kernel(const GemmArgs p) {
   // AT: block b's 1 KiB sits whole in the tiled codes (row blocks past M read the last one)
   // kKTail: K may end inside a tile (formats with groups below 128 only; A in operand order has whole ones)
   constexpr bool kKTail = (GPT > 1 || kFp4) && !AT;
+  constexpr int kABase = kKTail ? kABias : 0;
   uint32_t a_voff[A_PER];
   const int64_t nblk16 = (p.M + 15) / 16;
 #pragma unroll
@@ -154,11 +155,11 @@ gemm_dma_kernel(const GemmArgs p) {
     } else {
       int64_t ar;
       const bool ok = lrow_source(p, blk_row0 + (b >> 1) * 16 + (lane & 15), ar);
-      a_voff[i] = (uint32_t)((ok ? ar : 0) * p.ldx) + (b & 1) * 64 + 16 * (lane >> 4);
+      a_voff[i] = a_piece((uint32_t)((ok ? ar : 0) * p.ldx), b & 1, lane) + kABase;
     }
   }
   const int ktail = K - (KT - 1) * kTileK;
-  const uint32_t a_back = (wave & 1) * 64 + 16 * (lane >> 4) >= ktail ? kTileK : 0;
+  const uint32_t back = a_back(wave & 1, lane, ktail);
   static_assert(NW % 2 == 0, "a wave's A blocks are all the same half");
   // seeds: wave w copies rows 64 (w % (BM / 64)) + lane of the tile (waves past BM / 64 copy the same
   // rows again, so every wave issues one DMA per step and one vmcnt count holds)
@@ -219,9 +220,8 @@ gemm_dma_kernel(const GemmArgs p) {
       const int gs = gstrip(c >> 6, ok);
       b_voff[i] = (uint32_t)(((size_t)gs * KT * 64 + (c & 63)) * 16);
       if constexpr (kLutZ) {
-        const int l = c & 63, n = gs * 16 + (l & 15);
-        z_voff[i] = zero_word(l, n, GPT, N);
-        z_sh[i] = 4 * (n & 7);
+        z_voff[i] = zero_word(lane, gs * 16 + (lane & 15), GPT, N);
+        z_sh[i] = 4 * (lane & 7);
       }
     }
     bool ok;
@@ -245,7 +245,7 @@ gemm_dma_kernel(const GemmArgs p) {
     constexpr bool kRagged = kKTail && decltype(Tail)::value;  // the last tile is always loaded by a tail step
     const uint32_t live = decltype(Tail)::value ? (uint32_t)__builtin_amdgcn_readfirstlane(kt < KT ? -1 : 0) : 0xffffffffu;
     if constexpr (decltype(Tail)::value) kt = kt < KT ? kt : KT - 1;
-    const BufRsrc rs_a = make_rsrc(p.xq, live);
+    const BufRsrc rs_a = make_rsrc(p.xq - kABase, live);
     const BufRsrc rs_w = make_rsrc(wt, w_bytes & live);
     const BufRsrc rs_s = make_rsrc(scales, s_bytes & live);
     const BufRsrc rs_z = make_rsrc(zeros, z_bytes & live);
@@ -259,12 +259,10 @@ gemm_dma_kernel(const GemmArgs p) {
     }
     const uint32_t so_a = (uint32_t)__builtin_amdgcn_readfirstlane(AT ? kt * 2048 : kt * kTileK);
     if (part & 1) {
-      // the last tile of a K that is no multiple of 128: its chunks past K read the tile before (in
-      // bounds; the operand read masks them out)
-      const uint32_t back = kRagged ? a_back & (uint32_t)__builtin_amdgcn_readfirstlane(kt == KT - 1 ? -1 : 0) : 0u;
+      const uint32_t last = kRagged ? (uint32_t)__builtin_amdgcn_readfirstlane(kt == KT - 1 ? -1 : 0) : 0u;
 #pragma unroll
       for (int i = 0; i < A_PER; ++i)
-        lds_dma16(rs_a, st + (wave + i * NW) * 1024, a_voff[i] - back, so_a);
+        lds_dma16(rs_a, st + (wave + i * NW) * 1024, a_step(a_voff[i], back, last), so_a);
       if constexpr (kSeedL)
         lds_dma4(rs_seed, st + kSeedOff + (wave % kSeedW) * 256, seed_voff,
                  (uint32_t)__builtin_amdgcn_readfirstlane(kt * (int)p.seeds_ld * 4));
@@ -679,7 +677,7 @@ int launch_prefill_dma(const GemmArgs& p, int64_t rows_to_cover, int bm_rows, hi
   // 32-bit offsets within one matrix
   if ((int64_t)p.N * p.KT * 64 >= (int64_t)1 << 31) return kErrUnsupported;
   if (p.ldx % 16) return kErrUnsupported;  // A rows are read in 16-byte pieces, at 32-bit offsets
-  if ((p.a_by_token ? p.num_slots / p.top_k : p.M) * p.ldx > (int64_t)0xffffffff) return kErrUnsupported;
+  if ((p.a_by_token ? p.num_slots / p.top_k : p.M) * p.ldx > (int64_t)0xffffffff - kABias) return kErrUnsupported;
   if (p.a_tiled && (p.sorted_ids ? ((mode != kPSym && mode != kPAsym) || p.a_by_token != 0)
                                  : (bm_rows != 0 || prefill_gpt(mode) > 1)))
     return kErrUnsupported;

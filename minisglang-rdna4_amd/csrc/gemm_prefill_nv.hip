@@ -128,7 +128,7 @@ gemm_nv_kernel(const GemmArgs p) {
   const uint4* wt = p.wt + (size_t)(expert * p.w_expert_tiles) * 64;
   const unsigned char* scales = reinterpret_cast<const unsigned char*>(p.scales) + (size_t)(expert * p.s_expert_stride);
   const int32_t* glob = p.zeros + expert * p.z_expert_stride;
-  const BufRsrc rs_a = make_rsrc(p.xq, 0xffffffffu);
+  const BufRsrc rs_a = make_rsrc(p.xq - kABias, 0xffffffffu);
   const BufRsrc rs_w = make_rsrc(wt, (uint32_t)((size_t)nstrips * KT * kTileBytes));
   const BufRsrc rs_s = make_rsrc(scales, (uint32_t)((size_t)(K / 16) * N));
 
@@ -140,12 +140,12 @@ gemm_nv_kernel(const GemmArgs p) {
     const int b = wave + i * NW;
     int64_t ar;
     const bool ok = lrow_source(p, blk_row0 + (b >> 1) * 16 + (lane & 15), ar);
-    a_voff[i] = (uint32_t)((ok ? ar : 0) * p.ldx) + (b & 1) * 64 + 16 * (lane >> 4);
+    a_voff[i] = a_piece((uint32_t)((ok ? ar : 0) * p.ldx), b & 1, lane) + kABias;
   }
   // a K that is no multiple of 128: the last tile's chunks past K read the tile before (in bounds) and
   // are cleared in the operand read
   const int ktail = K - (KT - 1) * kTileK;
-  const uint32_t a_back = (wave & 1) * 64 + 16 * (lane >> 4) >= ktail ? kTileK : 0;
+  const uint32_t back = a_back(wave & 1, lane, ktail);
   static_assert(NW % 2 == 0, "a wave's A blocks are all the same half");
   // B: fp4 tile lane c = tid + i*T is lane c & 63 of strip c >> 6; its 16 bytes are the two
   // 16-element blocks 2q', 2q'+1 (q' = lane >> 4) of channel lane & 15; their scale bytes are
@@ -167,9 +167,10 @@ gemm_nv_kernel(const GemmArgs p) {
     constexpr int R = decltype(I)::value;
     unsigned char* st = astage(I);
     const uint32_t so_a = (uint32_t)__builtin_amdgcn_readfirstlane(kt * kTileK);
-    const uint32_t back = a_back & (uint32_t)__builtin_amdgcn_readfirstlane(kt == KT - 1 ? -1 : 0);
+    const uint32_t last = (uint32_t)__builtin_amdgcn_readfirstlane(kt == KT - 1 ? -1 : 0);
 #pragma unroll
-    for (int i = 0; i < A_PER; ++i) lds_dma16(rs_a, st + (wave + i * NW) * 1024, a_voff[i] - back, so_a);
+    for (int i = 0; i < A_PER; ++i)
+      lds_dma16(rs_a, st + (wave + i * NW) * 1024, a_step(a_voff[i], back, last), so_a);
     const uint32_t so_w = (uint32_t)__builtin_amdgcn_readfirstlane(kt * kTileBytes);
     const uint32_t so_s = (uint32_t)__builtin_amdgcn_readfirstlane(kt * 8 * N);
 #pragma unroll
@@ -347,7 +348,7 @@ int launch_prefill_nv(const GemmArgs& p, int64_t rows_to_cover, int bm_rows, hip
   if ((int64_t)p.N * p.KT * 64 >= (int64_t)1 << 31) return kErrUnsupported;
   if ((p.K / 16) * p.N >= (int64_t)1 << 32) return kErrUnsupported;
   if (p.ldx % 16) return kErrUnsupported;
-  if ((p.a_by_token ? p.num_slots / p.top_k : p.M) * p.ldx > (int64_t)0xffffffff) return kErrUnsupported;
+  if ((p.a_by_token ? p.num_slots / p.top_k : p.M) * p.ldx > (int64_t)0xffffffff - kABias) return kErrUnsupported;
   // W4A8_PREFILL_NV=0 leaves NVFP4 to the per-wave kernel (A/B measurements)
   static const bool enabled = [] {
     const char* e = getenv("W4A8_PREFILL_NV");

@@ -1,7 +1,8 @@
 """The prefill kernels' loads in the tiles of a K that is no multiple of 128, walked on the CPU: csrc/
 buf_offsets.h, whose functions form every offset of those loads, compiled for the host and asked for each
 lane of each step. A load must lie inside the matrix it reads (the last expert's, with nothing behind it)
-or past the size that the unit checks its vector offset against, where it gives zeros."""
+or past the size that the unit checks its vector offset against, where it gives zeros; a row of
+activations must be read inside its K bytes and without an offset that wraps."""
 import subprocess
 
 import pytest
@@ -25,7 +26,21 @@ static void load(const char* what, BufOffset o, uint64_t size, uint64_t bytes, i
 }
 
 int main(int argc, char** argv) {
-  const int K = atoi(argv[1]), N = atoi(argv[2]), KT = (K + 127) / 128;
+  const int K = atoi(argv[1]), N = atoi(argv[2]), KT = (K + 127) / 128, ktail = K - (KT - 1) * 128;
+  const uint64_t ldx = K + 16 * atoi(argv[3]);
+  // activations: three rows, the first at offset 0 (it also stands for rows without data)
+  for (int kt = 0; kt < KT; ++kt)
+    for (int half = 0; half < 2; ++half)
+      for (int lane = 0; lane < 64; ++lane)
+        for (uint64_t row = 0; row < 3; ++row) {
+          const uint32_t from = a_piece((uint32_t)(row * ldx), half, lane) + kABias;
+          const BufOffset o = {a_step(from, a_back(half, lane, ktail), kt == KT - 1 ? ~0u : 0u), (uint32_t)(kt * 128)};
+          if (o.v > from) fail("activations (below zero)", K, N, 0, kt, lane, o);
+          const uint64_t at = (uint64_t)o.v + o.s - kABias, in = (uint64_t)kt * 128 + 64 * half + 16 * (lane >> 4);
+          if (at < row * ldx || at + 16 > row * ldx + K) fail("activations", K, N, 0, kt, lane, o);
+          // the piece itself wherever it lies inside K
+          if (in + 16 <= (uint64_t)K && at != row * ldx + in) fail("activations (place)", K, N, 0, kt, lane, o);
+        }
   for (int kt = 0; kt < KT; ++kt) {
     // the kernels hand `ragged` to the steps that may load the last tile; steps before it are in range either way
     const bool ragged = kt == KT - 1;
@@ -66,6 +81,7 @@ def walk(tmp_path_factory):
 
 @pytest.mark.parametrize("K", [160, 192, 224, 256, 480, 544, 1088])
 @pytest.mark.parametrize("N", [16, 48, 1040])
-def test_ragged_tile_loads_stay_inside(walk, K, N):
-    r = subprocess.run([str(walk), str(K), str(N)], capture_output=True, text=True)
+@pytest.mark.parametrize("pad", [0, 3])
+def test_ragged_tile_loads_stay_inside(walk, K, N, pad):
+    r = subprocess.run([str(walk), str(K), str(N), str(pad)], capture_output=True, text=True)
     assert r.returncode == 0, r.stdout
