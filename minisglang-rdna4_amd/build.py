@@ -1,5 +1,5 @@
-"""Build libw4a8_mi355x.so (gfx950) from csrc/*.hip with hipcc and w4a8_host.so (the operators' host
-path, no device code) from csrc/host.cpp with the host compiler, in-tree.
+"""Build libw4a8_mi355x.so (gfx950) from csrc/*.hip and w4a8_host.so (the operators' host path, no device
+code) from csrc/host.cpp, both with hipcc, in-tree.
 
 Objects compile in parallel into _build/, the shared library lands in _lib/. Every call
 recompiles (the build is the "does it build" check), so keep it cheap: one object per source.
@@ -47,7 +47,8 @@ def _compile(src: Path) -> Path:
 
 
 def _build_host() -> Path:
-    """csrc/host.cpp against the installed torch's C++ libraries (loaded before it at run time)."""
+    """csrc/host.cpp against the installed torch's C++ libraries (loaded before it at run time). It records
+    the torch and Python it was built for; _host.py uses it with those only."""
     import sysconfig
 
     import torch
@@ -56,8 +57,9 @@ def _build_host() -> Path:
     out = LIBDIR / "w4a8_host.so"
     tmp = out.with_suffix(".so.tmp")
     rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
-    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-shared", "-fPIC", "-fvisibility=hidden",
-           "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+    built_for = f"torch {torch.__version__}, Python {sys.version_info.major}.{sys.version_info.minor}"
+    cmd = [_hipcc(), "-no-hip-rt", "-x", "c++", "-O2", "-std=c++17", "-shared", "-fPIC", "-fvisibility=hidden",
+           "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", f'-DW4A8_BUILT_FOR="{built_for}"',
            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}",
            f"-I{tdir / 'include'}", f"-I{tdir / 'include' / 'torch' / 'csrc' / 'api' / 'include'}", f"-I{rocm}/include",
            f"-I{sysconfig.get_paths()['include']}", str(CSRC / "host.cpp"), "-o", str(tmp), f"-L{tdir / 'lib'}",
@@ -81,7 +83,6 @@ def build(verbose: bool = False) -> Path:
     with cf.ThreadPoolExecutor(jobs) as ex:
         host = ex.submit(_build_host)
         objs = list(ex.map(_compile, srcs))
-        host.result()
     out = lib_path()
     tmp = out.with_suffix(".so.tmp")
     cmd = [_hipcc(), f"--offload-arch={ARCH}", "-shared", "-fPIC", *map(str, objs), "-o", str(tmp)]
@@ -89,6 +90,7 @@ def build(verbose: bool = False) -> Path:
     if r.returncode != 0:
         raise RuntimeError(f"link failed:\n{r.stderr[-4000:]}")
     os.replace(tmp, out)
+    host.result()  # after the link: the kernel library serves without the extension too
     if verbose:
         print(f"built {out}")
     return out

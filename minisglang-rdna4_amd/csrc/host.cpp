@@ -371,4 +371,11 @@ PyModuleDef module_def = {PyModuleDef_HEAD_INIT, "w4a8_host", nullptr, -1, metho
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit_w4a8_host() { return PyModule_Create(&module_def); }
+PyMODINIT_FUNC PyInit_w4a8_host() {
+  PyObject* m = PyModule_Create(&module_def);
+  if (m && PyModule_AddStringConstant(m, "built_for", W4A8_BUILT_FOR) < 0) {
+    Py_DECREF(m);
+    return nullptr;
+  }
+  return m;
+}

@@ -2,6 +2,7 @@
 same tensors, bit for bit, or the same refusal, whichever of the two serves it. The CPU part checks that
 it takes no CPU tensors and that its table of entry points is the C ABI's."""
 import re
+import warnings
 from pathlib import Path
 
 import pytest
@@ -30,6 +31,30 @@ def test_cpu_tensors_and_wrong_counts_are_left_alone():
     for f in (m.linear, m.rms_norm, m.moe, m.bind):
         with pytest.raises(TypeError):
             f(x)
+
+
+@pytest.mark.parametrize("why", ["missing", "another torch", "not a library"])
+def test_python_path_serves_without_the_extension(monkeypatch, tmp_path, why):
+    """One warning, then a stand-in that takes no call (the GPU tests below run every form on it)."""
+    host = pkg("_host")
+    monkeypatch.setattr(host, "_mod", None)
+    if why == "missing":
+        monkeypatch.setattr(host, "_PATH", tmp_path / "w4a8_host.so")
+    elif why == "another torch":
+        monkeypatch.setattr(host, "_running", lambda: "torch 1.0, Python 3.10")
+    else:
+        (tmp_path / "w4a8_host.so").write_bytes(b"not a library")
+        monkeypatch.setattr(host, "_PATH", tmp_path / "w4a8_host.so")
+    with pytest.warns(RuntimeWarning, match="Python host path"):
+        m = host.load()
+    with warnings.catch_warnings():
+        warnings.simplefilter("error")
+        assert host.load() is m
+    assert m.linear(*range(10)) is None and m.rms_norm(*range(6)) is None and m.moe(*range(16)) is None
+
+
+def test_the_built_extension_is_for_this_torch():
+    assert pkg("_host")._extension().built_for == pkg("_host")._running()
 
 
 class _Off:
