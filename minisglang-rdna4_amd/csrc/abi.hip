@@ -114,6 +114,8 @@ static bool dma_tiled_ok(const GemmArgs& p, int64_t min_n, int64_t min_rows) {
   return min_rows > 0 && p.M >= min_rows && p.N >= min_n && (int4 || mx) && p.K % 128 == 0 && p.KT >= 3 && !(p.silu && (p.N / 16) % 2) &&
          p.N * p.KT * 64 < ((int64_t)1 << 31) && p.M * p.K < ((int64_t)1 << 31);
 }
+// the other formats' operand-order GEMMs read no row-sum seeds
+static bool needs_seeds(const GemmArgs& p) { return p.wfmt == kInt4 && !p.zeros; }
 static bool dma_tiled_ok(const GemmArgs& p) { return dma_tiled_ok(p, 16384, tiled_min_rows()); }
 
 // w4a8_linear's own calls, whose quant is one launch in either layout, take it below that too:
@@ -304,7 +306,7 @@ int w4a8_gemm(const uint8_t* x_fp8, int64_t ldx, const float* act_scales, int64_
     const int64_t Mp = (M + 15) / 16 * 16;
     uint8_t* xt = reinterpret_cast<uint8_t*>(workspace);
     float* seeds = reinterpret_cast<float*>(xt + round256(Mp * K));
-    rc = launch_act_tile(x_fp8, ldx, M, K, xt, seeds, Mp, st);
+    rc = launch_act_tile(x_fp8, ldx, M, K, xt, needs_seeds(p) ? seeds : nullptr, Mp, st);
     if (rc) return hip_status(rc, "w4a8_gemm(act tile)");
     GemmArgs q = p;
     q.xq = xt; q.ldx = K; q.a_tiled = 1; q.seeds = seeds; q.seeds_ld = Mp;
@@ -348,7 +350,7 @@ int w4a8_linear(const void* x, int x_dtype, int64_t M, int64_t K, int64_t ldx, c
     const int64_t Mp = (M + 15) / 16 * 16;
     uint8_t* xt = reinterpret_cast<uint8_t*>(xs) + round256(M * 4);
     float* seeds = reinterpret_cast<float*>(xt + round256(Mp * K));
-    rc = launch_act_quant_tiled(x, x_dtype, M, K, ldx, xt, xs, wfmt == kInt4 && !zeros ? seeds : nullptr, Mp, nullptr, st);
+    rc = launch_act_quant_tiled(x, x_dtype, M, K, ldx, xt, xs, needs_seeds(p) ? seeds : nullptr, Mp, nullptr, st);
     if (rc) return hip_status(rc, "w4a8_linear(act quant, tiled)");
     GemmArgs q = p;
     q.xsrc = nullptr;
@@ -473,7 +475,7 @@ int w4a16_linear(const void* x, int x_dtype, int64_t M, int64_t K, int64_t ldx, 
       uint8_t* xt = reinterpret_cast<uint8_t*>(y);
       float* seeds = reinterpret_cast<float*>(xt + round256(Mp * K));
       if (round256(Mp * K) + round256(KT * Mp * 4) <= round256(T * M * N * 4)) {
-        rc = launch_act_tile(xq, ldq, q.M, K, xt, seeds, Mp, st);
+        rc = launch_act_tile(xq, ldq, q.M, K, xt, needs_seeds(q) ? seeds : nullptr, Mp, st);
         if (rc) return hip_status(rc, "w4a16_linear(act tile)");
         q.xq = xt; q.ldx = K; q.a_tiled = 1; q.seeds = seeds; q.seeds_ld = Mp;
       }

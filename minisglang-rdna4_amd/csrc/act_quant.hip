@@ -51,7 +51,8 @@ act_quant_wave_kernel(const uint16_t* __restrict__ x, int64_t ldx, int64_t M, in
 // 16-row block and 128-wide K tile one 2 KiB block at ((row / 16) * KT + kt) * 2048 whose two 1 KiB
 // halves hold, at lane l * 16, row (l & 15)'s bytes [16 (l >> 4), +16) and [64 + 16 (l >> 4), +16) of
 // the tile -- what the GEMM's operand read gives lane l, so its LDS-DMA copies whole 1 KiB runs
-// instead of 64-byte pieces of 16 rows. With them, per block and K tile, the GEMM's row-sum seed (the
+// instead of 64-byte pieces of 16 rows. With them, unless seeds is null (only symmetric int4 reads
+// them), per block and K tile, the GEMM's row-sum seed (the
 // e4m3 -0.5 splat MFMA on that operand: the same instruction on the same bytes, so the same bits) at
 // seeds[kt * seeds_ld + row], seeds_ld = M rounded up to 16. Rows past M in the last block are zero
 // codes. One wave per (block, 4 K tiles), four per workgroup; every lane active at the MFMA.
@@ -89,6 +90,7 @@ act_tile_kernel(const uint8_t* __restrict__ q, int64_t ldq, int64_t M, int KT, u
       uint8_t* dst = qt + (blk * KT + kt0 + t) * 2048 + lane * 16;
       *reinterpret_cast<uint4*>(dst) = h0;
       *reinterpret_cast<uint4*>(dst + 1024) = h1;
+      if (!seeds) continue;
       v8i a;
       a[0] = (int)h0.x; a[1] = (int)h0.y; a[2] = (int)h0.z; a[3] = (int)h0.w;
       a[4] = (int)h1.x; a[5] = (int)h1.y; a[6] = (int)h1.z; a[7] = (int)h1.w;

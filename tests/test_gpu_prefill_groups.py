@@ -172,3 +172,29 @@ def test_few_rows_in_operand_order(kernels, dev, fmt, M, N, K):
     ref = _row_major_gemm(q, sc, tiles, sd, zd, g, N, K, e2, x.dtype)
     torch.cuda.synchronize()
     assert torch.equal(out, ref)
+
+
+@pytest.mark.parametrize("fmt", ["sym", "asym", "mxfp4"])
+@pytest.mark.parametrize("M,K", [(1024, 384), (1037, 640)])
+def test_pair_rewrite_computes_seeds_where_they_are_read(kernels, dev, fmt, M, K):
+    """The producer pair's codes rewritten in operand order: the workspace's row-sum seeds are written for
+    symmetric int4 and left alone for the formats that read none; the outputs are the row-major GEMM's."""
+    N, g = 16384, 32 if fmt == "mxfp4" else 128
+    abi = pkg("_abi")
+    lib = abi.load()
+    w, s, z, e2, _ = _weight(fmt, 128, N, K, seed=M + K)
+    tiles, sd, zd = kernels.repack_w4(w.to(dev), e2), s.to(dev), None if z is None else z.to(dev)
+    x = synth.activations(M, K, seed=M).to(dev)
+    q, sc = kernels.act_quant(x)
+    wsb = lib.w4a8_gemm_workspace_bytes(M, N, K, abi.KERNEL_PREFILL)
+    ws = torch.full((wsb,), 0xA5, dtype=torch.uint8, device=dev)
+    out = torch.empty((M, N), dtype=x.dtype, device=dev)
+    abi.check(lib.w4a8_gemm(abi.ptr(q), K, abi.ptr(sc), M, abi.ptr(tiles), N, K, abi.ptr(sd),
+                            abi.SCALE_E8M0 if e2 else abi.SCALE_F16, abi.ptr(zd), abi.W_E2M1 if e2 else abi.W_INT4, g,
+                            abi.ptr(out), abi.BF16, N, 0, abi.ptr(ws), wsb, abi.KERNEL_PREFILL, abi.stream_of(x)), "w4a8_gemm")
+    ref = _row_major_gemm(q, sc, tiles, sd, zd, g, N, K, e2, x.dtype)
+    torch.cuda.synchronize()
+    assert torch.equal(out, ref)
+    Mp = (M + 15) // 16 * 16
+    seeds = ws[(Mp * K + 255) // 256 * 256:][:K // 128 * Mp * 4]
+    assert not bool((ws[:Mp * K] == 0xA5).all()) and bool((seeds == 0xA5).all()) == (fmt != "sym")
