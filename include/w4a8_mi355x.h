@@ -86,15 +86,21 @@ int w4a8_gemm(const uint8_t* x_fp8, int64_t ldx, const float* act_scales, int64_
               void* out, int out_dtype, int64_t ldo, int silu, void* workspace, int64_t workspace_bytes, int kernel,
               void* stream);
 
-/* Workspace bytes w4a8_linear may need for M rows of K inputs (the fp8 codes and scales of x when
- * they are not produced inside the GEMM kernel; for prefill calls of 128 rows or more, also the
- * codes again in the GEMM's operand order with one row-sum seed per row and 128 inputs, which int4
- * (groups of 128+) and MXFP4 weights of 2048+ output channels use from 1024 rows on, and below that
- * where it was measured to pay, x quantized straight into it);
+/* Workspace bytes w4a8_linear may need for M rows of K inputs, whatever the weight (the fp8 codes and
+ * scales of x when they are not produced inside the GEMM kernel; for prefill calls of 1024 rows or more,
+ * also the codes again in the GEMM's operand order with one row-sum seed per row and 128 inputs, which
+ * int4 (groups of 128+) and MXFP4 weights of 2048+ output channels use, x quantized straight into it);
  * -1 on bad sizes. w4a8_linear also accepts a workspace of just the codes and scales (M * K and
  * 4 * M bytes, each rounded up to 256): such calls run the GEMM on the row-major codes, with the
  * same outputs. */
 int64_t w4a8_linear_workspace_bytes(int64_t M, int64_t K);
+
+/* The same for one call's weight, fused arm and kernel choice (0 auto, 1 decode, 2 prefill): the codes and
+ * scales, and room for the operand order only where the call takes it, which some calls of 128 to 1023 rows
+ * do too (where it was measured to pay; with the bytes above they run on row-major codes). has_zeros: the
+ * zeros slot is given. -1 on arguments that w4a8_linear refuses. */
+int64_t w4a8_linear_workspace_bytes_for(int64_t M, int64_t N, int64_t K, int scale_fmt, int has_zeros, int wfmt,
+                                        int64_t group_size, int silu, int kernel);
 
 /* Dense W4A8 linear on bf16/fp16 activations x (M, ldx): per-token fp8 quant of x, then the GEMM of
  * w4a8_gemm, with the same outputs bit for bit as w4a8_act_quant followed by w4a8_gemm. This is
@@ -103,7 +109,7 @@ int64_t w4a8_linear_workspace_bytes(int64_t M, int64_t K);
  * rows the GEMV can quantize itself (int4 with groups of 128+ and MXFP4, up to 64 values per thread
  * of its row phase, 128 on weights of over 64 KiB per workgroup: at K = 4096 up to 8 rows, 16 on
  * the wide gate_up shape; see w4a8_linear_launch_count) are a single launch; otherwise one act-quant
- * launch writes the workspace (w4a8_linear_workspace_bytes, 16-byte aligned) first. */
+ * launch writes the workspace (w4a8_linear_workspace_bytes or _for, 16-byte aligned) first. */
 int w4a8_linear(const void* x, int x_dtype, int64_t M, int64_t K, int64_t ldx, const void* w_tile, int64_t N,
                 const void* scales, int scale_fmt, const int32_t* zeros, int wfmt, int64_t group_size, void* out,
                 int out_dtype, int64_t ldo, int silu, void* workspace, int64_t workspace_bytes, int kernel,

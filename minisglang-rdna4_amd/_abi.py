@@ -36,6 +36,8 @@ SIGNATURES = {
     "w4a8_gemm": (_c_int, [_vp, _c_i64, _vp, _c_i64, _vp, _c_i64, _c_i64, _vp, _c_int, _vp, _c_int, _c_i64,
                            _vp, _c_int, _c_i64, _c_int, _vp, _c_i64, _c_int, _vp]),
     "w4a8_linear_workspace_bytes": (_c_i64, [_c_i64, _c_i64]),
+    "w4a8_linear_workspace_bytes_for": (_c_i64, [_c_i64, _c_i64, _c_i64, _c_int, _c_int, _c_int, _c_i64, _c_int,
+                                                 _c_int]),
     "w4a8_linear": (_c_int, [_vp, _c_int, _c_i64, _c_i64, _c_i64, _vp, _c_i64, _vp, _c_int, _vp, _c_int, _c_i64,
                              _vp, _c_int, _c_i64, _c_int, _vp, _c_i64, _c_int, _vp]),
     # measurement probe (include/w4a8_probe.h), not part of the W4A8 path

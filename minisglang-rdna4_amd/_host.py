@@ -20,7 +20,7 @@ _PATH = Path(__file__).resolve().parent / "_lib" / "w4a8_host.so"
 
 # the members of host.cpp's Abi, in their order
 _ENTRY_POINTS = (
-    "w4a8_last_error", "w4a8_linear", "w4a8_linear_workspace_bytes", "w4a8_gemm", "w4a8_gemm_workspace_bytes",
+    "w4a8_last_error", "w4a8_linear", "w4a8_linear_workspace_bytes_for", "w4a8_gemm", "w4a8_gemm_workspace_bytes",
     "w4a8_rms_norm", "w4a8_moe_padded_capacity", "w4a8_moe_route_gemm1", "w4a8_moe_route_slots",
     "w4a8_moe_route_align", "w4a8_moe_gemm_workspace_bytes", "w4a8_moe_gemm", "w4a8_moe_gemm2_combine_supported",
     "w4a8_moe_gemm2_combine", "w4a8_moe_gemm_quant_workspace_bytes", "w4a8_moe_gemm_quant", "w4a8_moe_combine",

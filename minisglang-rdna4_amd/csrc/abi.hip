@@ -101,6 +101,7 @@ static int64_t tiled_min_rows() {
   }();
   return min_rows;
 }
+static bool tiled_rows(int64_t M) { return tiled_min_rows() > 0 && M >= tiled_min_rows(); }
 static int64_t tiled_min_n() {
   static const int64_t n = [] {
     const char* e = getenv("W4A8_PREFILL_TILED_N");
@@ -173,13 +174,12 @@ static int check_weights(const char* who, int64_t N, int64_t K, int scale_fmt, c
 }
 
 // w4a8_linear's workspace: the row-major codes and scales of x (what every call needs), then for
-// the calls that may take the tiled prefill (linear_tiled_min_rows) the codes of whole 16-row blocks in
+// the calls that take the tiled prefill (linear_tiled_ok) the codes of whole 16-row blocks in
 // the GEMM's operand order and one row-sum seed per row and K tile. A workspace of only the first
 // part is accepted; such calls run the row-major GEMM, with the same results.
 static int64_t round256(int64_t b);
 static int64_t linear_ws_rowmajor(int64_t M, int64_t K) { return round256(M * K) + round256(M * 4); }
-static int64_t linear_ws_tiled(int64_t M, int64_t K, int64_t min_rows) {
-  if (min_rows <= 0 || M < min_rows) return 0;
+static int64_t linear_ws_tiled(int64_t M, int64_t K) {
   const int64_t Mp = (M + 15) / 16 * 16, KT = (K + 127) / 128;
   return round256(Mp * K) + round256(KT * Mp * 4);
 }
@@ -241,7 +241,7 @@ int64_t w4a8_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int kernel) {
   if (M < 0 || N <= 0 || K <= 0) return -1;
   // prefill: room for the codes rewritten in the GEMM's operand order with their row-sum seeds,
   // which wide int4 and MXFP4 weights take (the call runs without it too, on the row-major codes)
-  if (kernel == 2 || (kernel == 0 && M > kGemvMaxRows)) return N >= 16384 ? linear_ws_tiled(M, K, tiled_min_rows()) : 0;
+  if (kernel == 2 || (kernel == 0 && M > kGemvMaxRows)) return N >= 16384 && tiled_rows(M) ? linear_ws_tiled(M, K) : 0;
   return (int64_t)gemv_workspace_bytes(M, N, K, 0, (M + 15) / 16);
 }
 
@@ -301,7 +301,7 @@ int w4a8_gemm(const uint8_t* x_fp8, int64_t ldx, const float* act_scales, int64_
   p.xq = x_fp8; p.ldx = ldx; p.act_scales = act_scales;
   const hipStream_t st = (hipStream_t)stream;
   const bool decode = kernel == 1 || (kernel == 0 && M <= kGemvMaxRows);
-  if (!decode && dma_tiled_ok(p) && workspace && aligned16(workspace) && workspace_bytes >= linear_ws_tiled(M, K, tiled_min_rows())) {
+  if (!decode && dma_tiled_ok(p) && workspace && aligned16(workspace) && workspace_bytes >= linear_ws_tiled(M, K)) {
     // the caller's codes rewritten in the GEMM's operand order with their seeds (as w4a8_linear)
     const int64_t Mp = (M + 15) / 16 * 16;
     uint8_t* xt = reinterpret_cast<uint8_t*>(workspace);
@@ -318,7 +318,20 @@ int w4a8_gemm(const uint8_t* x_fp8, int64_t ldx, const float* act_scales, int64_
 
 int64_t w4a8_linear_workspace_bytes(int64_t M, int64_t K) {
   if (M < 0 || K <= 0) return -1;
-  return linear_ws_rowmajor(M, K) + linear_ws_tiled(M, K, linear_tiled_min_rows());
+  return linear_ws_rowmajor(M, K) + (tiled_rows(M) ? linear_ws_tiled(M, K) : 0);
+}
+
+int64_t w4a8_linear_workspace_bytes_for(int64_t M, int64_t N, int64_t K, int scale_fmt, int has_zeros, int wfmt,
+                                        int64_t group_size, int silu, int kernel) {
+  // shapes and formats only: stand-in pointers (aligned, never dereferenced)
+  const void* fake = reinterpret_cast<const void*>(static_cast<uintptr_t>(256));
+  GemmArgs p;
+  if (dense_args("w4a8_linear_workspace_bytes_for", M, fake, N, K, fake, scale_fmt,
+                 has_zeros ? reinterpret_cast<const int32_t*>(fake) : nullptr, wfmt, group_size,
+                 const_cast<void*>(fake), kBF16, N, silu, kernel, p))
+    return -1;
+  const bool decode = kernel == 1 || (kernel == 0 && M <= kGemvMaxRows);
+  return linear_ws_rowmajor(M, K) + (!decode && linear_tiled_ok(p) ? linear_ws_tiled(M, K) : 0);
 }
 
 int w4a8_linear(const void* x, int x_dtype, int64_t M, int64_t K, int64_t ldx, const void* w_tile, int64_t N,
@@ -345,7 +358,7 @@ int w4a8_linear(const void* x, int x_dtype, int64_t M, int64_t K, int64_t ldx, c
                 (long long)workspace_bytes);
   uint8_t* xq = reinterpret_cast<uint8_t*>(workspace);
   float* xs = reinterpret_cast<float*>(xq + round256(M * K));
-  if (!decode && linear_tiled_ok(p) && workspace_bytes >= need + linear_ws_tiled(M, K, linear_tiled_min_rows())) {
+  if (!decode && linear_tiled_ok(p) && workspace_bytes >= need + linear_ws_tiled(M, K)) {
     // prefill on the DMA-staged kernel: x quantized straight into its operand order, with the seeds
     const int64_t Mp = (M + 15) / 16 * 16;
     uint8_t* xt = reinterpret_cast<uint8_t*>(xs) + round256(M * 4);

@@ -35,7 +35,7 @@ constexpr int kUnsupported = 2;  // the C ABI's status for a call it leaves to a
 struct Abi {
   decltype(&w4a8_last_error) last_error;
   decltype(&w4a8_linear) linear;
-  decltype(&w4a8_linear_workspace_bytes) linear_ws;
+  decltype(&w4a8_linear_workspace_bytes_for) linear_ws;
   decltype(&w4a8_gemm) gemm;
   decltype(&w4a8_gemm_workspace_bytes) gemm_ws;
   decltype(&w4a8_rms_norm) rms_norm;
@@ -167,13 +167,13 @@ PyObject* linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
     }
     const int64_t nout = silu ? N / 2 : N;
     at::Tensor out = empty(*x, {M, nout}, x->scalar_type());
-    const int64_t wsb = xq ? abi.gemm_ws(M, N, K, arm) : abi.linear_ws(M, K);
+    const int wfmt = e2m1 ? 1 : 0;
+    const int64_t wsb = xq ? abi.gemm_ws(M, N, K, arm) : abi.linear_ws(M, N, K, sfmt, z != nullptr, wfmt, group, silu, arm);
     at::Tensor ws;
     if (wsb > 0) ws = empty(*x, {wsb}, at::kByte);
     void* wp = ws.defined() ? ws.data_ptr() : nullptr;
     const int32_t* zp = z ? static_cast<const int32_t*>(z->data_ptr()) : nullptr;
     void* st = stream_of(*x);
-    const int wfmt = e2m1 ? 1 : 0;
     const int rc = unlocked([&] {
       return xq ? abi.gemm(static_cast<const uint8_t*>(xq->data_ptr()), K, static_cast<const float*>(xs->data_ptr()), M,
                            w->data_ptr(), N, K, s->data_ptr(), sfmt, zp, wfmt, group, out.data_ptr(), dt, nout, silu, wp,

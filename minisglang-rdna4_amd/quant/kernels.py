@@ -319,7 +319,8 @@ def _dense(x, w_packed, scales, w_zeros, group_size, weight_is_e2m1, x_fp8, act_
         # the op quantizes x itself: in the decode kernel's prologue when the rows fit, else with
         # one act-quant launch into the workspace
         x = x.contiguous()
-        ws_bytes = int(lib.w4a8_linear_workspace_bytes(M, K))
+        ws_bytes = int(lib.w4a8_linear_workspace_bytes_for(M, N, K, sfmt, int(w_zeros is not None), wfmt, group_size,
+                                                           int(silu), arm))
         ws = torch.empty((max(ws_bytes, 1),), dtype=torch.uint8, device=x.device)
         _abi.check(
             lib.w4a8_linear(_abi.ptr(x), _abi.dtype_code(x.dtype), M, K, K, _abi.ptr(tiles), N, _abi.ptr(sc),

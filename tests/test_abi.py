@@ -110,6 +110,38 @@ def test_host_validation_rejects_before_launch(lib):
     assert rc == 1 and b"slots" in lib.w4a8_last_error()
 
 
+def _operand_order(lib, M, N, K, fmt, group=128, silu=0, kernel=2):
+    """Whether w4a8_linear's call is sized for (and so takes) activations in operand order."""
+    sfmt, zeros, wfmt = {"sym": (0, 0, 0), "asym": (0, 1, 0), "mxfp4": (1, 0, 1), "nvfp4": (2, 1, 1)}[fmt]
+    row_major = (M * K + 255) // 256 * 256 + (M * 4 + 255) // 256 * 256
+    got = lib.w4a8_linear_workspace_bytes_for(M, N, K, sfmt, zeros, wfmt, group, silu, kernel)
+    Mp = (M + 15) // 16 * 16
+    tiled = (Mp * K + 255) // 256 * 256 + (K // 128 * Mp * 4 + 255) // 256 * 256
+    assert got in (row_major, row_major + tiled), (M, N, K, fmt, got)
+    return got > row_major
+
+
+@pytest.mark.parametrize("M", [1, 16, 17, 128, 512, 1023, 1024, 4000])
+def test_linear_workspace_is_sized_for_the_call(lib, M):
+    """Only calls that take the operand order ask for its room: none of NVFP4, groups of 32 and 64, narrow
+    weights, a K that is no multiple of 128 or the decode kernels; and the weight-blind size asks for it from
+    1024 rows."""
+    for N, K in ((2048, 4096), (28672, 4096), (4096, 14336)):
+        for fmt, g in (("nvfp4", 16), ("sym", 32), ("sym", 64), ("asym", 32), ("asym", 64)):
+            assert not _operand_order(lib, M, N, K, fmt, g)
+    for fmt, g in (("sym", 128), ("asym", 128), ("mxfp4", 32)):
+        assert not _operand_order(lib, M, 2032, 4096, fmt, g) and not _operand_order(lib, M, 28672, 256, fmt, g)
+        assert not _operand_order(lib, M, 28672, 4096, fmt, g, kernel=1)
+        assert _operand_order(lib, M, 28672, 4096, fmt, g, kernel=0) == _operand_order(lib, M, 28672, 4096, fmt, g) or M <= 16
+        if M >= 1024:
+            assert _operand_order(lib, M, 2048, 4096, fmt, g)
+    assert not _operand_order(lib, M, 28672, 4096 + 32, "mxfp4", 32)
+    K = 4096
+    row_major = (M * K + 255) // 256 * 256 + (M * 4 + 255) // 256 * 256
+    assert (lib.w4a8_linear_workspace_bytes(M, K) > row_major) == (M >= 1024)
+    assert lib.w4a8_linear_workspace_bytes_for(M, 24, K, 0, 0, 0, 128, 0, 2) == -1
+
+
 # ------------------------------------------------------------------------ provider refusals
 def _dense_args(M=4, K=256, N=64, g=128):
     x = torch.randn(M, K).to(torch.bfloat16)
