@@ -24,7 +24,7 @@ size_t gemv_workspace_bytes(int64_t M, int64_t N, int64_t K, int grouped, int64_
 int launch_prefill(const GemmArgs& p, int64_t rows_to_cover, int bm_rows, hipStream_t stream);
 int launch_prefill_staged(const GemmArgs& p, int64_t rows_to_cover, int bm_rows, hipStream_t stream);
 int launch_prefill_dma(const GemmArgs& p, int64_t rows_to_cover, int bm_rows, hipStream_t stream);
-bool prefill_takes_wide(const GemmArgs& p);
+DmaTile prefill_tile_tiled(const GemmArgs& p);
 int launch_moe_route(const void* logits, int dtype, int64_t T, int E, int top_k, int renorm, float* tw,
                      int32_t* ids, hipStream_t stream);
 int launch_moe_align(const int32_t* ids, int64_t numel, int E, int bm, int64_t P, int32_t* sorted_ids,
@@ -124,10 +124,15 @@ static bool dma_tiled_ok(const GemmArgs& p) { return dma_tiled_ok(p, 16384, tile
 //    rows and up only -> this: K=4096 N=28672 M=512 86 -> 72 and M=448 52.0 -> 45.7, K=8192 N=14336 M=900
 //    93 -> 77, AWQ K=4096 N=14336 M=1000 51.0 -> 45.5. On the smaller tiles it loses: K=14336 N=4096 M=512
 //    62 -> 78 (two quant passes over few rows), K=4096 N=6144 M=512 32 -> 34, N=14336 M=129 28 -> 31;
-//  - MXFP4 up to K=32768: K=14336 N=4096 M=200 23.7 -> 18.4 and M=700 44.1 -> 32.1, K=8192 N=8192 M=700
-//    37.1 -> 29.5, K=4096 N=14336 M=200 16.1 -> 13.9 (M=400 20.1 -> 20.4), K=8192 N=28672 M=200 to 1000
-//    within 3%; K=28672 N=8192 M=130 88.7 -> 81.0, M=400 136 -> 115, M=1000 189 -> 194, K=24576 N=4096
-//    M=130 60.6 -> 48.0. Longer rows take the two-pass quant, which lost at few rows (M=130 88.7 -> 108).
+//  - MXFP4 up to K=32768 on tiles of 64 and 128 columns, whose row-major DMA takes the most pieces per
+//    output. us, row-major -> this, both in one run: K=14336 N=4096 M=200 39.8 -> 30.6 and M=640 74.0 ->
+//    53.2, K=8192 N=8192 M=640 61.0 -> 47.6, K=4096 N=14336 M=200 26.9 -> 23.3, K=28672 N=8192 M=128 70.2
+//    -> 55.8 and M=768 188.9 -> 147.5, K=2048 N=6144 M=640 18.5 -> 16.4; at worst K=1024 N=4096 M=200 11.2
+//    -> 11.4. Longer rows take the two-pass quant, which lost at few rows (M=130 88.7 -> 108);
+//  - MXFP4 on 256-column tiles where the quant in that order costs no more than the row-major one: K=8192
+//    N=28672 M=640 139.4 -> 136.0, K=6144 N=28672 M=900 140.2 -> 133.1, K=2048 N=28672 M=640 48.2 -> 47.0.
+//    It does for rows of 2049 to 4096 elements up to 512 rows (K=4096 N=28672 M=200 32.9 -> 33.8, N=14336
+//    M=400 33.3 -> 34.0) and from K=16384 on (N=8192 M=1000 109.1 -> 111.3, K=28672 185.3 -> 190.2).
 // Below 128 rows nothing was measured to gain.
 static const int64_t kTiledFewRows = 128;
 static int64_t linear_tiled_min_rows() {
@@ -136,7 +141,10 @@ static int64_t linear_tiled_min_rows() {
 }
 static bool linear_tiled_ok(const GemmArgs& p) {
   if (p.M >= tiled_min_rows()) return dma_tiled_ok(p, tiled_min_n(), tiled_min_rows());
-  return dma_tiled_ok(p, tiled_min_n(), linear_tiled_min_rows()) && (p.wfmt == kE2M1 ? p.K <= 32768 : prefill_takes_wide(p));
+  if (!dma_tiled_ok(p, tiled_min_n(), linear_tiled_min_rows())) return false;
+  const bool wide = prefill_tile_tiled(p).bn == 256;
+  if (p.wfmt != kE2M1) return wide;
+  return wide ? p.K <= 14336 && (p.M > 512 || p.K <= 2048 || p.K > 4096) : p.K <= 32768;
 }
 
 // Bound on align blocks that can hold routed rows: every expert with rows contributes

@@ -70,4 +70,11 @@ struct GemmArgs {
   int64_t kps;        // tiles per split
 };
 
+// A dense prefill tile shape and what one K step of a full round of its workgroups (one per CU) costs,
+// relative to the others of its format (pick_tile, prefill.h).
+struct DmaTile {
+  int bm, bn;
+  float cost;
+};
+
 }  // namespace w4a8

@@ -660,8 +660,10 @@ static const DmaTile kInt4TiledA[] = {{256, 128, 1.0f}, {192, 128, 0.81f}, {128,
 static const DmaTile kMxTiles[] = {{256, 256, 1.0f}, {192, 256, 0.80f}, {128, 256, 0.60f}, {192, 128, 0.50f},
                                    {128, 128, 0.45f}, {64, 128, 0.33f}, {64, 64, 0.29f}};
 
-// whether a dense int4 call (groups of 128+) runs on 256 x 256 tiles given its activations in operand order
-bool prefill_takes_wide(const GemmArgs& p) { return kInt4TiledA[pick_tile(kInt4TiledA, p, p.M)].bn == 256; }
+// the tile of a dense int4 (groups of 128+) or MXFP4 call given its activations in operand order
+DmaTile prefill_tile_tiled(const GemmArgs& p) {
+  return p.wfmt == kE2M1 ? kMxTiles[pick_tile(kMxTiles, p, p.M)] : kInt4TiledA[pick_tile(kInt4TiledA, p, p.M)];
+}
 
 // int4 with groups of 32, 64 and 128+ and MXFP4, on 16-byte aligned rows; kErrUnsupported otherwise.
 // bm_rows: rows per workgroup the caller requires (grouped: 64 or 128; 0 for dense).

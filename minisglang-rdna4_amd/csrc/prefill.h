@@ -349,12 +349,6 @@ __device__ __forceinline__ void store_tile(const GemmArgs& p, const v4f (&acc)[R
   store_tile_scaled(p, acc, sc, valid, row0, lane, strip, scr);
 }
 
-// A dense tile shape and what one K step of a full round of its workgroups (one per CU) costs, relative
-// to the others of its format.
-struct DmaTile {
-  int bm, bn;
-  float cost;
-};
 // The tile whose rounds of the grid take least. Up to six rounds a partial round counts as a whole one
 // (M=1777 K=2560 N=9728 int4: 532 workgroups of 256 x 128, 2.08 rounds, 81.5 us; 760 of 192 x 128, 2.97
 // rounds, 74.0); over more rounds the workgroups drift apart and half of the partial one is charged.

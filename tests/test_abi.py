@@ -142,6 +142,23 @@ def test_linear_workspace_is_sized_for_the_call(lib, M):
     assert lib.w4a8_linear_workspace_bytes_for(M, 24, K, 0, 0, 0, 128, 0, 2) == -1
 
 
+# both sides of the few-row rule's lines, by the tile that a call's grid takes (its columns) and K
+@pytest.mark.parametrize("fmt,M,N,K,takes", [
+    ("mxfp4", 127, 4096, 14336, False), ("mxfp4", 128, 4096, 14336, True),
+    ("mxfp4", 640, 8192, 8192, True), ("mxfp4", 768, 8192, 28672, True), ("mxfp4", 400, 2048, 32768, True),
+    ("mxfp4", 400, 2048, 32896, False),  # the two-pass quant
+    # 256-column tiles
+    ("mxfp4", 900, 8192, 14336, True), ("mxfp4", 900, 8192, 14464, False), ("mxfp4", 1000, 8192, 28672, False),
+    ("mxfp4", 200, 28672, 4096, False), ("mxfp4", 200, 28672, 4224, True), ("mxfp4", 512, 28672, 4096, False),
+    ("mxfp4", 513, 28672, 4096, True), ("mxfp4", 400, 28672, 2048, True), ("mxfp4", 200, 28672, 2176, False),
+    ("mxfp4", 1024, 8192, 28672, True),
+    # int4: the 256 x 256 tile
+    ("sym", 512, 28672, 4096, True), ("sym", 512, 4096, 14336, False), ("sym", 512, 6144, 4096, False),
+    ("asym", 1000, 14336, 4096, True), ("asym", 129, 14336, 4096, False), ("sym", 1024, 6144, 4096, True)])
+def test_operand_order_rule(lib, fmt, M, N, K, takes):
+    assert _operand_order(lib, M, N, K, fmt, 32 if fmt == "mxfp4" else 128) == takes
+
+
 # ------------------------------------------------------------------------ provider refusals
 def _dense_args(M=4, K=256, N=64, g=128):
     x = torch.randn(M, K).to(torch.bfloat16)
