@@ -117,7 +117,12 @@ static bool dma_tiled_ok(const GemmArgs& p, int64_t min_n, int64_t min_rows) {
 }
 // the other formats' operand-order GEMMs read no row-sum seeds
 static bool needs_seeds(const GemmArgs& p) { return p.wfmt == kInt4 && !p.zeros; }
-static bool dma_tiled_ok(const GemmArgs& p) { return dma_tiled_ok(p, 16384, tiled_min_rows()); }
+// the producer pair's calls. With zero points the row-major kernel has no row sums to save, so the rewrite
+// pays through the 256 x 256 tile only (AWQ K=8192 N=28672 M=1500 446 -> 375 us; on the other tiles K=4096
+// N=16384 M=1500 121.9 -> 124.5)
+static bool dma_tiled_ok(const GemmArgs& p) {
+  return dma_tiled_ok(p, 16384, tiled_min_rows()) && (!p.zeros || prefill_tile_tiled(p).bn == 256);
+}
 
 // w4a8_linear's own calls, whose quant is one launch in either layout, take it below that too:
 //  - int4 where the 256 x 256 tile is the cheapest of its grid (it takes operand order only). us, 1024
@@ -133,14 +138,19 @@ static bool dma_tiled_ok(const GemmArgs& p) { return dma_tiled_ok(p, 16384, tile
 //    N=28672 M=640 139.4 -> 136.0, K=6144 N=28672 M=900 140.2 -> 133.1, K=2048 N=28672 M=640 48.2 -> 47.0.
 //    It does for rows of 2049 to 4096 elements up to 512 rows (K=4096 N=28672 M=200 32.9 -> 33.8, N=14336
 //    M=400 33.3 -> 34.0) and from K=16384 on (N=8192 M=1000 109.1 -> 111.3, K=28672 185.3 -> 190.2).
-// Below 128 rows nothing was measured to gain.
+// Below 128 rows nothing was measured to gain. From 1024 rows on, int4 with zero points (no row sums to save)
+// takes it on the 256 x 256 tile, and on the others up to K = 4096 where the GEMM is two rounds of the grid or
+// more: AWQ K=2560 N=9728 M=1777 76.4 -> 74.3 us, K=4096 N=6144 M=3000 111.9 -> 109.9, but M=1024 48.0 ->
+// 49.0, K=4096 N=4096 M=1500 42.9 -> 44.3, K=14336 N=4096 M=1200 113.7 -> 122.9, K=28672 M=1200 217 -> 251.
 static const int64_t kTiledFewRows = 128;
 static int64_t linear_tiled_min_rows() {
   const int64_t n = tiled_min_rows();
   return n < kTiledFewRows ? n : kTiledFewRows;
 }
 static bool linear_tiled_ok(const GemmArgs& p) {
-  if (p.M >= tiled_min_rows()) return dma_tiled_ok(p, tiled_min_n(), tiled_min_rows());
+  if (p.M >= tiled_min_rows())
+    return dma_tiled_ok(p, tiled_min_n(), tiled_min_rows()) &&
+           (!p.zeros || prefill_tile_tiled(p).bn == 256 || (p.K <= 4096 && p.M * p.N >= 1 << 24));
   if (!dma_tiled_ok(p, tiled_min_n(), linear_tiled_min_rows())) return false;
   const bool wide = prefill_tile_tiled(p).bn == 256;
   if (p.wfmt != kE2M1) return wide;

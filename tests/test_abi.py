@@ -134,7 +134,7 @@ def test_linear_workspace_is_sized_for_the_call(lib, M):
         assert not _operand_order(lib, M, 28672, 4096, fmt, g, kernel=1)
         assert _operand_order(lib, M, 28672, 4096, fmt, g, kernel=0) == _operand_order(lib, M, 28672, 4096, fmt, g) or M <= 16
         if M >= 1024:
-            assert _operand_order(lib, M, 2048, 4096, fmt, g)
+            assert _operand_order(lib, M, 2048, 4096, fmt, g) == (fmt != "asym")
     assert not _operand_order(lib, M, 28672, 4096 + 32, "mxfp4", 32)
     K = 4096
     row_major = (M * K + 255) // 256 * 256 + (M * 4 + 255) // 256 * 256
@@ -154,7 +154,10 @@ def test_linear_workspace_is_sized_for_the_call(lib, M):
     ("mxfp4", 1024, 8192, 28672, True),
     # int4: the 256 x 256 tile
     ("sym", 512, 28672, 4096, True), ("sym", 512, 4096, 14336, False), ("sym", 512, 6144, 4096, False),
-    ("asym", 1000, 14336, 4096, True), ("asym", 129, 14336, 4096, False), ("sym", 1024, 6144, 4096, True)])
+    ("asym", 1000, 14336, 4096, True), ("asym", 129, 14336, 4096, False), ("sym", 1024, 6144, 4096, True),
+    # zero points from 1024 rows: that tile, or a K up to 4096 and two rounds of the grid
+    ("asym", 2048, 8192, 8192, True), ("asym", 1200, 4096, 14336, False), ("asym", 1777, 9728, 2560, True),
+    ("asym", 3000, 6144, 4096, True), ("asym", 3000, 6144, 4224, False), ("asym", 1777, 6144, 4096, False)])
 def test_operand_order_rule(lib, fmt, M, N, K, takes):
     assert _operand_order(lib, M, N, K, fmt, 32 if fmt == "mxfp4" else 128) == takes
 
