@@ -85,8 +85,8 @@ static bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 
 
 static const int kGemvMaxRows = 16;
 
-// Dense int4 (groups of 128+) and MXFP4 prefill calls of at least W4A8_PREFILL_TILED rows (default 1024; 0 turns it
-// off) that the DMA-staged kernel takes (its own checks, launch_prefill_dma) have their codes in
+// Dense int4 (groups of 128+) and MXFP4 prefill calls of at least W4A8_PREFILL_TILED rows (0 turns it off;
+// unset: 1024, and fewer where linear_tiled_ok says so) that the DMA-staged kernel takes (its own checks, launch_prefill_dma) have their codes in
 // that kernel's operand order with the row-sum seeds, which it then reads instead of computing them.
 // w4a8_linear quantizes x straight into that order (act_quant_tiled_lds_kernel, one launch as the
 // row-major quant) on weights of at least W4A8_PREFILL_TILED_N output channels (default 2048:
@@ -143,15 +143,12 @@ static bool dma_tiled_ok(const GemmArgs& p) {
 // more: AWQ K=2560 N=9728 M=1777 76.4 -> 74.3 us, K=4096 N=6144 M=3000 111.9 -> 109.9, but M=1024 48.0 ->
 // 49.0, K=4096 N=4096 M=1500 42.9 -> 44.3, K=14336 N=4096 M=1200 113.7 -> 122.9, K=28672 M=1200 217 -> 251.
 static const int64_t kTiledFewRows = 128;
-static int64_t linear_tiled_min_rows() {
-  const int64_t n = tiled_min_rows();
-  return n < kTiledFewRows ? n : kTiledFewRows;
-}
 static bool linear_tiled_ok(const GemmArgs& p) {
   if (p.M >= tiled_min_rows())
     return dma_tiled_ok(p, tiled_min_n(), tiled_min_rows()) &&
            (!p.zeros || prefill_tile_tiled(p).bn == 256 || (p.K <= 4096 && p.M * p.N >= 1 << 24));
-  if (!dma_tiled_ok(p, tiled_min_n(), linear_tiled_min_rows())) return false;
+  static const bool row_count_given = getenv("W4A8_PREFILL_TILED") != nullptr;
+  if (row_count_given || !dma_tiled_ok(p, tiled_min_n(), kTiledFewRows)) return false;
   const bool wide = prefill_tile_tiled(p).bn == 256;
   if (p.wfmt != kE2M1) return wide;
   return wide ? p.K <= 14336 && (p.M > 512 || p.K <= 2048 || p.K > 4096) : p.K <= 32768;

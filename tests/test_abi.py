@@ -1,6 +1,9 @@
 """C ABI surface and host-side refusal behaviour -- no kernel launches, runs without a GPU."""
 import ctypes
+import os
 import re
+import subprocess
+import sys
 from pathlib import Path
 
 import pytest
@@ -160,6 +163,20 @@ def test_linear_workspace_is_sized_for_the_call(lib, M):
     ("asym", 3000, 6144, 4096, True), ("asym", 3000, 6144, 4224, False), ("asym", 1777, 6144, 4096, False)])
 def test_operand_order_rule(lib, fmt, M, N, K, takes):
     assert _operand_order(lib, M, N, K, fmt, 32 if fmt == "mxfp4" else 128) == takes
+
+
+@pytest.mark.parametrize("value,takes", [(None, [200, 1023, 1024, 8192]), ("1024", [1024, 8192]), ("8192", [8192]),
+                                         ("100", [200, 1023, 1024, 8192]), ("0", [])])
+def test_operand_order_row_switch(value, takes):
+    """W4A8_PREFILL_TILED is the least row count of the operand order, below the default too; 0 turns it off."""
+    env = {k: v for k, v in os.environ.items() if k != "W4A8_PREFILL_TILED"}
+    if value is not None:
+        env["W4A8_PREFILL_TILED"] = value
+    code = (f"import ctypes; f = ctypes.CDLL({str(pkg('_abi').lib_path())!r}).w4a8_linear_workspace_bytes_for\n"
+            "i = ctypes.c_int64; f.restype = i; f.argtypes = [i, i, i] + [ctypes.c_int] * 3 + [i] + [ctypes.c_int] * 2\n"
+            "print([m for m in (99, 200, 1023, 1024, 8192) if f(m, 4096, 14336, 1, 0, 1, 32, 0, 2) > m * 14336 * 3 // 2])")
+    r = subprocess.run([sys.executable, "-c", code], env=env, capture_output=True, text=True, check=True)
+    assert r.stdout.strip() == str(takes)
 
 
 # ------------------------------------------------------------------------ provider refusals
