@@ -40,7 +40,8 @@ SIGNATURES = {
                                                  _c_int]),
     "w4a8_linear": (_c_int, [_vp, _c_int, _c_i64, _c_i64, _c_i64, _vp, _c_i64, _vp, _c_int, _vp, _c_int, _c_i64,
                              _vp, _c_int, _c_i64, _c_int, _vp, _c_i64, _c_int, _vp]),
-    # measurement probe (include/w4a8_probe.h), not part of the W4A8 path
+    # measurement probes (include/w4a8_probe.h), not part of the W4A8 path
+    "w4a8_probe_prefill_tile": (_c_int, [_c_i64, _c_i64, _c_i64, _c_int, _c_int, _c_int, _c_i64, _c_int, _c_int]),
     "w4a8_probe_read": (_c_int, [_vp, _c_i64, _c_int, _c_int, _c_int, _vp, _vp]),
     "w4a8_linear_launch_count": (_c_int, [_c_i64, _c_i64, _c_i64, _c_int, _c_int, _c_int, _c_int, _c_i64, _c_int,
                                           _c_int]),

@@ -9,6 +9,7 @@
 
 #include "gemm_args.h"
 #include "../../include/w4a8_mi355x.h"
+#include "../../include/w4a8_probe.h"
 
 namespace w4a8 {
 int launch_act_quant(const void* x, int dtype, int64_t M, int64_t K, int64_t ldx, uint8_t* q,
@@ -24,7 +25,7 @@ size_t gemv_workspace_bytes(int64_t M, int64_t N, int64_t K, int grouped, int64_
 int launch_prefill(const GemmArgs& p, int64_t rows_to_cover, int bm_rows, hipStream_t stream);
 int launch_prefill_staged(const GemmArgs& p, int64_t rows_to_cover, int bm_rows, hipStream_t stream);
 int launch_prefill_dma(const GemmArgs& p, int64_t rows_to_cover, int bm_rows, hipStream_t stream);
-DmaTile prefill_tile_tiled(const GemmArgs& p);
+DmaTile prefill_tile(const GemmArgs& p, bool a_tiled);
 int launch_moe_route(const void* logits, int dtype, int64_t T, int E, int top_k, int renorm, float* tw,
                      int32_t* ids, hipStream_t stream);
 int launch_moe_align(const int32_t* ids, int64_t numel, int E, int bm, int64_t P, int32_t* sorted_ids,
@@ -121,7 +122,7 @@ static bool needs_seeds(const GemmArgs& p) { return p.wfmt == kInt4 && !p.zeros;
 // pays through the 256 x 256 tile only (AWQ K=8192 N=28672 M=1500 446 -> 375 us; on the other tiles K=4096
 // N=16384 M=1500 121.9 -> 124.5)
 static bool dma_tiled_ok(const GemmArgs& p) {
-  return dma_tiled_ok(p, 16384, tiled_min_rows()) && (!p.zeros || prefill_tile_tiled(p).bn == 256);
+  return dma_tiled_ok(p, 16384, tiled_min_rows()) && (!p.zeros || prefill_tile(p, true).bn == 256);
 }
 
 // w4a8_linear's own calls, whose quant is one launch in either layout, take it below that too:
@@ -146,10 +147,10 @@ static const int64_t kTiledFewRows = 128;
 static bool linear_tiled_ok(const GemmArgs& p) {
   if (p.M >= tiled_min_rows())
     return dma_tiled_ok(p, tiled_min_n(), tiled_min_rows()) &&
-           (!p.zeros || prefill_tile_tiled(p).bn == 256 || (p.K <= 4096 && p.M * p.N >= 1 << 24));
+           (!p.zeros || prefill_tile(p, true).bn == 256 || (p.K <= 4096 && p.M * p.N >= 1 << 24));
   static const bool row_count_given = getenv("W4A8_PREFILL_TILED") != nullptr;
   if (row_count_given || !dma_tiled_ok(p, tiled_min_n(), kTiledFewRows)) return false;
-  const bool wide = prefill_tile_tiled(p).bn == 256;
+  const bool wide = prefill_tile(p, true).bn == 256;
   if (p.wfmt != kE2M1) return wide;
   return wide ? p.K <= 14336 && (p.M > 512 || p.K <= 2048 || p.K > 4096) : p.K <= 32768;
 }
@@ -413,6 +414,19 @@ int w4a8_linear_launch_count(int64_t M, int64_t N, int64_t K, int x_dtype, int s
 }
 
 }  // extern "C"
+
+extern "C" int w4a8_probe_prefill_tile(int64_t M, int64_t N, int64_t K, int scale_fmt, int has_zeros, int wfmt,
+                                       int64_t group_size, int silu, int operand_order) {
+  const void* fake = reinterpret_cast<const void*>(static_cast<uintptr_t>(256));
+  GemmArgs p;
+  int rc = dense_args("w4a8_probe_prefill_tile", M, fake, N, K, fake, scale_fmt,
+                      has_zeros ? reinterpret_cast<const int32_t*>(fake) : nullptr, wfmt, group_size,
+                      const_cast<void*>(fake), kBF16, N, silu, 2, p);
+  if (rc) return -rc;
+  if (M == 0 || scale_fmt == kScaleE4M3) return 0;
+  const DmaTile t = prefill_tile(p, operand_order != 0);
+  return t.bm << 16 | t.bn;
+}
 
 // ---- W4A16: unquantized bf16/fp16 activations, split exactly into fp8 terms (w4a16.hip)
 static int64_t round16(int64_t b) { return (b + 15) / 16 * 16; }

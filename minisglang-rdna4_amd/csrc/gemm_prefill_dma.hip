@@ -660,9 +660,10 @@ static const DmaTile kInt4TiledA[] = {{256, 128, 1.0f}, {192, 128, 0.81f}, {128,
 static const DmaTile kMxTiles[] = {{256, 256, 1.0f}, {192, 256, 0.80f}, {128, 256, 0.60f}, {192, 128, 0.50f},
                                    {128, 128, 0.45f}, {64, 128, 0.33f}, {64, 64, 0.29f}};
 
-// the tile of a dense int4 (groups of 128+) or MXFP4 call given its activations in operand order
-DmaTile prefill_tile_tiled(const GemmArgs& p) {
-  return p.wfmt == kE2M1 ? kMxTiles[pick_tile(kMxTiles, p, p.M)] : kInt4TiledA[pick_tile(kInt4TiledA, p, p.M)];
+// the tile that launch_prefill_dma gives a dense call, its activations in operand order or not
+DmaTile prefill_tile(const GemmArgs& p, bool a_tiled) {
+  if (p.wfmt == kE2M1) return kMxTiles[pick_tile(kMxTiles, p, p.M)];
+  return a_tiled ? kInt4TiledA[pick_tile(kInt4TiledA, p, p.M)] : kInt4Tiles[pick_tile(kInt4Tiles, p, p.M)];
 }
 
 // int4 with groups of 32, 64 and 128+ and MXFP4, on 16-byte aligned rows; kErrUnsupported otherwise.

@@ -22,6 +22,23 @@ def _weight(fmt, g, N, K, seed, E=None):
     return (*synth.int4_weight(N, K, g, seed=seed, asym=fmt == "asym", scale_floor=1e-4, E=E), False, False)
 
 
+def _call(fmt):
+    """(scale_fmt, has_zeros, wfmt) of a format, as the C ABI's planning calls take them."""
+    return {"sym": (0, 0, 0), "asym": (0, 1, 0), "mxfp4": (1, 0, 1), "nvfp4": (2, 1, 1)}[fmt]
+
+
+def _tile(fmt, g, M, N, K, silu=False, operand_order=False):
+    """The (rows, columns) of the dense tile that a call runs on."""
+    t = pkg("_abi").load().w4a8_probe_prefill_tile(M, N, K, *_call(fmt), g, int(silu), int(operand_order))
+    return t >> 16, t & 0xFFFF
+
+
+def _operand_order(fmt, g, M, N, K, silu=False):
+    """Whether w4a8_linear takes the call's activations in operand order (it asks for the room)."""
+    row_major = (M * K + 255) // 256 * 256 + (M * 4 + 255) // 256 * 256
+    return pkg("_abi").load().w4a8_linear_workspace_bytes_for(M, N, K, *_call(fmt), g, int(silu), 2) > row_major
+
+
 FMTS = [("sym", 32), ("asym", 32), ("sym", 64), ("asym", 64), ("asym", 128), ("asym", 256), ("mxfp4", 32), ("nvfp4", 16)]
 
 
@@ -78,14 +95,18 @@ def test_moe_groups_and_k_tails(kernels, oracle, dev, fmt, g, h, i, bm):
     assert np.isfinite(res["out"].float().cpu().numpy()).all()
 
 
-# one row past 64, 128, 192 and 256 rows, and sizes that take each dense tile shape: 64 x 64 (few
-# workgroups), 64 x 128, 128 x 128, 192- and 256-row tiles, and MXFP4's 256-wide ones
+# one row past 64, 128, 192 and 256 rows, and sizes that take each dense tile shape of row-major int4 and of
+# MXFP4 (NVFP4 has int4's)
 @pytest.mark.parametrize("fmt,g", [("sym", 128), ("asym", 32), ("mxfp4", 32), ("nvfp4", 16)])
-@pytest.mark.parametrize("M,N", [(65, 80), (129, 8208), (193, 12304), (321, 14352), (577, 16400), (1153, 8208)])
-def test_dense_tile_shapes(kernels, oracle, dev, fmt, g, M, N):
+@pytest.mark.parametrize("M,N,int4,mxfp4", [(65, 80, (64, 64), (64, 64)), (129, 8208, (64, 128), (64, 128)),
+                                            (193, 12304, (128, 128), (128, 128)), (321, 14352, (192, 128), (192, 128)),
+                                            (391, 14320, (256, 128), (128, 256)), (577, 16400, (128, 128), (256, 256)),
+                                            (1153, 8208, (192, 128), (192, 256))])
+def test_dense_tile_shapes(kernels, oracle, dev, fmt, g, M, N, int4, mxfp4):
     """Every tile shape gives a row the same bits: the call's rows against the same rows in calls of
     seven, and those against the oracle."""
     K = 384
+    assert fmt == "nvfp4" or _tile(fmt, g, M, N, K) == (mxfp4 if fmt == "mxfp4" else int4)
     w, s, z, e2, nv = _weight(fmt, g, N, K, seed=M + N)
     x = synth.activations(M, K, seed=M + 1)
     tiles, sd = kernels.repack_w4(w.to(dev), weight_is_e2m1=e2), s.to(dev)
@@ -110,6 +131,8 @@ def test_wide_tile_matches_the_others(kernels, dev, M, N, K, silu, asym, g):
     without a workspace) on the same codes."""
     if K % g:
         pytest.skip("group does not divide K")
+    fmt = "asym" if asym else "sym"
+    assert _operand_order(fmt, g, M, N, K, silu) and _tile(fmt, g, M, N, K, silu, True) == (256, 256)
     abi = pkg("_abi")
     lib = abi.load()
     w, s, z = synth.int4_weight(N, K, g, seed=N + K, asym=asym, scale_floor=1e-4)
@@ -130,13 +153,14 @@ def test_wide_tile_matches_the_others(kernels, dev, M, N, K, silu, asym, g):
     assert torch.equal(out, ref), f"max {(out.float() - ref.float()).abs().max().item():.3e}"
 
 
-@pytest.mark.parametrize("fmt", ["asym", "mxfp4"])
+# zero points take it at such K through the 256 x 256 tile only, so on the wider weight
+@pytest.mark.parametrize("fmt,N", [("asym", 13056), ("mxfp4", 2048)])
 @pytest.mark.parametrize("M,K", [(1024, 4224), (1037, 8192), (1026, 8320), (1100, 16384), (1030, 16512)])
-def test_long_rows_quantized_in_operand_order(kernels, dev, fmt, M, K):
+def test_long_rows_quantized_in_operand_order(kernels, dev, fmt, N, M, K):
     """Rows of more than 4096 elements on formats without seeds: four rows per workgroup up to 16384
     elements (one and two chunks per thread, ragged row blocks), two passes beyond on more than 1024 rows,
     bit for bit against the row-major quant and GEMM."""
-    N = 2048
+    assert _operand_order(fmt, 32 if fmt == "mxfp4" else 128, M, N, K)
     abi = pkg("_abi")
     lib = abi.load()
     w, s, z, e2, _ = _weight(fmt, 128, N, K, seed=K)
@@ -156,15 +180,16 @@ def test_long_rows_quantized_in_operand_order(kernels, dev, fmt, M, K):
 
 # below 1024 rows: int4 where 256 x 256 tiles fit the grid (one quant kernel each side of K = 4096),
 # MXFP4 from 128 rows up to K = 32768 (three and four chunks per thread), and one row or K tile outside each
-@pytest.mark.parametrize("fmt,M,N,K", [("sym", 448, 28672, 512), ("sym", 511, 24576, 4224), ("asym", 500, 28672, 384),
-                                        ("asym", 1023, 14336, 4224), ("mxfp4", 127, 2048, 384), ("mxfp4", 128, 2048, 384),
-                                        ("mxfp4", 129, 2064, 4224), ("mxfp4", 1023, 2048, 16384),
-                                        ("mxfp4", 200, 2048, 16512), ("mxfp4", 130, 2032, 512), ("mxfp4", 1023, 2048, 24576),
-                                        ("mxfp4", 131, 2048, 24704), ("mxfp4", 1024, 2048, 32768),
-                                        ("mxfp4", 1025, 2048, 28672), ("mxfp4", 200, 2048, 32896)])
-def test_few_rows_in_operand_order(kernels, dev, fmt, M, N, K):
+@pytest.mark.parametrize("fmt,M,N,K,takes", [
+    ("sym", 448, 28672, 512, True), ("sym", 511, 24576, 4224, True), ("asym", 500, 28672, 384, True),
+    ("asym", 1023, 14336, 4224, True), ("mxfp4", 127, 2048, 384, False), ("mxfp4", 128, 2048, 384, True),
+    ("mxfp4", 129, 2064, 4224, True), ("mxfp4", 1023, 2048, 16384, True), ("mxfp4", 200, 2048, 16512, True),
+    ("mxfp4", 130, 2032, 512, False), ("mxfp4", 1023, 2048, 24576, True), ("mxfp4", 131, 2048, 24704, True),
+    ("mxfp4", 1024, 2048, 32768, True), ("mxfp4", 1025, 2048, 28672, True), ("mxfp4", 200, 2048, 32896, False)])
+def test_few_rows_in_operand_order(kernels, dev, fmt, M, N, K, takes):
     w, s, z, e2, _ = _weight(fmt, 128, N, K, seed=M + K)
     g = 32 if e2 else 128
+    assert _operand_order(fmt, g, M, N, K) == takes
     tiles, sd, zd = kernels.repack_w4(w.to(dev), e2), s.to(dev), None if z is None else z.to(dev)
     x = synth.activations(M, K, seed=M, outliers=True).to(dev)
     q, sc = kernels.act_quant(x)

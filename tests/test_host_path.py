@@ -104,6 +104,39 @@ def _weight(fmt, N, K, dev, E=None):
 @pytest.mark.gpu
 @pytest.mark.parametrize("fmt", ["sym", "asym", "asym64", "mxfp4", "nvfp4"])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_plain_calls_are_served_by_the_extension(kernels, dev, fmt, dtype):
+    """What the comparisons below do not show, since a call that the extension leaves is the Python path's on
+    both sides: it takes the calls it is there for."""
+    m = pkg("_host").load()
+    assert m is not pkg("_host")._Absent
+    E, H, I = 8, 512, 256
+    w, s, z, g, e2 = _weight(fmt, 96, H, dev)
+    t = kernels.repack_w4(w, weight_is_e2m1=e2)
+    w13, s13, z13, _, _ = _weight(fmt, 2 * I, H, dev, E=E)
+    w2, s2, z2, _, _ = _weight(fmt, H, I, dev, E=E)
+    t13, t2 = kernels.repack_w4(w13, e2), kernels.repack_w4(w2, e2)
+    abi = pkg("_abi")
+    for M in (1, 16, 17, 70):
+        x = synth.activations(M, H, seed=M, dtype=dtype).to(dev)
+        lg = synth.router_logits(M, E, seed=M).to(dev)
+        q, sc = kernels.act_quant(x)
+        out, arm = m.linear(x, t, s, z, g, e2, None, None, False, abi.KERNEL_AUTO)
+        assert arm == (abi.KERNEL_DECODE if M <= 16 else abi.KERNEL_PREFILL)
+        for call in (m.linear(x, t, s, z, g, e2, q, sc, False, abi.KERNEL_AUTO),
+                     m.linear(x, torch.nn.Parameter(t, requires_grad=False), s, z, g, e2, None, None, False, abi.KERNEL_AUTO)):
+            assert torch.equal(call[0], out)
+        if M <= 16:
+            assert m.linear(x, t, s, z, g, e2, None, None, True, abi.KERNEL_DECODE)[0].shape == (M, 48)
+        assert m.rms_norm(x, None, 1e-6, False, None, False).shape == (M, H)
+        assert len(m.rms_norm(x, x[0].clone(), 1e-6, False, x.clone(), True)) == 3
+        bm = 16 if M <= 16 else 64
+        assert m.moe(x, t13, s13, z13, t2, s2, z2, lg, 2, True, e2, bm, M == 1, True, True, M <= 16)[0].shape == (M, H)
+    torch.cuda.synchronize()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("fmt", ["sym", "asym", "asym64", "mxfp4", "nvfp4"])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_linear_forms(kernels, dev, monkeypatch, fmt, dtype):
     K, N = 512, 96
     w, s, z, g, e2 = _weight(fmt, N, K, dev)
