@@ -1,4 +1,4 @@
-"""W4A8 decode-GEMV sweep benchmark on one MI355X.
+"""W4A8 decode-GEMV sweep benchmark on one MI355X at Llama-3-8B layer shapes.
 
 One step = the W4A8 quantized linear (per-token fp8 act-quant + int4 x fp8 GEMM, bf16 out) at the
 four Llama-3-8B layer shapes (qkv 4096x6144, o_proj 4096x4096, gate_up 4096x28672, down 14336x4096)
@@ -13,16 +13,16 @@ the largest shape (gate_up, M=1, one launch per call): algorithmic bytes per lau
 time from HIP events on the launch stream, against 8 TB/s. decode_per_shape times every call of the
 step on its own (GB/s and fraction per shape and M). cpu_baseline is the reference's
 dequantize-then-matmul CPU path (oracle/baseline.py): the whole sweep step on all host cores, median
-of 5 passes, with the CPU model, rank 0 only. prefill_config3 is configs[2]/[3]: every shape at
+of 5 passes, with the CPU model, rank 0 only. prefill_config3 is the int4 prefill: every shape at
 M = 512, 2048, 8192 on the producer pair (act-quant outside the timed region).
 
-other_configs reports the remaining BASELINE configs through the same operator API: cfg1 (AWQ
+other_configs reports the other workloads through the same operator API: cfg1 (AWQ
 zero-point int4, M=16, K=2560, N=9728), cfg4 (MoE E=128 top-8 H=2048 I=768, T in {1,16,256,4096})
 and cfg5 (MXFP4 E8M0, K x N in {8192x28672, 28672x8192}, M in {1,16,4096}); GB/s against 8 TB/s
 for the decode sizes, TFLOPS against the 5 PFLOPS fp8 peak for the large ones.
 
 next_formats reports the W4A16 arm (unquantized activations) and NVFP4 through the same operator
-API (not BASELINE configs; the shapes are the gate_up ones above).
+API (the shapes are the gate_up ones above).
 
 producer_norm_step times the same sweep with its inputs coming out of the RMSNorm + residual-add
 producer: once with the linear quantizing its bf16 input, once with the producer's fp8 pair
@@ -135,7 +135,7 @@ def roofline_leg(kernels, dev, reps: int = 60) -> dict:
 
 
 def prefill_leg(kernels, dev) -> dict:
-    """TFLOPS of the MFMA GEMM at every configs[2]/[3] shape (M = 512, 2048, 8192), one warm call
+    """TFLOPS of the MFMA GEMM at every Llama-3-8B prefill shape (M = 512, 2048, 8192), one warm call
     then 5 timed calls on the producer pair (x_fp8, act_scales): the act-quant launch is outside the
     timed region (in_op_quant_us adds it back for one shape per M)."""
     import torch
@@ -168,7 +168,7 @@ def prefill_leg(kernels, dev) -> dict:
 
 
 def decode_shapes_leg(kernels, dev) -> dict:
-    """Every configs[1] call on its own: (shape, M) -> mean us per call (act-quant + GEMV, or the
+    """Every call of the decode sweep on its own: (shape, M) -> mean us per call (act-quant + GEMV, or the
     one fused launch) with back-to-back launches, weights rotated over more than 600 MB (over twice
     the MALL) so every call streams from HBM; GB/s on the algorithmic bytes and the fraction of the
     8 TB/s peak."""
@@ -215,7 +215,7 @@ def profile_prefill(kernels, dev, fmt: str, M: int, K: int, N: int) -> dict:
 
 
 def profile_moe(kernels, dev, T: int) -> dict:
-    """One configs[4] MoE call shape (E=128, top-8, H=2048, I=768, int4 g128), 2 warm + 5 timed
+    """One MoE call shape (E=128, top-8, H=2048, I=768, int4 g128), 2 warm + 5 timed
     calls, for kernel-trace and counter runs."""
     import torch
 
@@ -316,7 +316,7 @@ def _tflops(flops: float, us: float) -> dict:
 
 
 def configs_leg(kernels, dev) -> dict:
-    """The other BASELINE configs through the product's operator API, weights rotated over more
+    """The other workloads through the product's operator API, weights rotated over more
     than twice the 256 MB MALL for the bandwidth-bound cases: cfg1 (AWQ zero-point int4 g128,
     M=16, K=2560, N=9728), cfg4 (MoE E=128 top-8 H=2048 I=768, int4 g128 fp16 scales, T in
     {1,16,32,256,4096}) and cfg5 (MXFP4 E8M0 block-32 at K=8192,N=28672 and K=28672,N=8192, M in
@@ -387,7 +387,7 @@ def configs_leg(kernels, dev) -> dict:
 
 
 def formats_leg(kernels, dev) -> dict:
-    """The formats beyond the BASELINE configs, through the same operator API: the W4A16 arm
+    """The further formats, through the same operator API: the W4A16 arm
     (unquantized bf16 activations; GPTQ-sym int4 g128 at the gate_up shape K=4096, N=28672, M in
     {1, 16, 2048}) and NVFP4 (e2m1 + e4m3 block-16 scales + per-channel global; W4A8 at the cfg5
     gate_up shape K=8192, N=28672, M in {1, 16, 4096}, and W4A16 at M=1). Weights rotate over more
@@ -442,7 +442,7 @@ def formats_leg(kernels, dev) -> dict:
 
 
 def producer_leg(kernels, dev, weights, steps: int = 100) -> dict:
-    """The configs[1] sweep with its activations produced by the RMSNorm + residual-add producer, in
+    """The decode sweep with its activations produced by the RMSNorm + residual-add producer, in
     two graph-replayed steps of 20 (norm, linear) pairs: `in_op_quant` runs rms_norm_add then
     w4a8_linear on bf16 x (the linear quantizes), `producer_pair` runs rms_norm_add_quant then
     w4a8_linear on the (x_fp8, act_scales) pair it emitted. Same weights as the headline step."""
@@ -496,7 +496,7 @@ def producer_leg(kernels, dev, weights, steps: int = 100) -> dict:
 
 
 def launches_per_step() -> int:
-    """Kernel launches of one configs[1] step (w4a8_linear_launch_count over its 20 calls)."""
+    """Kernel launches of one decode step (w4a8_linear_launch_count over its 20 calls)."""
     lib = importlib.import_module("minisglang-rdna4_amd._abi").load()
     return sum(lib.w4a8_linear_launch_count(M, N, K, 0, 0, 0, 0, GROUP, 0, 0) for M in MS for (K, N) in SHAPES)
 
@@ -516,7 +516,7 @@ def main() -> int:
     ap.add_argument("--profile-prefill", nargs=4, metavar=("FMT", "M", "K", "N"),
                     help="time one prefill GEMM (FMT int4, mxfp4 or nvfp4) and exit, for counter runs")
     ap.add_argument("--profile-moe", type=int, metavar="T",
-                    help="time one configs[4] MoE call of T tokens and exit, for trace and counter runs")
+                    help="time one MoE call of T tokens and exit, for trace and counter runs")
     args = ap.parse_args()
     world = int(os.environ.get("WORLD_SIZE", "1"))
     if args.gpus != 1 or world != 1:
@@ -620,7 +620,7 @@ def main() -> int:
         "data": "synthetic (seeded): GPTQ-sym int4 g128 codes U{0..15}, fp16 scales |N(0,0.02)|, bf16 N(0,1) "
                 "activations with 0.1% channels x50",
         "config": {
-            "workload": "configs[1]: decode W4A8 GEMM sweep at Llama-3-8B layer shapes, M in {1,2,4,8,16}; one step = "
+            "workload": "decode W4A8 GEMM sweep at Llama-3-8B layer shapes, M in {1,2,4,8,16}; one step = "
                         "20 calls (per-token act quant + GEMM each), HIP-graph replayed",
             "launches_per_step": launches_per_step(),
             "shapes_KxN": [f"{K}x{N}" for K, N in SHAPES],

@@ -329,16 +329,16 @@ act_quant_tiled_short_kernel(const uint16_t* __restrict__ x, int64_t ldx, int64_
   }
 }
 
-// The same for rows of 4097 to 16384 elements, and of up to 32768 in calls of up to 1024 rows, with x read once: a workgroup of 16 waves holds 4 rows in
-// registers (thread t: the 8-element chunks t + 1024 i of each), takes their maxima through one barrier,
-// and writes each chunk's 8 codes straight to their operand-order place. Four rows are the fewest whose
-// pieces fill a 64-byte segment of the output (4 rows x 16 bytes), which L2 then writes whole. The
-// two-pass kernel has a quarter as many workgroups and reads x twice: whole MXFP4 calls at K=8192 N=8192
-// M=1024 66.5 -> 59.3 us, K=14336 N=4096 M=2000 109 -> 106. Longer rows need it only while the two passes
-// have few workgroups: K=28672 N=8192 M=1024 209 -> 193 us and M=400 136 -> 115, K=24576 N=4096 M=1024
-// 119 -> 103, but K=28672 N=8192 M=2000 344 -> 349 and M=4096 690 -> 705. Calls that need seeds keep the two
-// passes (the tiles pass through its registers, where reading the codes back would cost what the second
-// read of x does).
+// The same for rows of 4097 to 16384 elements, and of up to 32768 in calls of up to 1024 rows, with x read
+// once: a workgroup of 16 waves holds 4 rows in registers (thread t: the 8-element chunks t + 1024 i of
+// each), takes their maxima through one barrier, and writes each chunk's 8 codes straight to their
+// operand-order place. Four rows are the fewest whose pieces fill a 64-byte segment of the output (4 rows x
+// 16 bytes), which L2 then writes whole. The two-pass kernel has a quarter as many workgroups and reads x
+// twice. Whole MXFP4 calls on the two passes -> on this: K=8192 N=8192 M=1024 66.5 -> 59.3 us, K=14336
+// N=4096 M=2000 109 -> 106. Longer rows need it only while the two passes have few workgroups: K=28672
+// N=8192 M=1024 209 -> 193, K=24576 N=4096 M=1024 119 -> 103, but K=28672 N=8192 M=2000 344 -> 349 and
+// M=4096 690 -> 705. Calls that need seeds keep the two passes (the tiles pass through its registers, where
+// reading the codes back would cost what the second read of x does).
 template <int CPT>
 __global__ void __launch_bounds__(1024)
 act_quant_tiled_rows_kernel(const uint16_t* __restrict__ x, int64_t ldx, int64_t M, int64_t K, int dtype,

@@ -65,7 +65,7 @@ GemvPlan plan_gemv(const GemmArgs& p, int64_t row_blocks, bool quant_src) {
   // narrower dense weights (o_proj, down at 4096 channels) run one strip each, twice the grid
   // (grouped MoE calls keep two: their grids already span the routed experts, except for decode
   // batches of at most 64 slots, whose few blocks hold a row or two each: one strip there, twice
-  // the grid; configs[4] T=1 21.0 -> 19.7 us, T=2 25.4 -> 23.0, T=8 46.7 -> 45.8; and gemm1 (the
+  // the grid; MoE E=128 top-8 H=2048 I=768 T=1 21.0 -> 19.7 us, T=2 25.4 -> 23.0, T=8 46.7 -> 45.8; and gemm1 (the
   // silu arm) up to 256 slots, whose blocks hold a few rows: T=16 66.1 -> 62.1 us, T=32 83.7 ->
   // 80.6, where T=256 measured 126.8 -> 130.8 with one strip)
   pl.nstr = rows > 4 && (p.sorted_ids || strips >= 384) ? 2 : 1;
@@ -120,7 +120,7 @@ GemvPlan plan_gemv(const GemmArgs& p, int64_t row_blocks, bool quant_src) {
 // The strip-walking GEMV (gemv_walk.hip) for one row block of bf16/fp16 rows, int4 with groups of
 // 128+ or MXFP4. Its cost over the weight stream is the row phase, where every workgroup quantizes
 // all M x K values, vpt of them per thread of its 8 waves. Measured on MI355X against act quant +
-// gemv_kernel (configs[1] shapes, configs[0], configs[5] and a few odd shapes; outputs equal bit for
+// gemv_kernel (Llama-3-8B shapes, K=2560 N=9728, MXFP4 K=8192 N=28672 and a few odd shapes; outputs equal bit for
 // bit):
 //   * vpt <= 96: the walk is faster or ties at every shape (K=4096 N=4096 M=4 6.0 against 8.2 us,
 //     K=4096 N=6144 M=8 8.1 against 9.0, K=14336 N=4096 M=2 10.0 against 11.9, K=2560 N=9728 asym
@@ -189,7 +189,7 @@ bool plan_gemv_walk(const GemmArgs& p, int64_t row_blocks, WalkPlan& wp) {
 // window sets their registers and occupancy (NS=4: 160 VGPRs with 4 tiles, 104 with 2; 3 and 4
 // waves per SIMD become 4 and 6), and more resident waves keep more loads in flight than a longer
 // window per wave. Measured on MI355X against the 4-tile window, outputs equal bit for bit (the
-// window does not change the summation order): configs[4] MoE whole call T=16 60.7 -> 56.3 us,
+// window does not change the summation order): MoE (E=128 top-8 H=2048 I=768) whole call T=16 60.7 -> 56.3 us,
 // T=32 79.4 -> 72.4, T=256 118.8 -> 110.2, T=512 171.0 -> 155.6 (3 tiles: between the two; 1
 // tile: 1-2 us slower than 2 at T <= 64); dense K=14336 N=4096 M=16 16.4 -> 15.3 us, K=4096
 // N=4096 M=16 8.48 -> 8.25, the other decode-sweep calls within 0.5%.

@@ -1,5 +1,5 @@
 // Large-M W4A8 GEMM (prefill band and grouped MoE GEMMs) with the activation tile copied straight
-// from global memory into LDS by the buffer unit (buffer_load ... lds), three LDS stages deep.
+// from global memory into LDS by the buffer unit (buffer_load ... lds), three LDS stages deep (the 64 x 64 tile four).
 //
 // The math of the reference's wmma_tiled_tuned arm and of its grouped MoE GEMMs
 // (python/minisgl/quant/kernels.py:1632, 1686-1734, 744-773): y[m,n] = s_m * sum_g scale[g,n] *
@@ -16,15 +16,15 @@
 //   writes it to LDS, with its fp16 scales. Symmetric groups of 128+ are unpacked as q - 7.5 with one
 //   table lookup and the half step taken back through the row sums; the other forms as e4m3(q - z),
 //   which needs no row sums (decode_lut4). With zero points applied per accumulator instead (two FMAs
-//   per element and a row-sum MFMA per row block) M=1777 K=2560 N=9728 took 102 us, so 86. Groups of
-//   32 on the kernel that masks the full-rate MFMA and loads operands straight from global memory:
-//   M=2048 K=2816 N=2048 196 us, here 44.
+//   per element and a row-sum MFMA per row block) a call of M=1777 K=2560 N=9728 on row-major 256 x 128
+//   tiles took 102 us, so 86. Groups of 32 on the kernel that masks the full-rate MFMA and loads operands
+//   straight from global memory: M=2048 K=2816 N=2048 196 us a call, here 42.
 // Each stage is its own __shared__ array and every stage index is a compile-time constant (the K
-// loop is unrolled by three), so the compiler tells the stages apart: reading stage k does not
-// wait for the DMAs in flight to stages k+1 and k+2. Step k issues the loads of step k+2 (int4:
-// between its MFMAs), computes step k, writes the int4 registers of step k+1, then waits for its
-// own step-k+1 loads (a counted vmcnt, the loads of step k+2 stay in flight) and meets the other
-// waves at one s_barrier.
+// loop is unrolled by the stages), so the compiler tells the stages apart: reading stage k does not
+// wait for the DMAs in flight to the later ones. With three stages step k issues the loads of step
+// k+2 (int4: between its MFMAs), computes step k, writes the int4 registers of step k+1, then waits
+// for its own step-k+1 loads (a counted vmcnt, the loads of step k+2 stay in flight) and meets the
+// other waves at one s_barrier; with four, everything is loaded one step earlier.
 #include "prefill.h"
 
 namespace w4a8 {
@@ -515,14 +515,14 @@ gemm_dma_kernel(const GemmArgs p) {
     }
   };
 
-  // one pipelined step kt (stage C = kt % 3): loads of kt+2, MFMAs of kt, int4 registers of kt+1
-  // to LDS, wait for kt+1's loads, barrier. The loads of kt+2 are issued between the step's MFMAs
+  // one pipelined step kt (stage C = kt % NST): loads of kt+D, MFMAs of kt, int4 registers of kt+1
+  // to LDS, wait for kt+1's loads, barrier. The loads of kt+D are issued between the step's MFMAs
   // instead of ahead of them all (int4: the weight loads after the first strip's, ahead of the
   // unpack of kt+1's weights, and the A DMAs after the second's; MXFP4: all after the second row
   // block's): at the top of the step every wave's loads would meet in the address unit's queue
-  // while the step's first MFMAs wait (1-4% on configs[3] and configs[5] shapes). The weight
+  // while the step's first MFMAs wait (1-4% on int4 and MXFP4 shapes from 2048 rows). The weight
   // registers go first because the unpack one step later waits on them, while the A DMAs are only
-  // waited for at the end of the next step (weights first: configs[3] 2-8% faster, MoE T=4096 2%).
+  // waited for at the end of the next step (weights first: int4 2-8% faster from 2048 rows, MoE T=4096 2%).
   auto step = [&](auto C, int kt, auto Tail) __attribute__((always_inline)) {
     if (decltype(Tail)::value && kt >= KT) return;
     constexpr int c = decltype(C)::value, n1 = (c + 1) % NST, nd = (c + D) % NST;

@@ -1,5 +1,6 @@
 // The dense int4 prefill GEMM (groups of 128+) on 256 x 256 tiles, for activations in operand order
-// (GemmArgs::a_tiled), symmetric with their row-sum seeds or with zero points; the math and the bits of gemm_prefill_dma.hip's tiles.
+// (GemmArgs::a_tiled), symmetric with their row-sum seeds or with zero points; the math and the bits of
+// gemm_prefill_dma.hip's tiles.
 //
 // What bounds the 256 x 128 tile there is not its MFMAs but what goes with each: 1 KiB of LDS operands
 // per MFMA, and a barrier every 16 of them. A 256 x 256 tile halves the barriers and takes a quarter
@@ -12,10 +13,10 @@
 //   * two stages of 32 KiB activations, 32 KiB unpacked weights, scales and seeds. Activations, scales
 //     and seeds go to LDS by LDS-DMA at the start of the step before theirs, which is twice as long as a
 //     256 x 128 step; the 4-bit weights are loaded to registers two steps ahead and unpacked one ahead.
-// Whole calls, 256 x 128 -> 256 x 256, us: K=4096 N=28672 M=8192 1134 -> 955 (2.0 PFLOP/s), N=6144 M=8192
-// 259 -> 220, N=4096 M=8192 181 -> 153, K=14336 N=4096 M=4096 308 -> 267, K=1024 N=4096 M=4096 37.0 -> 32.1.
-// With zero points (row-major 256 x 128 tiles before, two FMAs per output and step): N=28672 M=8192
-// 1325 -> 970, N=14336 M=3000 279 -> 204.
+// Whole calls, operand order on 256 x 128 -> 256 x 256, us: K=4096 N=28672 M=8192 1134 -> 955 (2.0
+// PFLOP/s), N=6144 M=8192 259 -> 220, N=4096 M=8192 181 -> 153, K=14336 N=4096 M=4096 308 -> 267, K=1024
+// N=4096 M=4096 37.0 -> 32.1. With zero points, row-major codes on the tiles they take -> operand order on
+// this one: K=4096 N=28672 M=8192 1167 -> 1006, N=14336 M=3000 239 -> 208, N=4096 M=8192 177 -> 159.
 // The unpack placed one row block earlier or later, the DMAs ahead of the step's LDS reads, and a raised
 // wave priority around the MFMAs all measured within 1%.
 #include "prefill.h"

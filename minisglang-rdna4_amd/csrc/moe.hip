@@ -307,7 +307,7 @@ constexpr int kPrepMaxSlots = 256;
 // in issue order (volatile keeps the compiler to that order), so no barrier separates the steps.
 // ids in LDS; base_s, cnt_s, mask_s, total_s: LDS for the expert starts, the counts, the chunk
 // masks and ntp. Against align_block (which the prep launch ran past 64 slots, where a loop over
-// every slot per lane counted the experts): configs[4] T=16 prep launch 8.1 -> 7.6 us.
+// every slot per lane counted the experts): E=128 top-8 T=16 prep launch 8.1 -> 7.6 us.
 template <int EPL>
 __device__ __forceinline__ void align_wave(const int32_t* ids, int numel, int E, int bm, int64_t P,
                                            int32_t* __restrict__ sorted_ids, int32_t* __restrict__ expert_ids,

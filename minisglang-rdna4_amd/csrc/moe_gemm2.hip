@@ -262,12 +262,12 @@ bool moe_gemm2_combine_fits(int64_t K, int scale_fmt, bool has_zeros, int wfmt, 
   return fmt && wide_ok && K % kTileK == 0 && K <= 16 * kTileK && top_k >= 1 && top_k <= kG2cMaxSlots;
 }
 
-// The 8-tile, 8-slot kernel (the configs[4] decode shape) takes two strips per workgroup from 8
+// The 8-tile, 8-slot kernel (E=128 top-8 decode) takes two strips per workgroup from 8
 // tokens on: each wave quantizes its slot's row once for both and keeps twice the weight bytes in
-// flight (configs[4], whole call: T=8 39.8 -> 38.5 us, T=12 55.7 -> 54.7, T=16 64.0 -> 62.9); below
+// flight (E=128 top-8 H=2048 I=768, whole call: T=8 39.8 -> 38.5 us, T=12 55.7 -> 54.7, T=16 64.0 -> 62.9); below
 // 8 tokens the grid of half as many workgroups leaves CUs idle (T=1 15.5 -> 16.9). Four strips
 // were slower at every T. Each strip's arithmetic is the same, so the bits are too. K of up to 6
-// tiles (inter 768, the configs[4] experts) takes a 6-tile kernel: the registers of the two tiles
+// tiles (inter 768) takes a 6-tile kernel: the registers of the two tiles
 // the 8-tile one loads and never uses went to occupancy (two strips: 108 -> 88 VGPRs, 4 -> 5 waves
 // per SIMD; T=16 whole call 56.7 -> 54.4 us, T=1..12 within the runs' noise). The tiles past KT
 // are never used either way, so the bits are the same.

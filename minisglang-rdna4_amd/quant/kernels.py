@@ -48,7 +48,7 @@ _MOE_MID_MAX_ROWS = 44
 # up to _MOE_G2C_MAX_TOKENS tokens; MINISGL_MOE_G2FUSE=0 keeps the unfused path (requant, gemm2
 # into (P, H) f32, combine), which gives the same bits. The fused kernel reads each routed expert's
 # weights once per token where the grouped gemm2 reads them once per expert; measured on MI355X at
-# configs[4] (whole w4a8_moe call, fused / unfused, us): T=1 25.2/29.5, 2 28.7/33.8, 4 34.0/39.0,
+# E=128 top-8 H=2048 I=768 (whole w4a8_moe call, fused / unfused, us): T=1 25.2/29.5, 2 28.7/33.8, 4 34.0/39.0,
 # 8 47.6/50.3, 12 60.7/59.9, 16 75.4/68.9 at first; with the fused kernel's tile loads all issued
 # before their first use, T=10 49.8/55.3, 12 57.0/62.7, 14 62.8/67.6, 16 66.6/69.4 -- so up to 16.
 _MOE_G2FUSE = os.environ.get("MINISGL_MOE_G2FUSE", "1") != "0"
@@ -516,7 +516,7 @@ def _moe_block_m(num_tokens: int, num_experts: int, top_k: int, flag_gemm1: bool
 
 def _moe_block_m_auto(num_tokens: int, num_experts: int, top_k: int) -> int:
     """The tile height w4a8_moe picks when the caller gives none, from MI355X measurements of these
-    kernels at the configs[4] shape (E=128, top-8, H=2048, I=768), whole call, us:
+    kernels at E=128, top-8, H=2048, I=768, whole call, us:
     - the skinny grouped GEMV (16-row blocks) up to 32 routed rows per expert, where it streams
       each expert's weights once per 16 rows (T=256: 121, against 173 with 64-row tiles and 194
       with 128; T=512, 32 rows: 178 against 180 and 197);
@@ -847,7 +847,7 @@ def _moe_forward(x, w13, w13_scales, w13_zeros, w2, w2_scales, w2_zeros, gating_
 
     # Up to _MOE_SLOTS_MAX tokens on the decode arm: one block per slot instead of the align (one
     # token's experts are distinct, so the align would share no block either; a few tokens share
-    # few, and a shared expert's weights are then streamed once per slot). configs[4], whole call,
+    # few, and a shared expert's weights are then streamed once per slot). E=128 top-8, whole call,
     # align -> slots: T=1 23.9 -> 21.1 us, T=2 28.5 -> 25.6, T=4 34.3 -> 31.0, T=8 50.9 -> 47.8;
     # T=16 68.8 -> 79.0, so the align stays from there on
     slots = M <= _MOE_SLOTS_MAX and block_m < 64

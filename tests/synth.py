@@ -1,4 +1,4 @@
-"""Seeded synthetic inputs for the five BASELINE workloads (shared by tests and bench.py).
+"""Seeded synthetic inputs for the five benchmark workloads (shared by tests and bench.py).
 
 Everything is generated on the CPU with a torch.Generator, so the same seed yields the same
 bytes on every machine; callers move tensors to the GPU themselves.

@@ -256,7 +256,7 @@ def test_moe_scale_guard_fp16_and_unknown():
 
 def test_moe_block_m_policy():
     bm = pkg("quant.kernels")._moe_block_m
-    # BASELINE MoE config: E=128, top-8
+    # E=128, top-8
     assert [bm(T, 128, 8, flag_gemm1=True) for T in (1, 16, 256, 4096)] == [16, 16, 64, 128]
     assert bm(64, 32, 4) == 16 and bm(2048, 32, 4) == 128
 
@@ -281,7 +281,7 @@ def test_pick_dense_kernel():
 
 
 def test_linear_launch_count(lib):
-    """Launches per w4a8_linear call (host-only planner query): the configs[1] step's calls are single
+    """Launches per w4a8_linear call (host-only planner query): the calls of a decode step at Llama-3-8B shapes are single
     launches (the GEMV quantizes its rows) except the two 14336-wide down projections at 8 and 16
     rows; prefill calls and sub-tile groups take the act-quant launch first."""
     step = {}

@@ -3,7 +3,7 @@
 Bars: fp8 activation codes and scales bit-exact; GEMM outputs within 2e-3 relative L2 of the
 oracle's f64 result (the contract), within 5e-4 relative L2 of that result rounded to the output
 dtype (what f32 accumulation leaves: see assert_close_to_oracle), with an element-wise structural
-guard. Full BASELINE sizes are checked against the oracle where it finishes in seconds (every
+guard. Full sizes are checked against the oracle where it finishes in seconds (every
 decode shape), and through row subsets plus bit-exact row-split invariance for the prefill shapes.
 The decode arm is checked for M-invariance: rows[0:m] alone equal the same rows inside a 16-row
 call, bit for bit.
@@ -96,7 +96,7 @@ def _oracle_dense(oracle, x, w, s, z, g, e2m1=False):
 
 
 def test_config1_awq_asym_m16(kernels, oracle, dev):
-    """BASELINE config 1: M=16, K=2560, N=9728, AWQ asym int4 g128, scales |N(0,.02)|+1e-4."""
+    """M=16, K=2560, N=9728, AWQ asym int4 g128, scales |N(0,.02)|+1e-4."""
     M, K, N, g = 16, 2560, 9728, 128
     x = synth.activations(M, K, seed=101)
     w, s, z = synth.int4_weight(N, K, g, seed=102, asym=True, scale_floor=1e-4)
@@ -113,7 +113,7 @@ LLAMA_SHAPES = [(4096, 6144), (4096, 4096), (4096, 28672), (14336, 4096)]  # (K,
 
 @pytest.mark.parametrize("K,N", LLAMA_SHAPES)
 def test_config2_decode_sweep(kernels, oracle, dev, K, N):
-    """BASELINE config 2: GPTQ sym int4 g128 at the four Llama-3-8B layer shapes, M in {1,2,4,8,16},
+    """GPTQ sym int4 g128 at the four Llama-3-8B layer shapes, M in {1,2,4,8,16},
     activations with 0.1% x50 outlier channels. Every M is checked in full against the oracle."""
     g = 128
     x = synth.activations(16, K, seed=200 + K + N, outliers=True)
@@ -136,7 +136,7 @@ M_INV_CASES = [(4096, 6144, 128, "sym"), (4096, 4096, 128, "sym"), (4096, 28672,
 def test_decode_m_invariance(kernels, dev, K, N, g, fmt):
     """The decode arm's self-invariance (tools/quant_m_invariance.py:119-130; the reference records
     worst max|delta| = 0 in _qminv_dense.txt:30-33): rows[0:m] computed alone equal rows[0:m] inside
-    a 16-row call, bit for bit, for m = 1..16 -- the Llama-3-8B shapes, configs[0], a 600-strip
+    a 16-row call, bit for bit, for m = 1..16 -- the Llama-3-8B shapes, K=2560 N=9728, a 600-strip
     weight whose two-strip grid is small, a sub-tile group and MXFP4. The fused silu arm is held to
     the same."""
     x = synth.activations(16, K, seed=K + N + g, outliers=True).to(dev)
@@ -199,7 +199,7 @@ def test_decode_fp16_activations(kernels, oracle, dev):
 # ------------------------------------------------------------------------------- prefill GEMM
 @pytest.mark.parametrize("K,N", LLAMA_SHAPES)
 def test_config3_prefill(kernels, oracle, dev, K, N):
-    """the same shapes at M in {512, 2048, 8192} on the MFMA arm. A row subset
+    """The same shapes at M in {512, 2048, 8192} on the MFMA arm. A row subset
     of each run is checked against the oracle; every row must equal the row computed alone
     (bit-exact row-split / M-invariance)."""
     g = 128
@@ -245,7 +245,7 @@ def test_decode_and_prefill_arms_agree(kernels, oracle, dev):
 # ------------------------------------------------------------------------------- MXFP4
 @pytest.mark.parametrize("K,N", [(8192, 28672), (28672, 8192)])
 def test_config5_mxfp4(kernels, oracle, dev, K, N):
-    """e2m1 codes, E8M0 block-32 scales (exponents in [-8, 0]), M in {1, 16, 4096}."""
+    """MXFP4: e2m1 codes, E8M0 block-32 scales (exponents in [-8, 0]), M in {1, 16, 4096}."""
     w, s8 = synth.mxfp4_weight(N, K, seed=500 + K)
     tiles = kernels.repack_w4(w.to(dev), weight_is_e2m1=True)
     sd = s8.to(dev)

@@ -1,4 +1,4 @@
-"""GPU parity of the grouped W4A8 MoE path (BASELINE config 4 and its MXFP4 twin).
+"""GPU parity of the grouped W4A8 MoE path (E=128 top-8 H=2048 I=768, int4 and MXFP4).
 
 Route ids and the align arrays are integer work: bit-exact against the oracle. Routing weights are
 f32 softmax ratios: within 1e-6 relative. The MoE output is checked stage by stage against the
@@ -275,7 +275,7 @@ def _assert_end_to_end(got, ref, stage2_ref, rel2, what):
 
 @pytest.mark.parametrize("T", [1, 16, 256, 4096])
 def test_config4_moe(kernels, oracle, dev, experts, T):
-    """BASELINE config 4: E=128 top-8, H=2048, I=768, int4 g128 sym, T in {1, 16, 256, 4096}, on
+    """E=128 top-8, H=2048, I=768, int4 g128 sym, T in {1, 16, 256, 4096}, on
     every token up to 32 and on 32 tokens spread over the larger batches. Asserted: each stage
     (gemm1 + silu; requant + gemm2 + combine, each fed the GPU's own input) within 2e-3 relative L2
     of the oracle; end to end against the oracle's full f64 forward, relative L2 at most the GPU's

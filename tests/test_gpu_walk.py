@@ -15,7 +15,7 @@ from test_gpu_dense import _oracle_dense, assert_close_to_oracle
 
 pytestmark = pytest.mark.gpu
 
-# (K, N, format): the configs[1] shapes, configs[0], MXFP4 at configs[5]'s down shape, a 5-wave and
+# (K, N, format): the Llama-3-8B shapes, K=2560 N=9728, MXFP4 at K=28672 N=8192, a 5-wave and
 # a 6-wave K split (threads per row not a power of two), a one-tile K, an N that is not a multiple
 # of 32, a two-strip weight, and NVFP4 (which walks above 4 rows)
 CASES = [(4096, 6144, "sym"), (4096, 4096, "sym"), (4096, 28672, "sym"), (14336, 4096, "sym"),
@@ -111,7 +111,7 @@ def test_walk_special_rows(kernels, dev):
 
 
 def test_walk_against_oracle(kernels, oracle, dev):
-    """Walked calls at configs[1]'s gate_up and down shapes against the oracle directly."""
+    """Walked calls at the Llama-3-8B gate_up and down shapes against the oracle directly."""
     for K, N in [(4096, 28672), (14336, 4096)]:
         w, s, _, g, _, tiles, sd, _ = _weights(K, N, "sym", dev, seed=K)
         x = synth.activations(4, K, seed=N, outliers=True)
