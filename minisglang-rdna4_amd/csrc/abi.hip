@@ -511,8 +511,8 @@ int w4a16_linear(const void* x, int x_dtype, int64_t M, int64_t K, int64_t ldx, 
     GemmArgs q = p;
     q.out = out; q.ldo = ldo; q.out_dtype = kBF16; q.silu = silu; q.tsum2 = 1;
     if (dma_tiled_ok(q)) {
-      // wide symmetric int4: the terms' codes rewritten in the GEMM's operand order with their
-      // row-sum seeds, into the f32 rows' space that this path leaves unused
+      // wide weights: the terms' codes rewritten in the GEMM's operand order (symmetric int4: with
+      // their row-sum seeds), into the f32 rows' space that this path leaves unused
       const int64_t Mp = round16(q.M), KT = q.KT;
       uint8_t* xt = reinterpret_cast<uint8_t*>(y);
       float* seeds = reinterpret_cast<float*>(xt + round256(Mp * K));
