@@ -1,9 +1,11 @@
-// Offsets of the prefill kernels' buffer loads on a K that ends inside a 128-wide tile. Plain functions,
+// Offsets of the GEMM kernels' buffer loads on a K that ends inside a 128-wide tile. Plain functions,
 // so that a host program can walk every lane of every load (tests/test_ragged_offsets.py).
 //
 // Of a load's two offsets only the vector one is checked against the descriptor's size; the scalar one is
 // added behind the check. A load that may fall outside its matrix therefore carries everything in the
-// vector offset, where a read past the end gives zeros, and no vector offset goes below zero.
+// vector offset, where a read past the end gives zeros (the prefill kernels), or moves the descriptor's
+// start and size in its place (the decode kernels, whose lanes it costs nothing); and no vector offset goes
+// below zero.
 #pragma once
 #include <stdint.h>
 
@@ -46,6 +48,13 @@ W4A8_HD uint32_t e8m0_word(int lane, int strip, int N) {
 // e4m3 scale byte of block 2q + h of a tile, channel lane & 15 of a strip
 W4A8_HD uint32_t e4m3_byte(int lane, int h, int strip, int N) {
   return (uint32_t)((2 * (lane >> 4) + h) * N + strip * 16 + (lane & 15));
+}
+// Decode kernels: bytes from tile kt's first E8M0 row to the end of the scales, the size of the descriptor
+// that starts there; and where the e4m3 row of block ss of tile kt starts, the last row again for blocks past K
+W4A8_HD uint32_t e8m0_bytes_left(int kt, int K, int N) { return (uint32_t)((K / 32 - kt * 4) * N); }
+W4A8_HD uint32_t e4m3_row(int kt, int ss, int K, int N) {
+  const uint32_t row = (uint32_t)((kt * 8 + ss) * N), last = (uint32_t)((K / 16 - 1) * N);
+  return row < last ? row : last;
 }
 // a scale or zero load, its rows starting at byte `so` of the matrix; ragged: in a tile that may have
 // fewer rows than the load covers

@@ -18,6 +18,7 @@
 // tiles before its first MFMA, so it keeps a chunk's worth of weight bytes in flight. Waves reduce
 // through LDS in a fixed order: results do not depend on timing, and no second kernel is needed.
 #pragma once
+#include "buf_offsets.h"
 #include "gemm_args.h"
 #include "moe_route.h"
 
@@ -389,14 +390,15 @@ __global__ void __launch_bounds__(512) gemv_kernel(const GemmArgs p, int tpw) {
         sc[t >> 1][j][t & 1] = bload16(rs_s, (uint32_t)n * 2, (uint32_t)(g * N * 2));
         if (!SYM) zw[t][j] = zeros ? bload32(rs_z, (uint32_t)(n / 8) * 4, (uint32_t)(g * (N / 8) * 4)) : 0x88888888u;
       } else if (MODE == kModeE8M0) {
-        // blocks past K read as 0 (2^-127) from the descriptor's bound; their activations are 0
-        sb[t][j] = (int)bload8(rs_s, (uint32_t)((lane >> 4) * N + n), (uint32_t)(kt * 4 * N));
+        // blocks past K read as 0 (2^-127) from the bound of what is left of the scales; their activations are 0
+        const BufRsrc rs_t = make_rsrc(reinterpret_cast<const char*>(scales) + kt * 4 * N, e8m0_bytes_left(kt, K, N));
+        sb[t][j] = (int)bload8(rs_t, (uint32_t)((lane >> 4) * N + n), 0);
       } else if (MODE == kModeNV) {
-        // groups past K read as 0 from the descriptor's bound (a zero scale)
+        // groups past K read the last one again; their activations are 0
 #pragma unroll
         for (int ss = 0; ss < 8; ++ss)
           nvs[MODE == kModeNV ? t : 0][j][ss >> 1][ss & 1] =
-              (unsigned short)bload8(rs_s, (uint32_t)n, (uint32_t)((kt * 8 + ss) * N));
+              (unsigned short)bload8(rs_s, (uint32_t)n, e4m3_row(kt, ss, K, N));
       }
     }
   };

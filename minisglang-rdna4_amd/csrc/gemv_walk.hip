@@ -110,13 +110,15 @@ __global__ void __launch_bounds__(512) gemv_walk_kernel(const GemmArgs p, const 
         sc[s >> 1][j][s & 1] = bload16(rs_s, (uint32_t)n * 2, (uint32_t)(gi * N * 2));
         if (!SYM) zw[s][j] = bload32(rs_z, (uint32_t)(n / 8) * 4, (uint32_t)(gi * (N / 8) * 4));
       } else if (MODE == kModeE8M0) {
-        sb[s][j] = (int)bload8(rs_s, (uint32_t)((lane >> 4) * N + n), (uint32_t)(kt * 4 * N));
+        // blocks past K read as 0 (2^-127) from the bound of what is left of the scales; their activations are 0
+        const BufRsrc rs_t = make_rsrc(reinterpret_cast<const char*>(p.scales) + kt * 4 * N, e8m0_bytes_left(kt, K, N));
+        sb[s][j] = (int)bload8(rs_t, (uint32_t)((lane >> 4) * N + n), 0);
       } else {
-        // groups past K read as 0 from the descriptor's bound (a zero scale)
+        // groups past K read the last one again; their activations are 0
 #pragma unroll
         for (int ss = 0; ss < 8; ++ss)
           nvs[MODE == kModeNV ? s : 0][j][ss >> 1][ss & 1] =
-              (unsigned short)bload8(rs_s, (uint32_t)n, (uint32_t)((kt * 8 + ss) * N));
+              (unsigned short)bload8(rs_s, (uint32_t)n, e4m3_row(kt, ss, K, N));
       }
     }
   };

@@ -1,4 +1,4 @@
-"""The prefill kernels' loads in the tiles of a K that is no multiple of 128, walked on the CPU: csrc/
+"""The GEMM kernels' loads in the tiles of a K that is no multiple of 128, walked on the CPU: csrc/
 buf_offsets.h, whose functions form every offset of those loads, compiled for the host and asked for each
 lane of each step. A load must lie inside the matrix it reads (the last expert's, with nothing behind it)
 or past the size that the unit checks its vector offset against, where it gives zeros; a row of
@@ -19,10 +19,14 @@ static void fail(const char* what, int K, int N, int g, int kt, int lane, BufOff
   printf("%s: K=%d N=%d group=%d tile %d lane %d: offsets %u + %u\n", what, K, N, g, kt, lane, o.v, o.s);
   exit(1);
 }
-// inside the matrix, or wholly past its checked size
-static void load(const char* what, BufOffset o, uint64_t size, uint64_t bytes, int K, int N, int g, int kt, int lane) {
+// inside the matrix, or wholly past the size that the vector offset is checked against
+static void load(const char* what, BufOffset o, uint64_t size, uint64_t bytes, uint64_t checked, int K, int N, int g, int kt,
+                 int lane) {
   const uint64_t at = (uint64_t)o.v + o.s;
-  if (!(at + size <= bytes || o.v >= bytes)) fail(what, K, N, g, kt, lane, o);
+  if (!(at + size <= bytes || o.v >= checked)) fail(what, K, N, g, kt, lane, o);
+}
+static void load(const char* what, BufOffset o, uint64_t size, uint64_t bytes, int K, int N, int g, int kt, int lane) {
+  load(what, o, size, bytes, bytes, K, N, g, kt, lane);
 }
 
 int main(int argc, char** argv) {
@@ -56,6 +60,15 @@ int main(int argc, char** argv) {
           for (int c = 0; c < gpt; ++c)
             load("scales", row_step(scale_piece(c, strip, lane & 1, N), (uint32_t)(kt * gpt * N * 2), ragged), 16, s_bytes, K,
                  N, g, kt, lane);
+        }
+        // decode kernels: the descriptor starts at the tile's rows; a row for every block
+        const uint64_t left = e8m0_bytes_left(kt, K, N), from = (uint64_t)kt * 4 * N;
+        if (from + left != (uint64_t)K / 32 * N) fail("E8M0 descriptor", K, N, 32, kt, lane, {0, (uint32_t)from});
+        for (int ss = 0; ss < 8; ++ss) {
+          const uint32_t row = e4m3_row(kt, ss, K, N);
+          load("e4m3 row", {(uint32_t)(strip * 16 + (lane & 15)), row}, 1, (uint64_t)K / 16 * N, ~0ull, K, N, 16,
+               kt, lane);
+          if (kt * 128 + ss * 16 < K && row != (uint32_t)((kt * 8 + ss) * N)) fail("e4m3 row (place)", K, N, 16, kt, lane, {0, row});
         }
         if (K % 32 == 0)
           load("E8M0 bytes", row_step(e8m0_word(lane, strip, N), (uint32_t)(kt * 4 * N), ragged), 4, (uint64_t)K / 32 * N, K,
